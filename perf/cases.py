@@ -1,0 +1,697 @@
+"""The calls whose speed matters, as data: what each one stands for, its
+inputs, one pass through the public entry points, and the bytes and operations
+it cannot do without. Frames come from the seeded procedural room
+(sicp_synth_*), every case at the sizes and voxel sizes of the tests and of
+bench.py; `draw` gives others of the same ranges, odd sizes among them.
+
+Sequences are replayed forwards and backwards, so a system or a map can be
+stepped any number of times with neighbouring frames following each other.
+"""
+import ctypes
+import math
+from concurrent.futures import ThreadPoolExecutor
+
+import numpy as np
+import torch
+
+from semantic_icpslam_amd import binding as B
+
+DEPTH_SCALE, CUTOFF, DEPTH_MIN, DEPTH_MAX = 1000.0, 3.0, 0.1, 3.0
+
+
+def listed():
+    return [
+        # The coarsest tracking level of a 640x480 frame: one Gauss-Newton
+        # step whose 6x6 system the caller solves on the host (ICPStep as
+        # Tracker::ComputeSE3 calls it). Launches and the round trip count.
+        dict(name="icp_step_160x120", op="icp", cols=160, rows=120, fp32=False, host=True),
+        # The largest image of the step, odd sized, in the compensated FP32
+        # form, its sums left on the device.
+        dict(name="icp_step_1279x719_fp32", op="icp", cols=1279, rows=719, fp32=True, host=False),
+        # The photometric step (RGBStep) at the middle level, host results.
+        dict(name="rgb_step_320x240", op="rgb", cols=320, rows=240),
+        # A frame's image pyramids through the single operations
+        # (Frame::FillImages and ResizeImages): 19 calls.
+        dict(name="images_640x480", op="images", cols=640, rows=480),
+        # A small camera, the pose read back after every frame.
+        dict(name="frame_320x240", op="frame", cols=320, rows=240, voxel=0.01, blocks=60000,
+             photometric=False, precision=False, unify=False, graph=False, result=True, frames=8),
+        # The headline sequence: 640x480, 5 mm, labels, a frame a graph launch.
+        dict(name="frame_640x480", op="frame", cols=640, rows=480, voxel=0.005, blocks=400000,
+             photometric=False, precision=False, unify=False, graph=True, result=False, frames=8),
+        # The same with the reference's own defaults: photometric tracking
+        # and the neighbour label pass, plain launches.
+        dict(name="frame_640x480_photometric", op="frame", cols=640, rows=480, voxel=0.005,
+             blocks=400000, photometric=True, precision=False, unify=True, graph=False,
+             result=False, frames=8),
+        # A large camera in the precision form (half TSDF, compensated sums).
+        dict(name="frame_1280x720_precision", op="frame", cols=1280, rows=720, voxel=0.004,
+             blocks=300000, photometric=False, precision=True, unify=False, graph=True,
+             result=False, frames=6),
+        # Eight sequences of uneven resolution advanced together.
+        dict(name="batch_8", op="batch", systems=8, blocks=300000, shared=False, frames=6),
+        # Mapping at given poses through the map's own entry points, 2 mm
+        # voxels: allocation, fusion with labels, depth ranges, raycast.
+        dict(name="map_640x480_2mm", op="map", cols=640, rows=480, voxel=0.002, blocks=200000,
+             precision=False, unify=False, frames=8),
+        # The surface of a mapped view as triangles.
+        dict(name="mesh_640x480", op="mesh", cols=640, rows=480, voxel=0.005, blocks=100000,
+             triangles=1000000, precision=False, frames=5),
+        # The raycast's derivative for 10k pixels, pose and TSDF gradients
+        # (a step of an optimiser, which clears the TSDF gradient).
+        dict(name="adjoint_1280x720", op="adjoint", cols=1280, rows=720, voxel=0.002,
+             blocks=1 << 16, pixels=10000, frames=2),
+    ]
+
+
+def draw(rng):
+    def size(lo, hi):
+        cols = int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+        rows = max(8, int(cols * rng.choice([0.5625, 0.75, 0.7])) + rng.randrange(-3, 4))
+        return cols, rows
+
+    def voxel(cols):  # 5 mm at 640 columns, finer with more of them
+        return round(min(0.012, max(0.003, 0.005 * 640 / cols * rng.uniform(0.8, 1.5))), 5)
+
+    op = rng.choice(["icp", "icp", "rgb", "images", "frame", "frame", "frame", "batch", "map",
+                     "mesh", "adjoint"])
+    flag = lambda: rng.random() < 0.5
+    if op == "icp":
+        cols, rows = size(80, 1280)
+        return dict(op=op, cols=cols, rows=rows, fp32=flag(), host=flag())
+    if op in ("rgb", "images"):
+        cols, rows = size(80, 1280)
+        return dict(op=op, cols=cols, rows=rows)
+    if op == "frame":
+        cols, rows = size(160, 1100)
+        return dict(op=op, cols=cols, rows=rows, voxel=voxel(cols), blocks=200000,
+                    photometric=flag(), precision=flag(), unify=rng.random() < 0.25,
+                    graph=flag(), result=flag(), frames=6)
+    if op == "batch":
+        return dict(op=op, systems=rng.randrange(2, 8), blocks=200000, shared=flag(), frames=5)
+    cols, rows = size(160, 900)
+    if op == "map":
+        return dict(op=op, cols=cols, rows=rows, voxel=max(0.002, round(0.6 * voxel(cols), 5)),
+                    blocks=200000, precision=flag(), unify=rng.random() < 0.25, frames=6)
+    if op == "mesh":
+        return dict(op=op, cols=cols, rows=rows, voxel=voxel(cols), blocks=100000,
+                    triangles=2000000, precision=flag(), frames=4)
+    return dict(op=op, cols=cols, rows=rows, voxel=round(0.6 * voxel(cols), 5), blocks=1 << 16,
+                pixels=int(math.exp(rng.uniform(math.log(500), math.log(20000)))), frames=2)
+
+
+# ------------------------------------------------------------------ inputs --
+def _camera(cols, rows):
+    f = 0.8203125 * cols  # 525 at 640 columns
+    return f, f, (cols - 1) / 2.0, (rows - 1) / 2.0
+
+
+def _render(cols, rows, seed, frames):
+    """`frames` (depth u16, rgb u8x3, labels u8) host images and their poses."""
+    syn = B.Synth(cols, rows, *_camera(cols, rows), seed=seed)
+    with ThreadPoolExecutor(max_workers=8) as ex:
+        out = list(ex.map(syn.render, frames))
+    return out, [syn.pose(i) for i in frames]
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _turn(i, n):
+    """Index of step i of a sequence of n frames run forwards and backwards."""
+    if n == 1:
+        return 0
+    k = i % (2 * (n - 1))
+    return k if k < n else 2 * (n - 1) - k
+
+
+def _maps(depth_u16, cols, rows):
+    """Vertex and normal maps (rows, cols, 4) of a depth image, as float32."""
+    fx, fy, cx, cy = (np.float32(v) for v in _camera(cols, rows))
+    z = depth_u16.astype(np.float32) / np.float32(DEPTH_SCALE)
+    bad = ~((z > 0.1) & (z < CUTOFF))
+    x, y = np.meshgrid(np.arange(cols, dtype=np.float32), np.arange(rows, dtype=np.float32))
+    v = np.stack([z * (x - cx) / fx, z * (y - cy) / fy, z, np.ones_like(z)], -1)
+    v[bad] = np.nan
+    n = np.full_like(v, np.nan)
+    a, b = v[:-1, 1:, :3] - v[:-1, :-1, :3], v[1:, :-1, :3] - v[:-1, :-1, :3]
+    c = np.cross(a, b)
+    with np.errstate(invalid="ignore", divide="ignore"):
+        c = c / np.linalg.norm(c, axis=-1, keepdims=True)
+    n[:-1, :-1, :3] = c
+    n[:-1, :-1, 3] = np.where(np.isnan(c[..., 0]), np.nan, 1.0)
+    return v, n
+
+
+def _step_inputs(case, seed):
+    """Two neighbouring frames' maps and intensities, and their poses."""
+    cols, rows = case["cols"], case["rows"]
+    fr, poses = _render(cols, rows, seed, [4, 5])
+    (vl, nl), (vc, nc) = (_maps(f[0], cols, rows) for f in fr)
+    gray = [(0.299 * f[1][..., 0] + 0.587 * f[1][..., 1] + 0.114 * f[1][..., 2]).astype(np.uint8)
+            for f in fr]
+    g = np.pad(gray[1].astype(np.int32), 1, mode="edge")
+    dx = (g[:-2, 2:] - g[:-2, :-2] + 2 * (g[1:-1, 2:] - g[1:-1, :-2]) + g[2:, 2:] - g[2:, :-2])
+    dy = (g[2:, :-2] - g[:-2, :-2] + 2 * (g[2:, 1:-1] - g[:-2, 1:-1]) + g[2:, 2:] - g[:-2, 2:])
+    return dict(vc=vc, vl=vl, nc=nc, nl=nl, gl=gray[0], gc=gray[1], dx=dx.astype(np.int16),
+                dy=dy.astype(np.int16), last=poses[0], curr=poses[0])
+
+
+class _DeviceImage:
+    """A device image of the library's own (sicp_system_frame_image) as an
+    array that torch can view. A view keeps this object, and with it the
+    system that owns the memory, for as long as it lives."""
+
+    def __init__(self, system, im, channels):
+        self.system = system
+        self.__cuda_array_interface__ = dict(
+            shape=(im.rows, im.cols, channels), typestr="<f4", data=(im.ptr, False), version=3,
+            strides=(im.pitch, 4 * channels, 4))
+
+
+# ----------------------------------------------------------------- prepare --
+def prepare(case, seed):
+    return _PREPARE[case["op"]](case, seed)
+
+
+def _prepare_icp(case, seed):
+    h = _step_inputs(case, seed)
+    t = {k: _dev(h[k]) for k in ("vc", "vl", "nc", "nl")}
+    s = dict(case=case, t=t, im=[B.image(t[k]) for k in ("vc", "vl", "nc", "nl")],
+             curr=B.pose_f(h["curr"]), last=B.pose_f(h["last"]),
+             K=B.intrinsics(*_camera(case["cols"], case["rows"])),
+             scratch=torch.zeros(B.lib().sicp_icp_partials_size(), dtype=torch.uint8,
+                                 device="cuda"),
+             sums=torch.zeros(29, dtype=torch.float32, device="cuda"))
+    s["fn"] = B.lib().sicp_icp_step_fp32 if case["fp32"] else B.lib().sicp_icp_step
+    return s
+
+
+def _prepare_rgb(case, seed):
+    h = _step_inputs(case, seed)
+    names = ("gc", "gl", "vc", "vl", "dx", "dy")
+    t = {k: _dev(h[k]) for k in names}
+    size = B.lib().sicp_rgb_scratch_size(case["cols"], case["rows"])
+    return dict(case=case, t=t, im=[B.image(t[k]) for k in names], curr=B.pose_f(h["curr"]),
+                last=B.pose_f(h["last"]), K=B.intrinsics(*_camera(case["cols"], case["rows"])),
+                size=size, scratch=torch.zeros(size, dtype=torch.uint8, device="cuda"),
+                sums=torch.zeros(29, dtype=torch.float32, device="cuda"))
+
+
+def _prepare_images(case, seed):
+    cols, rows = case["cols"], case["rows"]
+    (frame,), _ = _render(cols, rows, seed, [3])
+    t = dict(depth=_dev(frame[0]), rgb=_dev(frame[1]))
+    new = lambda c, r, ch, dt: torch.zeros((r, c, ch) if ch > 1 else (r, c), dtype=dt,
+                                           device="cuda")
+    f32, u8, i16 = torch.float32, torch.uint8, torch.int16
+    t["raw"] = new(cols, rows, 1, f32)
+    for i in range(3):
+        c, r = cols >> i, rows >> i
+        t["d%d" % i], t["g%d" % i] = new(c, r, 1, f32), new(c, r, 1, u8)
+        for k in ("v", "n", "mv", "mn"):
+            t["%s%d" % (k, i)] = new(c, r, 4, f32)
+        t["dx%d" % i], t["dy%d" % i] = new(c, r, 1, i16), new(c, r, 1, i16)
+    mv, mn = _maps(frame[0], cols, rows)
+    t["mv0"], t["mn0"] = _dev(mv), _dev(mn)
+    im = {k: B.image(v) for k, v in t.items()}
+    L, fk = B.lib(), _camera(cols, rows)
+    calls = [(L.sicp_filter_depth, (im["depth"], im["raw"], im["d0"], DEPTH_SCALE, CUTOFF)),
+             (L.sicp_image_to_intensity, (im["rgb"], im["g0"]))]
+    for i in range(3):
+        if i:
+            calls += [(L.sicp_pyrdown_gauss_f32, (im["d%d" % (i - 1)], im["d%d" % i])),
+                      (L.sicp_pyrdown_gauss_u8, (im["g%d" % (i - 1)], im["g%d" % i])),
+                      (L.sicp_resize_map, (im["mv%d" % (i - 1)], im["mn%d" % (i - 1)],
+                                           im["mv%d" % i], im["mn%d" % i]))]
+        k = [float(np.float32(v) / np.float32(1 << i)) for v in fk]
+        calls += [(L.sicp_compute_vmap, (im["d%d" % i], im["v%d" % i], *k, CUTOFF)),
+                  (L.sicp_compute_nmap, (im["v%d" % i], im["n%d" % i])),
+                  (L.sicp_compute_derivative_image, (im["g%d" % i], im["dx%d" % i],
+                                                     im["dy%d" % i]))]
+    out = {k: v for k, v in t.items() if k not in ("depth", "rgb", "mv0", "mn0")}
+    return dict(case=case, t=t, calls=calls, out=out)
+
+
+def _system(case, cols, rows, voxel, spread=1):
+    cfg = B.system_config(cols, rows, *_camera(cols, rows), voxel, 3 * voxel, 1 << 20,
+                          case["blocks"])
+    cfg.icp_spread = spread
+    if case.get("photometric"):
+        cfg.icp_only = 0
+    if case.get("precision"):
+        cfg.icp_sums_fp32, cfg.map.tsdf_half, cfg.map.max_weight = 1, 1, 128
+    cfg.map.unify_labels = 1 if case.get("unify") else 0
+    return B.System(cfg)
+
+
+def _model(system, views):
+    """The level-0 model maps of the frame just grabbed (system's buffers)."""
+    out = []
+    for which in (0, 1):
+        im = system.frame_image(which)
+        if im.ptr not in views:
+            views[im.ptr] = torch.as_tensor(_DeviceImage(system, im, 4), device="cuda")
+        out.append(views[im.ptr])
+    return out
+
+
+def _prepare_frame(case, seed):
+    host, _ = _render(case["cols"], case["rows"], seed, range(case["frames"]))
+    s = dict(case=case, frames=[tuple(_dev(a) for a in f) for f in host], i=0, views={},
+             system=_system(case, case["cols"], case["rows"], case["voxel"]))
+    for _ in range(4):  # a map to track against
+        _run_frame(s)
+    return s
+
+
+_BATCH = [(640, 480, 0.005), (320, 240, 0.008), (1280, 720, 0.004)]
+
+
+def _prepare_batch(case, seed):
+    systems, frames = [], []
+    for k in range(case["systems"]):  # 3 x 640x480, 3 x 320x240, 2 x 1280x720 of eight
+        cols, rows, voxel = _BATCH[k % 3]
+        host, _ = _render(cols, rows, 16 * seed + k, range(case["frames"]))
+        frames.append([tuple(_dev(a) for a in f) for f in host])
+        systems.append(_system(case, cols, rows, voxel, spread=0))
+    batch = B.Batch(systems)
+    batch.set_shared_tracking(case["shared"])
+    s = dict(case=case, systems=systems, frames=frames, batch=batch, i=0, views={})
+    for _ in range(3):
+        _run_batch(s)
+    return s
+
+
+def _mapped(case, seed, n):
+    """A map and `n` frames as sicp_fuse_map_color takes them."""
+    cols, rows = case["cols"], case["rows"]
+    host, poses = _render(cols, rows, seed, range(0, 2 * n, 2))
+    cfg = B.map_config(case["voxel"], 3 * case["voxel"], 1 << 20, case["blocks"])
+    cfg.max_cols, cfg.max_rows = cols, rows
+    cfg.unify_labels = 1 if case.get("unify") else 0
+    if case.get("precision"):
+        cfg.tsdf_half, cfg.max_weight = 1, 128
+    frames = []
+    for (d, rgb, lab), T in zip(host, poses):
+        z = d.astype(np.float32) / np.float32(DEPTH_SCALE)
+        z[~(z < CUTOFF)] = np.nan
+        t = [_dev(z), _dev(rgb), _dev(_maps(d, cols, rows)[1]), _dev(lab)]
+        frames.append((t, [B.image(x) for x in t], B.pose_f(T)))
+    return B.Map(cfg), frames, B.intrinsics(*_camera(cols, rows))
+
+
+def _fuse(m, frame, K):
+    B.check(B.lib().sicp_fuse_map_color(m.h, *frame[1], 1, ctypes.byref(frame[2]), None, K, None,
+                                        B.stream_ptr()), "fuse_map_color")
+
+
+def _zranges(cols, rows):
+    return [torch.zeros(((rows + 7) // 8, (cols + 7) // 8), dtype=torch.float32, device="cuda")
+            for _ in range(2)]
+
+
+def _prepare_map(case, seed):
+    m, frames, K = _mapped(case, seed, case["frames"])
+    maps = [torch.zeros((case["rows"], case["cols"], 4), dtype=torch.float32, device="cuda")
+            for _ in range(2)]
+    z = _zranges(case["cols"], case["rows"])
+    s = dict(case=case, map=m, frames=frames, K=K, maps=maps, z=z, i=0,
+             im=[B.image(x) for x in maps + z])
+    for _ in range(3):
+        _run_map(s)
+    return s
+
+
+def _prepare_mesh(case, seed):
+    m, frames, K = _mapped(case, seed, case["frames"])
+    for f in frames:
+        _fuse(m, f, K)
+    n = case["triangles"]
+    new = lambda dt: torch.zeros((n, 3, 3), dtype=dt, device="cuda")
+    torch.cuda.synchronize()
+    return dict(case=case, map=m, frames=frames,
+                out=[new(torch.float32), new(torch.float32), new(torch.uint8)])
+
+
+def _prepare_adjoint(case, seed):
+    cols, rows, n = case["cols"], case["rows"], case["pixels"]
+    m, frames, K = _mapped(case, seed, case["frames"])
+    for f in frames:
+        _fuse(m, f, K)
+    z = _zranges(cols, rows)
+    iz, pose = [B.image(x) for x in z], frames[-1][2]
+    B.check(B.lib().sicp_create_rendering_blocks(m.h, *iz, DEPTH_MAX, DEPTH_MIN,
+                                                 ctypes.byref(pose), None, K, None,
+                                                 B.stream_ptr()), "rendering_blocks")
+    rng = np.random.default_rng(seed)
+    put = lambda a: torch.from_numpy(a).cuda()
+    new = lambda shape, dt: torch.zeros(shape, dtype=dt, device="cuda")
+    f32 = torch.float32
+    return dict(case=case, map=m, frames=frames, z=z, iz=iz, pose=pose,
+                pix=put(rng.choice(cols * rows, n, replace=False).astype(np.int32)),
+                gv=put(rng.normal(size=(n, 3)).astype(np.float32)),
+                gn=put(rng.normal(size=(n, 3)).astype(np.float32)),
+                sdf=new(case["blocks"] * 512, f32), px=new((n, 6), f32),
+                pg=new(6, torch.float64),
+                scratch=new(B.lib().sicp_raycast_backward_scratch_size(), torch.uint8))
+
+
+_PREPARE = dict(icp=_prepare_icp, rgb=_prepare_rgb, images=_prepare_images, frame=_prepare_frame,
+                batch=_prepare_batch, map=_prepare_map, mesh=_prepare_mesh,
+                adjoint=_prepare_adjoint)
+
+
+# --------------------------------------------------------------------- run --
+def run(state):
+    return _RUN[state["case"]["op"]](state)
+
+
+def _ptr(a):
+    return a.ctypes.data_as(ctypes.c_void_p)
+
+
+def _run_icp(s):
+    args = (*s["im"], ctypes.byref(s["curr"]), ctypes.byref(s["last"]), s["K"],
+            s["scratch"].data_ptr(), s["sums"].data_ptr())
+    if not s["case"]["host"]:
+        B.check(s["fn"](*args, None, None, None, None, B.stream_ptr()), "icp_step")
+        return dict(sums=s["sums"])
+    A, b, res = np.zeros((6, 6)), np.zeros(6), np.zeros(2, np.float32)
+    B.check(s["fn"](*args, None, _ptr(A), _ptr(b), _ptr(res), B.stream_ptr()), "icp_step")
+    return dict(A=A, b=b, residual=res)
+
+
+def _run_rgb(s):
+    A, b, res = np.zeros((6, 6)), np.zeros(6), np.zeros(2, np.float32)
+    corr, sigma = np.zeros(2, np.int32), np.zeros(1, np.float32)
+    B.check(B.lib().sicp_rgb_step(*s["im"], ctypes.byref(s["curr"]), ctypes.byref(s["last"]),
+                                  s["K"], s["scratch"].data_ptr(), s["size"],
+                                  s["sums"].data_ptr(), None, _ptr(corr), _ptr(sigma), _ptr(A),
+                                  _ptr(b), _ptr(res), B.stream_ptr()), "rgb_step")
+    return dict(A=A, b=b, residual=res, corresp=corr, sigma=sigma)
+
+
+def _run_images(s):
+    st = B.stream_ptr()
+    for fn, args in s["calls"]:
+        B.check(fn(*args, st))
+    return s["out"]
+
+
+def _run_frame(s):
+    d, rgb, lab = s["frames"][_turn(s["i"], len(s["frames"]))]
+    s["i"] += 1
+    g = s["system"]
+    if s["case"]["graph"]:
+        g.grab_staged(d, rgb, lab)
+    else:
+        g.grab(d, rgb, lab)
+    out = dict(zip(("vmap", "nmap"), _model(g, s["views"])))
+    if s["case"]["result"]:
+        r = g.result()
+        out.update(pose=r["pose"], tracked=r["tracked"], icp_count=r["icp_count"],
+                   icp_error=np.float32(r["icp_error"]), visible=r["visible_blocks"],
+                   allocated=r["allocated_blocks"])
+    return out
+
+
+def _run_batch(s):
+    s["batch"].grab_staged([f[_turn(s["i"], len(f))] for f in s["frames"]])
+    s["i"] += 1
+    return [_model(g, s["views"]) for g in s["systems"]]
+
+
+def _run_map(s):
+    f = s["frames"][_turn(s["i"], len(s["frames"]))]
+    s["i"] += 1
+    _fuse(s["map"], f, s["K"])
+    L, st, pose = B.lib(), B.stream_ptr(), ctypes.byref(f[2])
+    vmap, nmap, zmin, zmax = s["im"]
+    B.check(L.sicp_create_rendering_blocks(s["map"].h, zmin, zmax, DEPTH_MAX, DEPTH_MIN, pose,
+                                           None, s["K"], None, st), "rendering_blocks")
+    B.check(L.sicp_raycast(s["map"].h, vmap, nmap, zmin, zmax, pose, None, s["K"], st), "raycast")
+    return dict(vmap=s["maps"][0], nmap=s["maps"][1], zmin=s["z"][0], zmax=s["z"][1])
+
+
+def _run_mesh(s):
+    found, total = ctypes.c_uint32(0), ctypes.c_uint32(0)
+    B.check(B.lib().sicp_mesh_scene(s["map"].h, *[t.data_ptr() for t in s["out"]],
+                                    s["case"]["triangles"], ctypes.byref(found),
+                                    ctypes.byref(total), B.stream_ptr()), "mesh_scene")
+    v, n, c = s["out"]  # triangle buffers of the caller's, filled from the front
+    return dict(vertices=v, normals=n, colours=c, found=found.value, total=total.value)
+
+
+def _run_adjoint(s):
+    c = s["case"]
+    fx, fy, cx, cy = _camera(c["cols"], c["rows"])
+    s["sdf"].zero_()
+    B.check(B.lib().sicp_raycast_backward(
+        s["map"].h, *s["iz"], ctypes.byref(s["pose"]), 1.0 / fx, 1.0 / fy, cx, cy, c["cols"],
+        c["rows"], s["pix"].data_ptr(), c["pixels"], s["gv"].data_ptr(), s["gn"].data_ptr(),
+        s["sdf"].data_ptr(), s["px"].data_ptr(), s["pg"].data_ptr(), s["scratch"].data_ptr(),
+        s["scratch"].numel(), B.stream_ptr()), "raycast_backward")
+    return dict(pose=s["pg"], pixels=s["px"], sdf=s["sdf"])
+
+
+_RUN = dict(icp=_run_icp, rgb=_run_rgb, images=_run_images, frame=_run_frame, batch=_run_batch,
+            map=_run_map, mesh=_run_mesh, adjoint=_run_adjoint)
+
+
+# -------------------------------------------------------------------- work --
+# Surfaces of the room lie at about 1.9 m: the voxels of a view are its
+# surface's area times the truncation band in front of and behind it, and a
+# block list entry, voxel or triangle is counted once.
+def _view_voxels(cols, rows, voxel):
+    area = cols * rows * (1.9 / (0.8203125 * cols)) ** 2 * 1.4
+    return area / voxel ** 2 * 6.0  # +-3 voxels
+
+
+def _images_bytes(cols, rows):
+    p = [(cols >> i) * (rows >> i) for i in range(3)]
+    return 5 * p[0] + 4 * p[0] + sum(q * (4 + 1 + 32 + 4) for q in p) + 32 * sum(p)
+
+
+def _map_bytes(cols, rows, voxel, precision=False):
+    # fusion: each voxel's record read and written, the frame read; raycast:
+    # the band's sdf and weight read, the two maps written
+    rec = 16 if precision else 20
+    return _view_voxels(cols, rows, voxel) * (2 * rec + 5) + cols * rows * (4 + 3 + 16 + 1 + 32)
+
+
+def _frame_work(cols, rows, voxel, precision=False, photometric=False):
+    px = cols * rows
+    icp = 10 * px + 5 * px / 4 + 3 * px / 16
+    return (_images_bytes(cols, rows) + icp * (64 + (12 if photometric else 0)) +
+            _map_bytes(cols, rows, voxel, precision),
+            icp * (300 + (100 if photometric else 0)) + px * 1500 +
+            _view_voxels(cols, rows, voxel) * 60)
+
+
+def work(case):
+    op = case["op"]
+    if op == "batch":
+        each = [_frame_work(*_BATCH[k % 3]) for k in range(case["systems"])]
+        return dict(bytes=sum(e[0] for e in each), flops=sum(e[1] for e in each))
+    cols, rows = case["cols"], case["rows"]
+    px = cols * rows
+    if op == "icp":
+        return dict(bytes=64 * px + 116, flops=300 * px)
+    if op == "rgb":
+        return dict(bytes=(32 + 2 + 4) * px + 116, flops=150 * px)
+    if op == "images":
+        return dict(bytes=_images_bytes(cols, rows), flops=700 * px)
+    voxels = _view_voxels(cols, rows, case["voxel"])
+    if op == "frame":
+        b, f = _frame_work(cols, rows, case["voxel"], case["precision"], case["photometric"])
+        return dict(bytes=b, flops=f)
+    if op == "map":
+        return dict(bytes=_map_bytes(cols, rows, case["voxel"], case["precision"]),
+                    flops=voxels * 60 + px * 800)
+    if op == "mesh":  # about two triangles per voxel of surface
+        tri = 2 * voxels / 6
+        return dict(bytes=voxels * 8 + tri * 81, flops=tri * 100)
+    return dict(bytes=4 * 512 * case["blocks"] + case["pixels"] * (28 + 24 + 8 * 8 * 8),
+                flops=case["pixels"] * 3000)
+
+
+# ------------------------------------------------------------------- exact --
+def exact(case, seed):
+    """The single operations in 64 bits. The systems, maps, meshes and the
+    adjoint have none: each is a chain of discrete decisions over a fused map,
+    which in plain array code takes minutes."""
+    fn = dict(icp=_exact_icp, rgb=_exact_rgb, images=_exact_images).get(case["op"])
+    return fn(case, seed) if fn else None
+
+
+def _pose64(T):
+    R = T[:3, :3].astype(np.float32).astype(np.float64)
+    return R, R.T, T[:3, 3].astype(np.float32).astype(np.float64)
+
+
+def _system64(rows_, count):
+    """A, b and the residual pair of the rows [J, r]."""
+    M = rows_.T @ rows_
+    return M[:6, :6], M[:6, 6], np.array([M[6, 6], float(count)])
+
+
+def _exact_icp(case, seed):
+    h = _step_inputs(case, seed)
+    fx, fy, cx, cy = (float(np.float32(v)) for v in _camera(case["cols"], case["rows"]))
+    Rc, _, tc = _pose64(h["curr"])
+    Rl, Rli, tl = _pose64(h["last"])
+    d = {k: h[k].astype(np.float64).reshape(-1, 4) for k in ("vc", "nc")}
+    ok = ~np.isnan(d["vc"][:, 0]) & ~(d["vc"][:, 2] < 1e-3)
+    vc, nc = d["vc"][ok, :3], d["nc"][ok, :3]
+    g = vc @ Rc.T + tc
+    p = (g - tl) @ Rli.T
+    u = np.trunc(p[:, 0] / p[:, 2] * fx + cx + 0.5)
+    v = np.trunc(p[:, 1] / p[:, 2] * fy + cy + 0.5)
+    ok = (u >= 0) & (v >= 0) & (u < case["cols"]) & (v < case["rows"])
+    g, nc, p = g[ok], nc[ok], p[ok]
+    at = v[ok].astype(int) * case["cols"] + u[ok].astype(int)
+    vl = h["vl"].astype(np.float64).reshape(-1, 4)[at, :3]
+    nl = h["nl"].astype(np.float64).reshape(-1, 4)[at, :3]
+    dist = np.linalg.norm(vl @ Rl.T + tl - g, axis=1)
+    sine = np.linalg.norm(np.cross(nc @ Rc.T, nl @ Rl.T), axis=1)
+    ok = (sine < 0.6) & (dist <= 0.1)
+    vl, nl, p = vl[ok], nl[ok], p[ok]
+    J = np.concatenate([-nl, np.cross(nl, vl), -(nl * (p - vl)).sum(1, keepdims=True)], 1)
+    A, b, res = _system64(J, len(J))
+    if case["host"]:
+        return dict(A=A, b=b, residual=res)
+    M = np.concatenate([A, b[:, None]], 1)
+    sums = [M[i, j] for i in range(6) for j in range(i, 7)]
+    return dict(sums=np.array(sums + list(res)))
+
+
+def _exact_rgb(case, seed):
+    h = _step_inputs(case, seed)
+    cols, rows = case["cols"], case["rows"]
+    fx, fy, cx, cy = (float(np.float32(v)) for v in _camera(cols, rows))
+    Rc, Rci, tc = _pose64(h["curr"])
+    Rl, Rli, tl = _pose64(h["last"])
+    g, gx, gy = (h[k].astype(np.int64) for k in ("gc", "dx", "dy"))
+    ok = np.zeros((rows, cols), bool)
+    ok[5:rows - 5, 5:cols - 5] = True
+    pos = g > 0
+    win = np.ones((rows, cols), bool)
+    for a in range(-2, 2):
+        for b in range(-2, 2):
+            win &= np.roll(pos, (-a, -b), (0, 1))
+    ok &= win & (gx * gx + gy * gy > 0) & ~np.isnan(h["vc"][..., 0])
+    i = np.nonzero(ok.reshape(-1))[0]
+    vc = h["vc"].astype(np.float64).reshape(-1, 4)[i]
+    p = (vc[:, :3] @ Rc.T + tc - tl) @ Rli.T
+    u = np.floor(fx * p[:, 0] / p[:, 2] + cx + 0.5)
+    v = np.floor(fy * p[:, 1] / p[:, 2] + cy + 0.5)
+    ok = (u >= 0) & (v >= 0) & (u < cols) & (v < rows)
+    i, vc = i[ok], vc[ok]
+    at = v[ok].astype(int) * cols + u[ok].astype(int)
+    vl = h["vl"].astype(np.float64).reshape(-1, 4)[at]
+    li = h["gl"].astype(np.int64).reshape(-1)[at]
+    ok = ~np.isnan(vl[:, 0]) & (np.linalg.norm(vl - vc, axis=1) < 0.1) & (li != 0)
+    i, vl, diff = i[ok], vl[ok, :3], (g.reshape(-1)[i] - li)[ok].astype(np.float64)
+    sigma = math.sqrt(float((diff * diff).sum()) / max(1, len(diff)))
+    w = sigma + np.abs(diff)
+    w = np.where(w < 1e-3, 1.0, 1.0 / np.maximum(w, 1e-30)) if sigma >= 1e-6 else np.ones_like(w)
+    q = (vl @ Rl.T + tl - tc) @ Rci.T
+    lx = gx.reshape(-1)[i] / 9.0 * fx / q[:, 2]
+    ly = gy.reshape(-1)[i] / 9.0 * fy / q[:, 2]
+    left = np.stack([lx, ly, -(lx * q[:, 0] + ly * q[:, 1]) / q[:, 2]], 1)
+    J = np.concatenate([left, np.cross(q, left), -diff[:, None]], 1) * w[:, None]
+    A, b, res = _system64(J, len(J))
+    return dict(A=A, b=b, residual=res, corresp=None, sigma=np.array([sigma]))
+
+
+def _shift(a, dy, dx):
+    """a[y + dy, x + dx] at clamped coordinates."""
+    r, c = a.shape[:2]
+    return a[np.clip(np.arange(r) + dy, 0, r - 1)][:, np.clip(np.arange(c) + dx, 0, c - 1)]
+
+
+def _exact_filter(d):
+    z = d.astype(np.float64) * float(np.float32(1.0 / DEPTH_SCALE))
+    rows, cols = z.shape
+    y, x = np.arange(rows)[:, None], np.arange(cols)[None, :]
+    s1, s2 = np.zeros_like(z), np.zeros_like(z)
+    for dy in range(-2, 3):
+        for dx in range(-2, 3):
+            cy, cx = y + dy, x + dx
+            on = ((cy >= 0) & (cy < np.minimum(y + 3, rows - 1)) & (cx >= 0) &
+                  (cx < np.minimum(x + 3, cols - 1)))
+            v = _shift(z, dy, dx)
+            w = np.where(on, np.exp(-((dx * dx + dy * dy) * 0.03125 + (z - v) ** 2 * 2.0)), 0.0)
+            s1 += w * v
+            s2 += w
+    with np.errstate(invalid="ignore", divide="ignore"):
+        f = s1 / s2
+    return np.where(z < CUTOFF, z, np.nan), np.where(f < CUTOFF, f, np.nan)
+
+
+def _exact_pyrdown(src):
+    rows, cols = src.shape
+    y, x = np.arange(rows // 2), np.arange(cols // 2)
+    ty, tx = np.minimum(2 * y + 3, rows - 1), np.minimum(2 * x + 3, cols - 1)
+    tap = np.array([1.0, 4.0, 6.0, 4.0, 1.0])
+    s, n = np.zeros((len(y), len(x))), np.zeros((len(y), len(x)))
+    for dy in range(5):
+        for dx in range(5):
+            cy, cx = 2 * y - 2 + dy, 2 * x - 2 + dx
+            v = src[np.clip(cy, 0, rows - 1)][:, np.clip(cx, 0, cols - 1)]
+            on = (((cy >= 0) & (cy < ty))[:, None] & ((cx >= 0) & (cx < tx))[None, :] &
+                  ~np.isnan(v))
+            w = tap[np.clip(ty - cy - 1, 0, 4)][:, None] * tap[np.clip(tx - cx - 1, 0, 4)][None]
+            s += np.where(on, v * w, 0.0)
+            n += np.where(on, w, 0.0)
+    with np.errstate(invalid="ignore", divide="ignore"):
+        return s / n
+
+
+def _exact_maps(z, k):
+    rows, cols = z.shape
+    fx, fy, cx, cy = k
+    x, y = np.arange(cols)[None, :], np.arange(rows)[:, None]
+    ok = (z > 0.1) & (z < CUTOFF)
+    nan = np.nan
+    v = np.stack([np.where(ok, z * (x - cx) / fx, nan), np.where(ok, z * (y - cy) / fy, nan), z,
+                  np.where(ok, 1.0, nan)], -1)
+    n = np.full(v.shape, nan)
+    c = np.cross(v[:-1, 1:, :3] - v[:-1, :-1, :3], v[1:, :-1, :3] - v[:-1, :-1, :3])
+    on = ok[:-1, :-1] & ok[:-1, 1:] & ok[1:, :-1]
+    with np.errstate(invalid="ignore", divide="ignore"):
+        c = c / np.linalg.norm(c, axis=-1, keepdims=True)
+    n[:-1, :-1, :3] = np.where(on[..., None], c, nan)
+    n[:-1, :-1, 3] = np.where(on, 1.0, nan)
+    return v, n
+
+
+def _exact_resize(v, n):
+    r, c = v.shape[0] // 2, v.shape[1] // 2
+    mean = lambda a: (a[0:2 * r:2, 0:2 * c:2] + a[0:2 * r:2, 1:2 * c:2] +
+                      a[1:2 * r:2, 0:2 * c:2] + a[1:2 * r:2, 1:2 * c:2]) / 4.0
+    v, n = mean(v), mean(n)
+    with np.errstate(invalid="ignore", divide="ignore"):
+        n = n / np.linalg.norm(n, axis=-1, keepdims=True)
+    return v, n
+
+
+def _exact_images(case, seed):
+    cols, rows = case["cols"], case["rows"]
+    (frame,), _ = _render(cols, rows, seed, [3])
+    out = {}
+    out["raw"], z = _exact_filter(frame[0])
+    mv, mn = (a.astype(np.float64) for a in _maps(frame[0], cols, rows))
+    for i in range(3):
+        if i:
+            z = _exact_pyrdown(z)
+            mv, mn = _exact_resize(mv, mn)
+            out["mv%d" % i], out["mn%d" % i] = mv, mn
+        k = [float(np.float32(v) / np.float32(1 << i)) for v in _camera(cols, rows)]
+        out["d%d" % i] = z
+        out["v%d" % i], out["n%d" % i] = _exact_maps(z, k)
+        for name in ("g", "dx", "dy"):
+            out["%s%d" % (name, i)] = None
+    return out
