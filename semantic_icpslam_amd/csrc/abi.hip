@@ -87,8 +87,9 @@ int map_alloc(const sicp_map_config& cfg, sicp_map** out) {
     MapDev& d = m->dev;
     if ((rc = dmalloc(m, &d.table, 2 * nb)) || (rc = dmalloc(m, &d.excess, nblk)) ||
         (rc = dmalloc(m, &d.blocks, nblk)) ||
-        (cfg.tsdf_half ? (rc = dmalloc(m, &d.geom_h, nblk * kBlockVoxels))
-                       : (rc = dmalloc(m, &d.geom, nblk * kBlockVoxels))) ||
+        // one block more than the heap's: the empty voxels of a missing block
+        (cfg.tsdf_half ? (rc = dmalloc(m, &d.geom_h, (nblk + 1) * kBlockVoxels))
+                       : (rc = dmalloc(m, &d.geom, (nblk + 1) * kBlockVoxels))) ||
         (rc = dmalloc(m, &d.sem, nblk * kBlockVoxels)) || (rc = dmalloc(m, &m->visible, nblk)) ||
         (rc = dmalloc(m, &m->ctr, 1))) {
         map_free(m);

@@ -45,7 +45,8 @@ SICP_DEV uint64_t mix64(uint64_t z) {
 
 // ----------------------------------------------------------------- reset --
 // ResetMap (FuseMap.cu:1251-1304): entries empty; the heap starts full. Voxels
-// of a block are cleared when the block is created.
+// of a block are cleared when the block is created; those past the heap's last
+// block stay empty (the raycast reads them for a missing block).
 __global__ void reset_table_kernel(MapDev m, AllocScratch a, uint32_t n_req) {
     const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -62,6 +63,13 @@ __global__ void reset_table_kernel(MapDev m, AllocScratch a, uint32_t n_req) {
     for (size_t i = tid; i < n_req; i += stride) {
         a.req_keys[i] = kEmptyKey;
         a.req_first[i] = kNoId;
+    }
+    if (tid < (size_t)kBlockVoxels) {
+        const size_t k = (size_t)m.num_blocks * kBlockVoxels + tid;
+        if (m.half)
+            m.geom_h[k] = kEmptyHalfVoxel;
+        else
+            ((uint2*)m.geom)[k] = make_uint2(0x7fffffffu, 0u);
     }
 }
 

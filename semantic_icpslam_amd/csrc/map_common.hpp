@@ -100,28 +100,43 @@ SICP_DEV EntryView load_entry(const sicp_hash_entry* p) {
 }
 
 // FindEntry (DeviceMap.cu:141-154) over the two-entry bucket (one 32-byte
-// read) and its overflow chain. Returns the heap slot or -1.
-SICP_DEV int table_lookup(const sicp_hash_entry* table, const sicp_hash_entry* excess,
-                          uint32_t nb, uint32_t nb_mask, int x, int y, int z) {
-    if (!key_in_range(x, y, z)) return -1;
+// read) and its overflow chain, in two parts so that a caller can have several
+// buckets' reads in flight: the bucket's entries, then the heap slot or -1.
+struct Probe {
+    EntryView e0, e1;
+    uint64_t key;
+    bool in_range;
+};
+SICP_DEV Probe probe_load(const sicp_hash_entry* table, uint32_t nb, uint32_t nb_mask, int x,
+                          int y, int z) {
     const uint32_t h =
         ((uint32_t)x * 73856093u) ^ ((uint32_t)y * 19349669u) ^ ((uint32_t)z * 83492791u);
     const uint32_t b = nb_mask ? (h & nb_mask) : (h % nb);
-    const uint64_t key = pack_key(x, y, z);
-    // Both entries are read and compared without a branch between them, so
-    // the two 16-byte loads are in flight together (one memory round trip).
-    EntryView e0 = load_entry(table + 2 * (size_t)b);
-    EntryView e1 = load_entry(table + 2 * (size_t)b + 1);
-    const int s1 = (e1.slot >= 0 && e1.key == key) ? e1.slot : -1;
-    const int s0 = (e0.slot >= 0 && e0.key == key) ? e0.slot : s1;
+    Probe p;
+    p.in_range = key_in_range(x, y, z);
+    p.key = pack_key(x, y, z);
+    p.e0 = load_entry(table + 2 * (size_t)b);
+    p.e1 = load_entry(table + 2 * (size_t)b + 1);
+    return p;
+}
+SICP_DEV int probe_result(const Probe& p, const sicp_hash_entry* excess) {
+    if (!p.in_range) return -1;
+    // Both entries compared without a branch between them
+    const int s1 = (p.e1.slot >= 0 && p.e1.key == p.key) ? p.e1.slot : -1;
+    const int s0 = (p.e0.slot >= 0 && p.e0.key == p.key) ? p.e0.slot : s1;
     if (s0 >= 0) return s0;
-    int n = e1.next;
+    int n = p.e1.next;
     while (n >= 0) {
         EntryView e = load_entry(excess + n);
-        if (e.key == key) return e.slot;
+        if (e.key == p.key) return e.slot;
         n = e.next;
     }
     return -1;
+}
+SICP_DEV int table_lookup(const sicp_hash_entry* table, const sicp_hash_entry* excess,
+                          uint32_t nb, uint32_t nb_mask, int x, int y, int z) {
+    if (!key_in_range(x, y, z)) return -1;
+    return probe_result(probe_load(table, nb, nb_mask, x, y, z), excess);
 }
 
 SICP_DEV int map_lookup(const MapDev& m, int x, int y, int z) {

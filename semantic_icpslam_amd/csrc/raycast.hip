@@ -249,36 +249,7 @@ __global__ __launch_bounds__(256) void prepass_lds_kernel(MapDev m, MapCounters*
 // DeviceMap.cu:169-201, for every int), and one cache compare per block.
 struct BlockCache {
     int x, y, z, slot;  // slot -1: empty
-    // The first pass's per-wavefront table of recent lookups (null elsewhere).
-    unsigned long long* lds = nullptr;
 };
-
-// A wavefront's 64 rays cross the same few blocks, so the first pass keeps a
-// direct-mapped table of its recent lookups in LDS, hits and misses alike:
-// 256 entries of one 64-bit word {tag = 1 + the block coordinates in 14 bits
-// each, slot + 1 (0: no block)}, written by atomic exchange so that lanes
-// storing the same entry at once never leave a torn word. Blocks outside
-// +-8192 per axis, and heaps above 2^21 - 2 blocks, go to the table directly.
-// The map is read-only during the raycast, so a cached answer is the table's.
-constexpr int kRayLdsEntries = 256;
-SICP_DEV int lds_lookup(const MapDev& m, unsigned long long* t, int bx, int by, int bz) {
-    const bool fits = (unsigned)(bx + 8192) < 16384u && (unsigned)(by + 8192) < 16384u &&
-                      (unsigned)(bz + 8192) < 16384u;
-    if (!fits) return map_lookup(m, bx, by, bz);
-    const unsigned long long tag = 1ull + (((unsigned long long)(bx & 0x3fff) << 28) |
-                                           ((unsigned long long)(by & 0x3fff) << 14) |
-                                           (unsigned long long)(bz & 0x3fff));
-    const uint32_t i = (((uint32_t)bx * 0x9E3779B1u) ^ ((uint32_t)by * 0x85EBCA77u) ^
-                        ((uint32_t)bz * 0xC2B2AE3Du)) >> 24;
-    const unsigned long long e = t[i];
-    if ((e >> 21) == tag) return (int)(e & 0x1fffffull) - 1;
-    const int s = map_lookup(m, bx, by, bz);
-    atomicExch(&t[i], (tag << 21) | (unsigned long long)(s + 1));
-    return s;
-}
-SICP_DEV int cached_lookup(const MapDev& m, const BlockCache& c, int bx, int by, int bz) {
-    return c.lds ? lds_lookup(m, c.lds, bx, by, bz) : map_lookup(m, bx, by, bz);
-}
 
 // make_int3 of one coordinate (VectorMath.h:36-42): the truncation, one less
 // where it exceeds the value — the floor, for every float (NaN and values
@@ -301,13 +272,13 @@ SICP_DEV long find_voxel_i(const MapDev& m, int vx, int vy, int vz, BlockCache& 
         valid = true;
         return (long)c.slot * kBlockVoxels + local_of(vx, vy, vz);
     }
-    const int slot = cached_lookup(m, c, bx, by, bz);
+    const int slot = map_lookup(m, bx, by, bz);
     if (slot < 0) {
         valid = false;
         return -1;
     }
     valid = true;
-    c = BlockCache{bx, by, bz, slot, c.lds};
+    c = BlockCache{bx, by, bz, slot};
     return (long)slot * kBlockVoxels + local_of(vx, vy, vz);
 }
 
@@ -339,7 +310,7 @@ SICP_DEV void corner_blocks(const MapDev& m, const AxisPair& X, const AxisPair& 
         if (dx > nx || dy > ny || dz > nz) continue;
         const int bx = dx ? (X.v1 >> 3) : bx0, by = dy ? (Y.v1 >> 3) : by0,
                   bz = dz ? (Z.v1 >> 3) : bz0;
-        const int sl = cache_has(c, bx, by, bz) ? c.slot : cached_lookup(m, c, bx, by, bz);
+        const int sl = cache_has(c, bx, by, bz) ? c.slot : map_lookup(m, bx, by, bz);
         s0 = b == 0 ? sl : s0;
         s1 = b == 1 ? sl : s1;
         s2 = b == 2 ? sl : s2;
@@ -433,69 +404,11 @@ SICP_DEV float read_sdf_interped(const MapDev& m, v3 pt, BlockCache& c, bool& va
     return interp_axes(m, axis_pair(pt.x), axis_pair(pt.y), axis_pair(pt.z), c, valid);
 }
 
-// Three interpolated reads with their 24 loads issued together.
-SICP_DEV void interp3(const MapDev& m, const BlockCache& c, const AxisPair (&P)[3][3],
-                      float (&s)[3], bool (&v)[3]) {
-    int i0[8], i1[8], i2[8];
-    interp_corners(m, P[0][0], P[0][1], P[0][2], c, i0, v[0]);
-    interp_corners(m, P[1][0], P[1][1], P[1][2], c, i1, v[1]);
-    interp_corners(m, P[2][0], P[2][1], P[2][2], c, i2, v[2]);
-    float a0[8], a1[8], a2[8];
-    interp_loads(m, i0, a0);
-    interp_loads(m, i1, a1);
-    interp_loads(m, i2, a2);
-    s[0] = interp_blend(a0, P[0][0], P[0][1], P[0][2]);
-    s[1] = interp_blend(a1, P[1][0], P[1][1], P[1][2]);
-    s[2] = interp_blend(a2, P[2][0], P[2][1], P[2][2]);
-}
-
-// Rendering::readNormal (RenderScene.cu:345-378): six interpolated reads at
-// pt +- 1 voxel along each axis (pt.a + 1.0f, pt.a + -1.0f), in order, the
-// first failing one deciding. The three centre values per axis are
-// decomposed once and shared by the six reads. The reads have no side
-// effect, so they run three at a time (their loads in flight together) and
-// the tests follow in the reference's order: the same result.
-SICP_DEV bool read_normal(const MapDev& m, v3 pt, BlockCache& c, const PoseF& pose, v3& n) {
-    const AxisPair xm = axis_pair(pt.x + -1.0f), x0 = axis_pair(pt.x), xp = axis_pair(pt.x + 1.0f);
-    const AxisPair ym = axis_pair(pt.y + -1.0f), y0 = axis_pair(pt.y), yp = axis_pair(pt.y + 1.0f);
-    const AxisPair zm = axis_pair(pt.z + -1.0f), z0 = axis_pair(pt.z), zp = axis_pair(pt.z + 1.0f);
-    float s[6];
-    bool ok[6];
-    {
-        const AxisPair P[3][3] = {{xp, y0, z0}, {xm, y0, z0}, {x0, yp, z0}};
-        float t[3];
-        bool v[3];
-        interp3(m, c, P, t, v);
-        for (int i = 0; i < 3; ++i) {
-            s[i] = t[i];
-            ok[i] = v[i];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-        if (isnan_(s[i]) || s[i] == 1.0f || !ok[i]) return false;
-    {
-        const AxisPair P[3][3] = {{x0, ym, z0}, {x0, y0, zp}, {x0, y0, zm}};
-        float t[3];
-        bool v[3];
-        interp3(m, c, P, t, v);
-        for (int i = 0; i < 3; ++i) {
-            s[3 + i] = t[i];
-            ok[3 + i] = v[i];
-        }
-    }
-#pragma unroll
-    for (int i = 3; i < 6; ++i)
-        if (isnan_(s[i]) || s[i] == 1.0f || !ok[i]) return false;
-    n = normalised(mv(pose.Rinv, mk(s[0] - s[1], s[2] - s[3], s[4] - s[5])));
-    return true;
-}
-
 struct RayArgs {
     float invfx, invfy, cx, cy;
     int cols, rows;
+    int tcols, trows;        // raycast_kernel: 8x8-pixel tiles across and down
     int first_pass_samples;  // the first pass's hand-over point (raycast_kernel only)
-    int lds_block_table;     // raycast_kernel: block lookups through its LDS table
 };
 
 // The ray of pixel (x, y) (RenderScene.cu:393-421): start point and unit
@@ -532,13 +445,259 @@ SICP_DEV bool ray_setup(const MapDev& m, const View<float>& zmin, const View<flo
 // Most rays end well before; the few that graze a surface for hundreds of
 // one-voxel steps would otherwise set the length of the whole launch.
 
-// First pass: one lane per ray, 8x8-pixel wavefronts (the zRange tile).
-__global__ __launch_bounds__(64, 5) void raycast_kernel(MapDev m, View<float4> vmap,
+// ---- first pass: one lane per ray -----------------------------------------
+// What bounds it: not bytes (it reads a tenth of what HBM could give it) but
+// the instructions and dependent memory round trips of each wavefront's march;
+// all wavefronts run at once (4800 at 640x480, up to six a SIMD), and the
+// launch lasts as long as the slowest one. Written as the
+// reference's loop, every iteration ran every path some lane needed — a
+// table probe, an interpolated read with its block lookups, a plain step —
+// 450 instructions and up to four dependent round trips, some 20 times. Here
+// a lane that needs a table probe or an interpolated read waits while the
+// others march on, and the waiting lanes are served together when enough of
+// them wait: the same samples, each ray's in the same order. First pass at
+// 640x480 / 5 mm 122 to 92 us, at 2 mm 186 to 149, 1280x720 / 4 mm (half)
+// 224 to 152, 320x240 / 1 cm 95 to 64.
+//
+// Blocks are named by a 30-bit tag relative to the wavefront's own origin
+// (10 bits an axis: a neighbour's tag is one addition away, and one compare
+// tests the lane's cached block), and a missing block by the heap slot
+// num_blocks, whose voxels are kept empty (NaN, weight 0), so that no read
+// tests for it. Rays that leave the 1024-block cube around the wavefront's
+// middle (16 m long at 2 mm voxels) are handed to the second pass.
+constexpr int kRayLdsEntries = 256;  // one 64-bit word each: tag + 1, slot
+constexpr uint32_t kTagX = 1u, kTagY = 1u << 10, kTagZ = 1u << 20;
+constexpr int kTagSpan = 1024;
+constexpr uint32_t kNoTag = 0xffffffffu;
+// Samples of a one-voxel run read together, and the waiting lanes' share that
+// has them served: measured at 640x480 / 5 mm, 2 mm, 1280x720 / 4 mm and
+// 320x240 / 1 cm, first pass in us: two samples 92, 149, 160, 66; one 101,
+// 153, 174, 74; three and four 110 to 118 (640x480). Serving the waiting
+// lanes when they are a third of the marching ones, as above; only when none
+// marches 135 (640x480); in every iteration 113; at half or a quarter the
+// same within 1.
+constexpr int kRayAhead = 2, kRayServe = 3;
+// Workgroups go to the eight XCDs in turn, each with an L2 of its own:
+// super-tiles of 8x8 tiles are given to one XCD, so that neighbouring rays
+// find their blocks' lines there (1280x720 160 to 152 us, 320x240 66 to 64,
+// the others the same; 4x4 and 2x2 gain less, 16x16 leaves XCDs uneven).
+constexpr int kRaySuper = 8;
+
+// The tag of block b relative to the wavefront's origin, and whether a point
+// lies well inside the cube that tags can name.
+SICP_DEV uint32_t block_tag(i3 b, uint32_t otag) {
+    return (uint32_t)b.x * kTagX + (uint32_t)b.y * kTagY + (uint32_t)b.z * kTagZ - otag;
+}
+SICP_DEV bool in_cube(v3 p, i3 o) {
+    const uint32_t x = (uint32_t)((floor_i(p.x) >> 3) - o.x - 4),
+                   y = (uint32_t)((floor_i(p.y) >> 3) - o.y - 4),
+                   z = (uint32_t)((floor_i(p.z) >> 3) - o.z - 4);
+    const uint32_t n = (uint32_t)(kTagSpan - 8);
+    return (x < n) & (y < n) & (z < n);
+}
+
+// The wavefront's lookup table: answers of the hash table, missing blocks
+// included. One wavefront per workgroup, so its accesses are ordered by its
+// own instruction order; entries are written by atomic exchange, so lanes
+// storing different blocks at one index leave one complete entry.
+template <bool kTable> struct RayTable {
+    unsigned long long* t;
+    SICP_DEV static uint32_t index(uint32_t tag) { return (tag * 0x9E3779B1u) >> 24; }
+    SICP_DEV bool get(uint32_t tag, uint32_t& slot) const {
+        if (!kTable) return false;
+        const unsigned long long e = t[index(tag)];
+        slot = (uint32_t)(e >> 32);
+        return (uint32_t)e == tag + 1u;
+    }
+    SICP_DEV void put(uint32_t tag, uint32_t slot) const {
+        if (kTable)
+            atomicExch(&t[index(tag)], ((unsigned long long)slot << 32) | (unsigned long long)(tag + 1u));
+    }
+};
+
+// The hash table's answer, num_blocks for a missing block.
+SICP_DEV uint32_t probe_slot(const MapDev& m, int bx, int by, int bz) {
+    const int s = map_lookup(m, bx, by, bz);
+    return s < 0 ? (uint32_t)m.num_blocks : (uint32_t)s;
+}
+
+// sdf (and weight) of a voxel of a slot that exists or is num_blocks.
+SICP_DEV float slot_sdf(const MapDev& m, uint32_t slot, uint32_t local) {
+    return vox_sdf(m, (size_t)slot * kBlockVoxels + local);
+}
+
+// The slots of the blocks (b & 1, b >> 1 & 1, b >> 2) past the block with tag
+// `tag0` and coordinates b0, along the axes where `n` is set; the others of
+// `s` are not written. `known`: s[0] is given. The table is asked for all of
+// them first, then the hash table for those it does not hold.
+template <bool kTable>
+SICP_DEV void box_slots(const MapDev& m, const RayTable<kTable>& lds, uint32_t tag0, i3 b0,
+                        bool nx, bool ny, bool nz, bool known, uint32_t (&s)[8]) {
+    uint32_t miss = 0;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const bool need = (!(b & 1) || nx) && (!(b & 2) || ny) && (!(b & 4) || nz) &&
+                          (b != 0 || !known);
+        if (need) {
+            const uint32_t tag = tag0 + ((b & 1) ? kTagX : 0u) + ((b & 2) ? kTagY : 0u) +
+                                 ((b & 4) ? kTagZ : 0u);
+            if (!lds.get(tag, s[b])) miss |= 1u << b;
+        }
+    }
+    while (miss) {
+        const int b = __ffs((int)miss) - 1;
+        miss &= miss - 1u;
+        const int dx = b & 1, dy = (b >> 1) & 1, dz = b >> 2;
+        const uint32_t sl = probe_slot(m, b0.x + dx, b0.y + dy, b0.z + dz);
+        lds.put(tag0 + (uint32_t)dx * kTagX + (uint32_t)dy * kTagY + (uint32_t)dz * kTagZ, sl);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[q] = q == b ? sl : s[q];
+    }
+}
+
+// Rendering::readSdfInterped (RenderScene.cu:310-343) at p. `known`: the
+// block of p's own voxel is `slot`.
+template <bool kTable>
+SICP_DEV float ray_interp(const MapDev& m, const RayTable<kTable>& lds, v3 p, uint32_t otag,
+                          bool known, uint32_t slot) {
+    const AxisPair X = axis_pair(p.x), Y = axis_pair(p.y), Z = axis_pair(p.z);
+    const i3 b0{X.v0 >> 3, Y.v0 >> 3, Z.v0 >> 3};
+    const bool nx = (X.v1 >> 3) != b0.x, ny = (Y.v1 >> 3) != b0.y, nz = (Z.v1 >> 3) != b0.z;
+    uint32_t s[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) s[b] = slot;
+    box_slots<kTable>(m, lds, block_tag(b0, otag), b0, nx, ny, nz, known, s);
+    const uint32_t ox[2] = {(uint32_t)X.v0 & 7u, (uint32_t)X.v1 & 7u};
+    const uint32_t oy[2] = {((uint32_t)Y.v0 & 7u) << 3, ((uint32_t)Y.v1 & 7u) << 3};
+    const uint32_t oz[2] = {((uint32_t)Z.v0 & 7u) << 6, ((uint32_t)Z.v1 & 7u) << 6};
+    float sd[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int cx = i & 1, cy = (i >> 1) & 1, cz = i >> 2;
+        // selects, so the slots stay in registers
+        const uint32_t a00 = cx && nx ? s[1] : s[0], a10 = cx && nx ? s[3] : s[2];
+        const uint32_t a01 = cx && nx ? s[5] : s[4], a11 = cx && nx ? s[7] : s[6];
+        const uint32_t c0 = cy && ny ? a10 : a00, c1 = cy && ny ? a11 : a01;
+        sd[i] = slot_sdf(m, cz && nz ? c1 : c0, ox[cx] | oy[cy] | oz[cz]);
+    }
+    return interp_blend(sd, X, Y, Z);
+}
+
+// One axis of the normal's reads: the voxel coordinates from the lower
+// corner of the read at -1 to the upper corner of the read at +1, four
+// consecutive ones. False where rounding makes them differ (p + 1 or p - 1
+// rounded to an integer that p's own floor does not lead to).
+struct NormalAxis {
+    int v;             // the first; the others follow
+    float fm, f0, fp;  // the fractions of the reads at -1, 0, +1
+};
+SICP_DEV bool normal_axis(float p, NormalAxis& a) {
+    const AxisPair lo = axis_pair(p + -1.0f), mid = axis_pair(p), hi = axis_pair(p + 1.0f);
+    a = NormalAxis{lo.v0, lo.frac, mid.frac, hi.frac};
+    const int v = lo.v0;
+    return lo.v1 == v + 1 && mid.v0 == v + 1 && mid.v1 == v + 2 && hi.v0 == v + 2 &&
+           hi.v1 == v + 3;
+}
+
+// Rendering::readNormal (RenderScene.cu:345-378): six interpolated reads
+// around p share 32 voxels of a 4x4x4 box in at most eight blocks, each
+// looked up and read once. A missing block reads NaN, so a read's value alone
+// decides. False without a normal.
+template <bool kTable>
+SICP_DEV void ray_normal_reads(const MapDev& m, const RayTable<kTable>& lds,
+                               const NormalAxis (&A)[3], uint32_t otag, float (&r)[6]) {
+    const i3 b0{A[0].v >> 3, A[1].v >> 3, A[2].v >> 3};
+    const bool nx = ((A[0].v + 3) >> 3) != b0.x, ny = ((A[1].v + 3) >> 3) != b0.y,
+               nz = ((A[2].v + 3) >> 3) != b0.z;
+    uint32_t s[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) s[b] = 0u;
+    box_slots<kTable>(m, lds, block_tag(b0, otag), b0, nx, ny, nz, false, s);
+    // coordinate i of an axis: its offset within its block, and whether that
+    // is the second block
+    uint32_t o[3][4];
+    bool up[3][4];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const int bb = a == 0 ? b0.x : (a == 1 ? b0.y : b0.z);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o[a][i] = ((uint32_t)(A[a].v + i) & 7u) << (3 * a);
+            up[a][i] = ((A[a].v + i) >> 3) != bb;
+        }
+    }
+    float d[4][4][4];  // [z][y][x]; only the 32 the reads touch are loaded
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        const uint32_t s00 = up[0][x] ? s[1] : s[0], s10 = up[0][x] ? s[3] : s[2];
+        const uint32_t s01 = up[0][x] ? s[5] : s[4], s11 = up[0][x] ? s[7] : s[6];
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const uint32_t t0 = up[1][y] ? s10 : s00, t1 = up[1][y] ? s11 : s01;
+#pragma unroll
+            for (int z = 0; z < 4; ++z) {
+                const int outer = (x == 0 || x == 3) + (y == 0 || y == 3) + (z == 0 || z == 3);
+                if (outer > 1) continue;
+                d[z][y][x] = slot_sdf(m, up[2][z] ? t1 : t0, o[0][x] | o[1][y] | o[2][z]);
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {  // +x, -x, +y, -y, +z, -z
+        const int a = k >> 1;
+        const int x = a == 0 ? ((k & 1) ? 0 : 2) : 1, y = a == 1 ? ((k & 1) ? 0 : 2) : 1,
+                  z = a == 2 ? ((k & 1) ? 0 : 2) : 1;
+        AxisPair X{0, 0, A[0].f0}, Y{0, 0, A[1].f0}, Z{0, 0, A[2].f0};
+        (a == 0 ? X : (a == 1 ? Y : Z)).frac = (k & 1) ? A[a].fm : A[a].fp;
+        const float sd[8] = {d[z][y][x],         d[z][y][x + 1],         d[z][y + 1][x],
+                             d[z][y + 1][x + 1], d[z + 1][y][x],         d[z + 1][y][x + 1],
+                             d[z + 1][y + 1][x], d[z + 1][y + 1][x + 1]};
+        r[k] = interp_blend(sd, X, Y, Z);
+    }
+}
+template <bool kTable>
+SICP_DEV bool ray_normal(const MapDev& m, const RayTable<kTable>& lds, v3 p, uint32_t otag,
+                         const PoseF& pose, v3& n) {
+    float r[6];
+    NormalAxis A[3];
+    const bool ax = normal_axis(p.x, A[0]), ay = normal_axis(p.y, A[1]),
+               az = normal_axis(p.z, A[2]);
+    if (ax && ay && az) {
+        ray_normal_reads<kTable>(m, lds, A, otag, r);
+    } else {
+#pragma unroll 1
+        for (int k = 0; k < 6; ++k) {
+            const float d = (k & 1) ? -1.0f : 1.0f;
+            const v3 q{k < 2 ? p.x + d : p.x, (k >> 1) == 1 ? p.y + d : p.y, k > 3 ? p.z + d : p.z};
+            const float v = ray_interp<kTable>(m, lds, q, otag, false, 0u);
+#pragma unroll
+            for (int j = 0; j < 6; ++j) r[j] = j == k ? v : r[j];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+        if (isnan_(r[k]) || r[k] == 1.0f) return false;
+    n = normalised(mv(pose.Rinv, mk(r[0] - r[1], r[2] - r[3], r[4] - r[5])));
+    return true;
+}
+
+// 8x8-pixel wavefronts (the zRange tile).
+template <bool kHalf, bool kTable>
+__global__ __launch_bounds__(64, 5) void raycast_kernel(MapDev map, View<float4> vmap,
                                                      View<float4> nmap, View<float> zmin,
                                                      View<float> zmax, PoseArg pa, RayArgs g,
                                                      const int* gate, const uint32_t* nonempty) {
-    const int x = blockIdx.x * 8 + (threadIdx.x & 7);
-    const int y = blockIdx.y * 8 + (threadIdx.x >> 3);
+    MapDev m = map;
+    m.half = kHalf;  // a constant: no test of the form per read
+    constexpr uint32_t kSuperTiles = kRaySuper * kRaySuper;
+    const uint32_t xcd = blockIdx.x & 7u, turn = blockIdx.x >> 3;
+    const uint32_t super = turn / kSuperTiles * 8u + xcd, in = turn % kSuperTiles;
+    const uint32_t across = ((uint32_t)g.tcols + kRaySuper - 1u) / kRaySuper;
+    const int bx = (int)(super % across * kRaySuper + in % kRaySuper);
+    const int by = (int)(super / across * kRaySuper + in / kRaySuper);
+    if (bx >= g.tcols || by >= g.trows) return;
+    const int x = bx * 8 + (threadIdx.x & 7);
+    const int y = by * 8 + (threadIdx.x >> 3);
     // the tile's depth range, the pose and the gates, loaded together
     const int ty = min(y, g.rows - 1) >> 3, tx = min(x, g.cols - 1) >> 3;
     const float z0 = early_load(&zmin.at(ty, tx)), z1 = early_load(&zmax.at(ty, tx));
@@ -548,71 +707,197 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(MapDev m, View<float4> v
     const uint32_t any = early_load(nonempty);
     const PoseF pose = load_pose(pa);
     if ((open == 0) | (any == 0u)) return;
-    // One wavefront per workgroup: the table is cleared before any lane uses
-    // it, and its accesses are ordered by the wavefront's own instruction
-    // order (no barrier needed).
-    __shared__ unsigned long long lookup_table[kRayLdsEntries];
+    __shared__ unsigned long long entries[kTable ? kRayLdsEntries : 1];
+    if (kTable) {
 #pragma unroll
-    for (int i = 0; i < kRayLdsEntries / 64; ++i) lookup_table[threadIdx.x + 64 * i] = 0ull;
-    if (x >= g.cols || y >= g.rows) return;
+        for (int i = 0; i < kRayLdsEntries / 64; ++i) entries[threadIdx.x + 64 * i] = 0ull;
+    }
+    const RayTable<kTable> lds{entries};
+    const bool inside = x < g.cols && y < g.rows;
     const float nan = qnanf();
     float4 vout = make_float4(nan, nan, nan, nan);
     float4 nout = vout;
-    Ray ray;
-    bool deferred = false;
+    Ray ray{};
+    const bool hits = inside && ray_setup(m, z0, z1, pose, g, x, y, ray);
+    // kMarch: takes samples; kProbe, kInterp: waits for a table probe or an
+    // interpolated read of its current sample; kEnd: the loop is over
+    enum { kMarch, kProbe, kInterp, kEnd };
+    int status = hits ? kMarch : kEnd;
+    bool deferred = false, back_face = false, crossed = false;
     v3 result{0.f, 0.f, 0.f};
-    float dist_s = 0.f, sdf = 1.0f;
-    if (ray_setup(m, z0, z1, pose, g, x, y, ray)) {
-        result = ray.start;
-        dist_s = ray.dist_s;
-        bool valid_sdf = false, back_face = false;
-        float step, prev_sdf;
-        BlockCache cache{0, 0, 0, -1,
-                         g.lds_block_table && m.num_blocks < (1 << 21) - 2 ? lookup_table
-                                                                            : nullptr};
-        int iters = 0;
-        while (dist_s < ray.dist_e) {
-            if (iters == g.first_pass_samples) {
-                deferred = true;
-                break;
+    float dist_s = 0.f, sdf = 1.0f, prev_sdf = 1.0f;
+    // The tags' origin: the block in the middle of the first ray, less half
+    // the span. A ray whose ends lie in the cube stays in it.
+    uint32_t otag = 0;
+    i3 o{0, 0, 0};
+    {
+        const unsigned long long some = __ballot(hits);
+        if (some) {
+            v3 mid{0.f, 0.f, 0.f};
+            if (hits) {
+                result = ray.start;
+                dist_s = ray.dist_s;
+                mid = add(ray.start, scale(0.5f * (ray.dist_e - ray.dist_s), ray.dir));
             }
-            ++iters;
-            prev_sdf = sdf;
-            long k = find_voxel_i(m, floor_i(result.x), floor_i(result.y), floor_i(result.z), cache,
-                                  valid_sdf);
-            if (k < 0) {
-                sdf = nan;
-            } else {
-                uint32_t wt;
-                vox_load(m, (size_t)k, sdf, wt);
-                if (wt == 0u) valid_sdf = false;
-            }
-            if (!valid_sdf) {
-                step = (float)kBlockSide;
-            } else {
-                if (sdf <= 0.1f && sdf >= -0.5f) sdf = read_sdf_interped(m, result, cache, valid_sdf);
-                if (prev_sdf < 0.f && sdf >= 0.f) {
-                    back_face = true;
-                    break;
+            const int src = __ffsll((long long)some) - 1;
+            o.x = (__builtin_amdgcn_readlane(floor_i(mid.x), src) >> 3) - kTagSpan / 2;
+            o.y = (__builtin_amdgcn_readlane(floor_i(mid.y), src) >> 3) - kTagSpan / 2;
+            o.z = (__builtin_amdgcn_readlane(floor_i(mid.z), src) >> 3) - kTagSpan / 2;
+            otag = (uint32_t)o.x * kTagX + (uint32_t)o.y * kTagY + (uint32_t)o.z * kTagZ;
+            if (hits) {
+                const v3 e = add(ray.start, scale(ray.dist_e - ray.dist_s, ray.dir));
+                if (!in_cube(ray.start, o) || !in_cube(e, o)) {
+                    deferred = true;
+                    status = kEnd;
                 }
-                if (prev_sdf > 0.f && sdf <= 0.f) break;
-                step = 1.0f;
             }
-            result = add(result, scale(step, ray.dir));
-            dist_s += step;
         }
-        if (!deferred && !back_face && sdf <= 0.0f) {
-            step = sdf * m.step_scale;
-            result = add(result, scale(step, ray.dir));
-            sdf = read_sdf_interped(m, result, cache, valid_sdf);
-            step = sdf * m.step_scale;
-            result = add(result, scale(step, ray.dir));
+    }
+    const v3 dir8 = scale((float)kBlockSide, ray.dir);
+    uint32_t tag = kNoTag, slot = 0;  // the lane's last lookup
+    int iters = 0;
+    for (;;) {
+        for (;;) {
+            const int marching = __popcll(__ballot(status == kMarch));
+            const int waiting = __popcll(__ballot(status == kProbe || status == kInterp));
+            if (marching == 0 || waiting * kRayServe > marching) break;
+            if (status != kMarch) continue;
+            if (!(dist_s < ray.dist_e)) {
+                status = kEnd;
+            } else if (iters == g.first_pass_samples) {
+                deferred = true;
+                status = kEnd;
+            } else {
+                const int vx = floor_i(result.x), vy = floor_i(result.y), vz = floor_i(result.z);
+                const uint32_t t = block_tag(i3{vx >> 3, vy >> 3, vz >> 3}, otag);
+                bool found = t == tag;
+                if (!found) {
+                    found = lds.get(t, slot);
+                    tag = found ? t : kNoTag;
+                }
+                if (!found) {
+                    status = kProbe;
+                } else if (slot == (uint32_t)m.num_blocks) {  // no block here
+                    prev_sdf = sdf;
+                    sdf = nan;
+                    ++iters;
+                    result = add(result, dir8);
+                    dist_s += (float)kBlockSide;
+                } else {
+                    // This sample and those that one-voxel steps would take
+                    // next in the same block, their loads in flight together
+                    v3 P[kRayAhead];
+                    bool same[kRayAhead];
+                    float s[kRayAhead];
+                    uint32_t wt[kRayAhead];
+                    P[0] = result;
+                    same[0] = true;
+                    uint32_t local = (uint32_t)local_of(vx, vy, vz);
+#pragma unroll
+                    for (int j = 0; j < kRayAhead; ++j) {
+                        if (j > 0) {
+                            P[j] = add(P[j - 1], ray.dir);
+                            const int wx = floor_i(P[j].x), wy = floor_i(P[j].y),
+                                      wz = floor_i(P[j].z);
+                            same[j] = same[j - 1] &&
+                                      (((wx ^ vx) | (wy ^ vy) | (wz ^ vz)) & ~7) == 0;
+                            local = same[j] ? (uint32_t)local_of(wx, wy, wz) : local;
+                        }
+                        vox_load(m, (size_t)slot * kBlockVoxels + local, s[j], wt[j]);
+                    }
+                    bool plain = true;
+#pragma unroll
+                    for (int j = 0; j < kRayAhead; ++j) {
+                        if (j > 0)
+                            plain = plain && same[j] && dist_s < ray.dist_e &&
+                                    iters != g.first_pass_samples;
+                        if (!plain) continue;
+                        prev_sdf = sdf;
+                        sdf = s[j];
+                        const bool valid = wt[j] != 0u;
+                        const bool band = valid && sdf <= 0.1f && sdf >= -0.5f;
+                        back_face = valid && prev_sdf < 0.f && sdf >= 0.f;
+                        crossed = valid && prev_sdf > 0.f && sdf <= 0.f;
+                        plain = valid && !band && !back_face && !crossed;
+                        if (band) {
+                            status = kInterp;
+                        } else {
+                            ++iters;
+                            if (back_face || crossed) {
+                                status = kEnd;
+                            } else {
+                                const float step = valid ? 1.0f : (float)kBlockSide;
+                                result = add(result, scale(step, ray.dir));
+                                dist_s += step;
+                            }
+                        }
+                    }
+                }
+            }
+        }
+        if (!__any(status != kEnd)) break;
+        if (status == kProbe) {
+            // In a run of missing blocks the block of the next block-width
+            // step is looked up too, both buckets' reads in flight at once
+            const bool run = isnan_(sdf);
+            const v3 q = add(result, dir8);
+            const i3 b{floor_i(result.x) >> 3, floor_i(result.y) >> 3, floor_i(result.z) >> 3};
+            i3 c{floor_i(q.x) >> 3, floor_i(q.y) >> 3, floor_i(q.z) >> 3};
+            if (!run) c = b;
+            const Probe pb = probe_load(m.table, m.nb, m.nb_mask, b.x, b.y, b.z);
+            const Probe pc = probe_load(m.table, m.nb, m.nb_mask, c.x, c.y, c.z);
+            const int sb = probe_result(pb, m.excess);
+            tag = block_tag(b, otag);
+            slot = sb < 0 ? (uint32_t)m.num_blocks : (uint32_t)sb;
+            lds.put(tag, slot);
+            if (run && sb < 0) {  // this sample: no block here
+                const int sc = probe_result(pc, m.excess);
+                ++iters;
+                result = q;
+                dist_s += (float)kBlockSide;
+                tag = block_tag(c, otag);
+                slot = sc < 0 ? (uint32_t)m.num_blocks : (uint32_t)sc;
+                lds.put(tag, slot);
+            }
+            status = kMarch;
+        }
+        if (status == kInterp) {
+            sdf = ray_interp<kTable>(m, lds, result, otag, true, slot);
+            ++iters;
+            back_face = prev_sdf < 0.f && sdf >= 0.f;
+            crossed = prev_sdf > 0.f && sdf <= 0.f;
+            if (back_face || crossed) {
+                status = kEnd;
+            } else {
+                result = add(result, ray.dir);
+                dist_s += 1.0f;
+                status = kMarch;
+            }
+        }
+    }
+    if (hits && !deferred && !back_face && sdf <= 0.0f) {
+        // the state the second pass would resume from, should it be needed
+        const v3 at = result;
+        const float sdf_in = crossed ? prev_sdf : sdf;
+        result = add(result, scale(sdf * m.step_scale, ray.dir));
+        bool ok = in_cube(result, o);
+        if (ok) {
+            sdf = ray_interp<kTable>(m, lds, result, otag, false, 0u);
+            result = add(result, scale(sdf * m.step_scale, ray.dir));
+            // (a NaN position has no normal: its reads would be NaN)
+            const bool number = !isnan_(result.x) && !isnan_(result.y) && !isnan_(result.z);
+            ok = !number || in_cube(result, o);
             v3 normal;
-            if (read_normal(m, result, cache, pose, normal)) {
+            if (ok && number && ray_normal<kTable>(m, lds, result, otag, pose, normal)) {
                 v3 r = mv(pose.Rinv, sub(scale(result, m.voxel), pose.t));
                 vout = make_float4(r.x, r.y, r.z, 1.0f);
                 nout = make_float4(normal.x, normal.y, normal.z, 1.0f);
             }
+        }
+        if (!ok) {
+            deferred = true;
+            result = at;
+            sdf = sdf_in;
         }
     }
     // Hand-over: one queue reservation per wavefront.
@@ -631,6 +916,7 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(MapDev m, View<float4> v
         }
         if (deferred) return;  // the second pass writes this pixel
     }
+    if (!inside) return;
     vmap.at(y, x) = vout;
     nmap.at(y, x) = nout;
 }
@@ -1111,7 +1397,7 @@ int launch_raycast_adjoint(MapDev m, View<float> zmin, View<float> zmax, PoseArg
                            const int32_t* pixels, int n, const float* grad_v,
                            const float* grad_n, float* grad_sdf, float* grad_px,
                            double* partials, double* grad_pose, hipStream_t s) {
-    AdjointArgs a{RayArgs{invfx, invfy, cx, cy, cols, rows, 0, 0}, pixels, n, grad_v, grad_n,
+    AdjointArgs a{RayArgs{invfx, invfy, cx, cy, cols, rows, 0, 0, 0}, pixels, n, grad_v, grad_n,
                   grad_sdf, grad_px, partials};
     int nb = (int)div_up(n > 0 ? n : 1, kAdjThreads);
     if (nb > kAdjMaxBlocks) nb = kAdjMaxBlocks;
@@ -1159,16 +1445,20 @@ int launch_raycast_gated(MapDev m, View<float4> vmap, View<float4> nmap, View<fl
         tune.second_pass_workgroups < 1 || tune.second_pass_workgroups > kRayTuneMaxWorkgroups ||
         (tune.lds_block_table != 0 && tune.lds_block_table != 1))
         return invalid("raycast: tuning outside 1..4096 samples, 1..65536 workgroups, table 0/1");
-    RayArgs g{invfx, invfy, cx, cy, vmap.cols, vmap.rows, tune.first_pass_samples,
-              tune.lds_block_table};
+    RayArgs g{invfx, invfy, cx, cy, vmap.cols, vmap.rows, (int)div_up(vmap.cols, 8), (int)div_up(vmap.rows, 8), tune.first_pass_samples};
     if (!gate) gate = m.one;
     if (!nonempty) nonempty = reinterpret_cast<const uint32_t*>(m.one);
     if (!queue_cleared) {
         ray_queue_reset_kernel<<<1, 1, 0, s>>>(m.rq_count);
         SICP_LAUNCH_CHECK("ray_queue_reset_kernel");
     }
-    dim3 grid(div_up(vmap.cols, 8), div_up(vmap.rows, 8));
-    raycast_kernel<<<grid, 64, 0, s>>>(m, vmap, nmap, zmin, zmax, pose, g, gate, nonempty);
+    // super-tiles rounded up to one for each XCD
+    const unsigned grid = div_up((long)div_up(g.tcols, kRaySuper) * div_up(g.trows, kRaySuper), 8) *
+                          8u * kRaySuper * kRaySuper;
+    auto* first = m.half ? (tune.lds_block_table ? raycast_kernel<true, true> : raycast_kernel<true, false>)
+                         : (tune.lds_block_table ? raycast_kernel<false, true>
+                                                 : raycast_kernel<false, false>);
+    first<<<grid, 64, 0, s>>>(m, vmap, nmap, zmin, zmax, pose, g, gate, nonempty);
     SICP_LAUNCH_CHECK("raycast_kernel");
     raycast_long_kernel<<<tune.second_pass_workgroups, kRayLongThreads, 0, s>>>(
         m, vmap, nmap, zmin, zmax, pose, g, gate, nonempty);

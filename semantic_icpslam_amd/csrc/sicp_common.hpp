@@ -102,7 +102,12 @@ SICP_DEV PoseF to_pose(const sicp_pose_f& p) {
     o.t = v3{p.t[0], p.t[1], p.t[2]};
     return o;
 }
-SICP_DEV PoseF load_pose(const PoseArg& a) { return to_pose(a.dev ? *a.dev : a.val); }
+// One branch on the pointer, each side whole (a select of the two sources
+// becomes a branch and a load per number).
+SICP_DEV PoseF load_pose(const PoseArg& a) {
+    if (a.dev) return to_pose(*a.dev);
+    return to_pose(a.val);
+}
 
 inline PoseArg make_pose_arg(const sicp_pose_f* host, const sicp_pose_f* dev) {
     PoseArg a{};
