@@ -166,6 +166,8 @@ int map_alloc(const sicp_map_config& cfg, sicp_map** out) {
 void map_free(sicp_map* m) {
     if (!m) return;
     for (void* p : m->owned) (void)hipFree(p);
+    if (m->mesh_counts) (void)hipFree(m->mesh_counts);
+    if (m->mesh_total) (void)hipHostFree(m->mesh_total);
     delete m;
 }
 

@@ -46,7 +46,7 @@ def main():
         f.write("// Generated by gen_mc_table.py from the reference's triangle table\n"
                 "// (Mapping/Constant.h:39-296): per sign case, the edge indices of its\n"
                 "// triangles in hexadecimal, three per triangle.\n"
-                "static const char* const kMcTriangles[256] = {\n")
+                "static constexpr const char* kMcTriangles[256] = {\n")
         for c in range(0, 256, 8):
             f.write("    " + " ".join('"%s",' % "".join("%x" % v for v in rows[k])
                                       for k in range(c, c + 8)) + "\n")

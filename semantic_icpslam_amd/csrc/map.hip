@@ -461,77 +461,6 @@ SICP_DEV uint2 chunk_offset(const uint32_t* sums, uint32_t w, uint32_t n) {
     return r;
 }
 
-__global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_t* in,
-                                                                   const uint32_t* n_dev,
-                                                                   uint32_t cap,
-                                                                   uint32_t* partials) {
-    const uint32_t n = n_dev ? min(*n_dev, cap) : cap;
-    const uint32_t base = blockIdx.x * kScanChunk + threadIdx.x * kScanPerThread;
-    uint32_t s = 0;
-#pragma unroll
-    for (int k = 0; k < kScanPerThread; ++k)
-        if (base + k < n) s += in[base + k];
-    uint32_t tot;
-    block_exclusive_scan(s, &tot);
-    if (threadIdx.x == 0) partials[blockIdx.x] = tot;
-}
-
-__global__ __launch_bounds__(1024) void scan_partials_kernel(uint32_t* partials, uint32_t nchunks,
-                                                             uint32_t* total_out) {
-    __shared__ uint32_t wave_tot[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t v[4], s = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        uint32_t idx = threadIdx.x * 4 + k;
-        v[k] = idx < nchunks ? partials[idx] : 0u;
-        s += v[k];
-    }
-    uint32_t inc = s;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        uint32_t t = __shfl_up(inc, off, 64);
-        if (lane >= off) inc += t;
-    }
-    if (lane == 63) wave_tot[wave] = inc;
-    __syncthreads();
-    uint32_t wbase = 0, tot = 0;
-    for (int w = 0; w < 16; ++w) {
-        if (w < wave) wbase += wave_tot[w];
-        tot += wave_tot[w];
-    }
-    uint32_t run = wbase + inc - s;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        uint32_t idx = threadIdx.x * 4 + k;
-        if (idx < nchunks) partials[idx] = run;
-        run += v[k];
-    }
-    if (threadIdx.x == 0) *total_out = tot;
-}
-
-__global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(const uint32_t* in,
-                                                                  uint32_t* out,
-                                                                  const uint32_t* n_dev,
-                                                                  uint32_t cap,
-                                                                  const uint32_t* partials) {
-    const uint32_t n = n_dev ? min(*n_dev, cap) : cap;
-    const uint32_t base = blockIdx.x * kScanChunk + threadIdx.x * kScanPerThread;
-    uint32_t v[kScanPerThread], s = 0;
-#pragma unroll
-    for (int k = 0; k < kScanPerThread; ++k) {
-        v[k] = (base + k < n) ? in[base + k] : 0u;
-        s += v[k];
-    }
-    uint32_t tot;
-    uint32_t run = partials[blockIdx.x] + block_exclusive_scan(s, &tot);
-#pragma unroll
-    for (int k = 0; k < kScanPerThread; ++k) {
-        if (base + k < n) out[base + k] = run;
-        run += v[k];
-    }
-}
-
 // ------------------------------------------------------------ visibility --
 struct VisArgs {
     float fx, fy, cx, cy;
@@ -926,20 +855,6 @@ static bool vis_chunks(const MapDev& m, uint32_t& nchunks) {
     if (nchunks == 0) nchunks = 1;
     return false;
 }
-int launch_scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_dev, uint32_t cap,
-                    uint32_t* partials, uint32_t* total_out, hipStream_t s) {
-    uint32_t nchunks = div_up(cap, kScanChunk);
-    if (nchunks == 0) nchunks = 1;
-    if (nchunks > kScanMaxChunks) return invalid("scan longer than 4M elements");
-    scan_reduce_kernel<<<nchunks, kScanThreads, 0, s>>>(in, n_dev, cap, partials);
-    SICP_LAUNCH_CHECK("scan_reduce_kernel");
-    scan_partials_kernel<<<1, 1024, 0, s>>>(partials, nchunks, total_out);
-    SICP_LAUNCH_CHECK("scan_partials_kernel");
-    scan_apply_kernel<<<nchunks, kScanThreads, 0, s>>>(in, out, n_dev, cap, partials);
-    SICP_LAUNCH_CHECK("scan_apply_kernel");
-    return SICP_OK;
-}
-
 int launch_map_reset(MapDev m, MapCounters* ctr, AllocScratch a, hipStream_t s) {
     reset_table_kernel<<<2048, 256, 0, s>>>(m, a, a.req_mask + 1);
     SICP_LAUNCH_CHECK("reset_table_kernel");

@@ -1,6 +1,7 @@
 // sicp_internal.hpp — host-side objects behind the opaque C ABI handles.
 #pragma once
 
+#include <atomic>
 #include <vector>
 
 #include "sicp_kernels.hpp"
@@ -14,7 +15,10 @@ struct sicp_map {
     uint32_t* unify_snap = nullptr;    // neighbour label pass: label snapshot, num_blocks * 512
     uint32_t* unify_mark = nullptr;    // per heap slot: epoch of the last snapshot
     uint32_t unify_epoch = 0;
-    std::vector<void*> owned;          // every device allocation of the map
+    std::atomic<bool> mesh_lent{false};  // mesh extraction: the memory below is in a call's use
+    uint32_t* mesh_counts = nullptr;   // device
+    uint32_t* mesh_total = nullptr;    // pinned host
+    std::vector<void*> owned;          // every other device allocation of the map
 };
 
 namespace sicp {

@@ -331,8 +331,4 @@ int launch_raycast_adjoint(MapDev m, View<float> zmin, View<float> zmax, PoseArg
                            double* partials, double* grad_pose, hipStream_t s);
 size_t raycast_adjoint_scratch_bytes();
 
-// Device exclusive scan of `n_dev` (device count, at most `cap`) u32 values.
-int launch_scan_u32(const uint32_t* in, uint32_t* out, const uint32_t* n_dev, uint32_t cap,
-                    uint32_t* partials, uint32_t* total_out, hipStream_t s);
-
 }  // namespace sicp
