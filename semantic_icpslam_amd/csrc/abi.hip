@@ -103,7 +103,7 @@ int map_alloc(const sicp_map_config& cfg, sicp_map** out) {
         (rc = dmalloc(m, &a.bucket_leader, nb)) || (rc = dmalloc(m, &a.bucket_head, nb)) ||
         (rc = dmalloc(m, &a.pending_next, q)) || (rc = dmalloc(m, &a.vis_flags, nblk)) ||
         (rc = dmalloc(m, &a.fuse_counts, (size_t)kFuseBlocks * 4)) ||
-        (rc = dmalloc(m, &d.rq, px)) || (rc = dmalloc(m, &d.rq_count, 1))) {
+        (rc = dmalloc(m, &a.pixels, px)) || (rc = dmalloc(m, &d.rq, px)) || (rc = dmalloc(m, &d.rq_count, 1))) {
         map_free(m);
         return rc;
     }
@@ -541,19 +541,16 @@ int sicp_fuse_map_color(sicp_map* map, sicp_image depth_f32, sicp_image rgb_u8x3
     PoseArg pa = pose_arg(pose_host, pose_dev);
     // FuseMapColor checks visibility against the map's own depth range
     // (FuseMap.cu:1080-1081); the allocation's last launch flags the blocks.
-    int rc = launch_allocate(map->dev, map->ctr, map->alloc, view<float>(depth_f32), pa, K,
+    const FuseImages im{view<uint8_t>(rgb_u8x3),
+                        num_detection > 0 ? view<float4>(nmap_f4) : View<float4>{},
+                        num_detection > 0 ? view<uint8_t>(mask_u8) : View<uint8_t>{},
+                        num_detection};
+    int rc = launch_allocate(map->dev, map->ctr, map->alloc, view<float>(depth_f32), im, pa, K,
                              VisFrustum{c, r, map->cfg.depth_max, map->cfg.depth_min}, nullptr, s);
     if (rc) return rc;
     rc = launch_visible_compact(map->dev, map->ctr, map->alloc, map->visible, nullptr, s);
     if (rc) return rc;
-    sicp_image nm = nmap_f4, mk = mask_u8;
-    if (num_detection <= 0) {
-        nm = depth_f32;  // unused by the kernel when num_detection <= 0
-        mk = depth_f32;
-    }
-    rc = launch_fuse(map->dev, map->ctr, map->visible, view<float>(depth_f32),
-                     view<uint8_t>(rgb_u8x3), view<float4>(nm), view<uint8_t>(mk), num_detection,
-                     pa, K, map->alloc.fuse_counts, nullptr, s);
+    rc = launch_fuse(map->dev, map->ctr, map->alloc, map->visible, c, r, im, pa, K, nullptr, s);
     if (rc) return rc;
     rc = launch_fuse_count(map->ctr, map->alloc.fuse_counts, nullptr, s);
     if (rc) return rc;

@@ -140,9 +140,27 @@ struct AllocArgs {
     int cols, rows;
 };
 
+// What the fusion reads of a pixel, in eight bytes: the depth (NaN where it
+// is none or outside the range) and r, g, b and the label. The fusion gathers
+// it once per voxel; gathering the images themselves (depth, three colour
+// bytes, a float4 normal of which x alone decides, the label) kept the units
+// that return gathered data busy four fifths of its time. The depth's sign
+// tells whether the pixel has a normal, where valid depths are positive.
+SICP_DEV bool depth_sign_free(const MapDev& m) { return m.dmin > 0.f; }
+SICP_DEV uint2 pack_pixel(const MapDev& m, float d, const FuseImages& im, int x, int y) {
+    const uint8_t* c = &im.rgb.at(y, 3 * x);
+    uint32_t w = (uint32_t)c[0] | (uint32_t)c[1] << 8 | (uint32_t)c[2] << 16;
+    if (isnan_(d) || d > m.dmax || d < m.dmin) d = qnanf();
+    if (im.num_detection > 0) {
+        w |= (uint32_t)im.mask.at(y, x) << 24;
+        if (depth_sign_free(m) && isnan_(im.nmap.at(y, x).x)) d = -d;
+    }
+    return make_uint2(__float_as_uint(d), w);
+}
+
 __global__ __launch_bounds__(256) void alloc_mark_kernel(MapDev m, MapCounters* ctr,
                                                          AllocScratch a, View<float> depth,
-                                                         PoseArg pa, AllocArgs g,
+                                                         FuseImages im, PoseArg pa, AllocArgs g,
                                                          const int* gate) {
     if (gate && *gate == 0) return;
     const int x = blockIdx.x * 64 + (threadIdx.x & 63);
@@ -150,6 +168,7 @@ __global__ __launch_bounds__(256) void alloc_mark_kernel(MapDev m, MapCounters* 
     if (x >= g.cols || y >= g.rows) return;
     const int i = y * g.cols + x;
     const PoseF pose = load_pose(pa);
+    a.pixels[i] = pack_pixel(m, depth.at(y, x), im, x, y);
     MarchSetup ms;
     unsigned long long mask = 0ull;
     if (march_setup(m, depth, x, y, pose, g.invfx, g.invfy, g.cx, g.cy, ms)) {
@@ -596,7 +615,7 @@ __global__ __launch_bounds__(kScanThreads) void vis_compact_kernel(MapDev m, Map
 struct FuseArgs {
     float fx, fy, cx, cy;
     int cols, rows;
-    int num_detection;
+    float trunc_rcp;  // 1 / truncation, rounded to nearest
 };
 
 SICP_DEV int palette_channel(int c, int L) {
@@ -605,16 +624,36 @@ SICP_DEV int palette_channel(int c, int L) {
     return prod % 255;
 }
 
-SICP_DEV uint8_t u8i(float v) { return (uint8_t)(uint32_t)(int)v; }
+SICP_DEV int u8i(float v) { return (int)(uint8_t)(uint32_t)(int)v; }
 
-// Fusion::createVoxels (FuseMap.cu:432-507) and, when num_detection > 0,
+// The running mean of one colour channel, (float)(c w + c0) / (w + 1) truncated:
+// an integer quotient of at most 65280 by at most 256, so half a unit of the
+// dividend more keeps an approximate reciprocal (within an ulp) exact.
+SICP_DEV int mean_channel(int c, int w, int c0, float y) {
+    return (int)(((float)(c * w + c0) + 0.5f) * y);
+}
+
+// Fusion::createVoxels (FuseMap.cu:432-507) and, with kSem,
 // Fusion::analyzeSemantics (FuseMap.cu:509-668) applied once to the same voxel.
-__global__ __launch_bounds__(256) void fuse_kernel(MapDev m, const MapCounters* ctr,
-                                                   const sicp_block* visible, View<float> depth,
-                                                   View<uint8_t> rgb, View<float4> nmap,
-                                                   View<uint8_t> mask, PoseArg pa, FuseArgs g,
+//
+// What bounds it: the return of gathered and streamed records to the lanes
+// and the latency of each voxel's chain (project, gather the pixel, read the
+// records, update, write), with the divisions' instructions on top. So a voxel
+// gathers one eight-byte pixel record (pack_pixel), reads eight of the
+// semantic record's twelve bytes, writes the four that a repeated label
+// changes, forms its quotients from shared reciprocals, and takes a new voxel
+// down the same path (one code for eight z steps: unrolled it did not stay in
+// the instruction cache). 640x480 / 5 mm 35.5 to 23.3 us a launch, at 2 mm
+// 307 to 172, 1280x720 / 4 mm (half) 53.7 to 32.4, 320x240 / 1 cm 25 to 16.3;
+// the packing adds 0.5 to 2 us to the allocation's first launch.
+template <bool kHalf, bool kSem>
+__global__ __launch_bounds__(256) void fuse_kernel(MapDev map, const MapCounters* ctr,
+                                                   const sicp_block* visible,
+                                                   const uint2* pixels, View<float4> nmap,
+                                                   PoseArg pa, FuseArgs g,
                                                    uint32_t* wave_counts, const int* gate) {
     if (gate && *gate == 0) return;
+    const MapDev& m = map;
     const uint32_t nvis = ctr->visible;
     const PoseF pose = load_pose(pa);
     const int lane = threadIdx.x & 63;
@@ -622,6 +661,7 @@ __global__ __launch_bounds__(256) void fuse_kernel(MapDev m, const MapCounters* 
     const uint32_t wave0 = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const uint32_t nwaves = gridDim.x * (blockDim.x >> 6);
     const float T = m.trunc;
+    const bool sign = kSem && depth_sign_free(m);
     uint32_t updated = 0;
     // Grid-stride over the visible blocks; the next block's record is loaded
     // while the current block is fused.
@@ -632,155 +672,167 @@ __global__ __launch_bounds__(256) void fuse_kernel(MapDev m, const MapCounters* 
         const size_t vbase = (size_t)blk.slot * kBlockVoxels + lane;
         const int bx = blk.x * kBlockSide + lx, by = blk.y * kBlockSide + ly;
         const int bz = blk.z * kBlockSide;
+#pragma unroll 1
         for (int lz = 0; lz < kBlockSide; ++lz) {
             v3 pw{(float)bx * m.voxel, (float)by * m.voxel, (float)(bz + lz) * m.voxel};
             v3 pc = mv(pose.Rinv, sub(pw, pose.t));
-            int u = (int)(g.fx * pc.x / pc.z + g.cx);
-            int v = (int)(g.fy * pc.y / pc.z + g.cy);
+            // fx x / z and fy y / z by one reciprocal; the division for a z
+            // whose reciprocal two steps do not give (all ones) or far out
+            const float ax = g.fx * pc.x, ay = g.fy * pc.y;
+            const float y0 = __builtin_amdgcn_rcpf(pc.z);
+            const float yz = rcp_step(pc.z, rcp_step(pc.z, y0));
+            float qx = quotient(ax, pc.z, yz), qy = quotient(ay, pc.z, yz);
+            if (!(fits(pc.z) && fabsf(ax) <= 0x1p60f && fabsf(ay) <= 0x1p60f &&
+                  (__float_as_uint(pc.z) & 0x7fffffu) != 0x7fffffu)) {
+                qx = ax / pc.z;
+                qy = ay / pc.z;
+            }
+            int u = (int)(qx + g.cx);
+            int v = (int)(qy + g.cy);
             if (u < 0 || v < 0 || u >= g.cols || v >= g.rows) continue;
-            float dp = depth.at(v, u);
-            if (isnan_(dp) || dp > m.dmax || dp < m.dmin) continue;
+            const uint2 px = pixels[v * g.cols + u];
+            float dp = __uint_as_float(px.x);
+            if (isnan_(dp)) continue;
+            const bool normal = !sign || dp > 0.f;
+            if (sign) dp = fabsf(dp);
             float sdf = dp - pc.z;
             if (!(sdf >= -T)) continue;
-            sdf = fminf(1.0f, sdf / T);
-            const uint8_t* c = &rgb.at(v, 3 * u);
-            const uint8_t c0 = c[0], c1 = c[1], c2 = c[2];
+            {
+                float q = quotient(sdf, T, g.trunc_rcp);
+                if (!(fits(sdf) && fits(T))) q = sdf / T;
+                sdf = fminf(1.0f, q);
+            }
+            const int c0 = (int)(px.y & 0xffu), c1 = (int)(px.y >> 8 & 0xffu),
+                      c2 = (int)(px.y >> 16 & 0xffu);
             const size_t kv = vbase + (size_t)lz * 64;
-            sicp_voxel_sem* sp = m.sem + kv;
-            sicp_voxel_geom gv;
-            sicp_voxel_sem sh;  // half form: the whole semantic record (it holds the colour)
-            if (m.half) {
-                const uint32_t w = m.geom_h[kv];
-                sh = *sp;
-                gv.sdf = h2f(w);
-                gv.weight = (uint8_t)((w >> 16) & 0xffu);
-                gv.r = sh.pad[0];
-                gv.g = sh.pad[1];
-                gv.b = sh.pad[2];
+            uint32_t* sp = (uint32_t*)(m.sem + kv);
+            // The records; an empty voxel's count as zeros, from which the
+            // updates below make a new voxel's (a mean over no weight is the
+            // frame's own value).
+            float old;
+            int w, r, gr, b;
+            uint32_t s0 = 0u, s1 = 0u, s2 = 0u;
+            if (kHalf) {  // the whole semantic record: it holds the colour
+                const uint32_t wd = m.geom_h[kv];
+                s0 = sp[0];
+                s1 = sp[1];
+                s2 = sp[2];
+                old = h2f(wd);
+                w = (int)(wd >> 16 & 0xffu);
+                r = (int)(s2 >> 8 & 0xffu);
+                gr = (int)(s2 >> 16 & 0xffu);
+                b = (int)(s2 >> 24);
             } else {
-                gv = m.geom[kv];
+                const uint2 wd = ((const uint2*)m.geom)[kv];
+                if (kSem) s0 = sp[0];
+                s1 = sp[1];
+                old = __uint_as_float(wd.x);
+                w = (int)(wd.y & 0xffu);
+                r = (int)(wd.y >> 8 & 0xffu);
+                gr = (int)(wd.y >> 16 & 0xffu);
+                b = (int)(wd.y >> 24);
             }
             ++updated;
-            bool new_voxel = gv.weight == 0;
-            if (new_voxel) {
-                gv.sdf = sdf;
-                gv.weight = 1;
-                gv.r = c0;
-                gv.g = c1;
-                gv.b = c2;
+            const bool new_voxel = w == 0;
+            old = new_voxel ? 0.f : old;
+            s0 = new_voxel ? 0u : s0;
+            s1 = new_voxel ? 0u : s1;
+            s2 = new_voxel ? 0u : s2;
+            int count = (int)(s0 & 0xffffu), count2 = (int)(s0 >> 16);
+            int label = (int)(s1 & 0xffu), label2 = (int)(s1 >> 8 & 0xffu);
+            int r2 = (int)(s1 >> 16 & 0xffu), g2 = (int)(s1 >> 24), b2 = (int)(s2 & 0xffu);
+            const float wn = (float)(w + 1);
+            const float yw = __builtin_amdgcn_rcpf(wn);
+            if (label == 0) {
+                r = mean_channel(r, w, c0, yw);
+                gr = mean_channel(gr, w, c1, yw);
+                b = mean_channel(b, w, c2, yw);
             }
-            sicp_voxel_sem sv;
-            const bool semantics = g.num_detection > 0;
-            if (new_voxel) {
-                sv = sicp_voxel_sem{};
-            } else if (m.half) {
-                sv = sh;
-            } else if (semantics) {
-                sv = *sp;
-            } else {
-                sv.label = 0;  // only the label is read below; loaded lazily
-                sv.label = ((const uint8_t*)sp)[4];
-            }
-            if (!new_voxel) {
-                int w = gv.weight;
-                if (sv.label == 0) {
-                    gv.r = u8i(((float)(gv.r * w) + (float)c0) / (float)(w + 1));
-                    gv.g = u8i(((float)(gv.g * w) + (float)c1) / (float)(w + 1));
-                    gv.b = u8i(((float)(gv.b * w) + (float)c2) / (float)(w + 1));
-                }
-                gv.sdf = (gv.sdf * (float)w + sdf) / (float)(w + 1);
-                gv.weight = (uint8_t)min(m.max_weight, w + 1);
-            }
-            if (semantics) {
-                float4 nl = nmap.at(v, u);
-                if (!isnan_(nl.x)) {
-                    const int L = mask.at(v, u);
-                    float val[3];
-                    if (L == 0) {
-                        val[0] = (float)c0;
-                        val[1] = (float)c1;
-                        val[2] = (float)c2;
-                    } else {
-                        val[0] = (float)palette_channel(0, L);
-                        val[1] = (float)palette_channel(1, L);
-                        val[2] = (float)palette_channel(2, L);
-                    }
+            const float num = old * (float)w + sdf;
+            sdf = quotient(num, wn, rcp_step(wn, yw));
+            if (!fits(num)) sdf = num / wn;
+            const int weight = min(m.max_weight, w + 1);
+            // what of the semantic record changed: the labels and the second
+            // colour's r, g beside them; the second colour's b
+            bool labels = new_voxel, blue2 = new_voxel;
+            if (kSem) {
+                bool has_normal = normal;
+                if (!sign) has_normal = !isnan_(nmap.at(v, u).x);
+                const int L = (int)(px.y >> 24);
+                if (has_normal && L == label) {  // the label again, or none again
+                    count = min(m.max_count, count + 1);
                     if (L != 0) {
-                        if (L == sv.label) {
-                            sv.count = (uint16_t)min(m.max_count, (int)sv.count + 1);
-                            gv.r = u8i(val[0]);
-                            gv.g = u8i(val[1]);
-                            gv.b = u8i(val[2]);
-                        } else {
-                            if (L == sv.label2) {
-                                sv.count2 = (uint16_t)min(m.max_count, (int)sv.count2 + 1);
-                                sv.r2 = u8i(val[0]);
-                                sv.g2 = u8i(val[1]);
-                                sv.b2 = u8i(val[2]);
-                            } else if (sv.count2 < 7) {
-                                sv.label2 = (uint8_t)L;
-                                sv.count2 = 1;
-                                sv.r2 = u8i(val[0]);
-                                sv.g2 = u8i(val[1]);
-                                sv.b2 = u8i(val[2]);
-                            }
-                            if (((int)sv.count < (int)sv.count2 && sv.label != 0) ||
-                                ((int)sv.count < (int)sv.count2 * 2 && sv.label == 0)) {
-                                uint8_t tl = sv.label;
-                                sv.label = sv.label2;
-                                sv.label2 = tl;
-                                uint16_t tc = sv.count;
-                                sv.count = sv.count2;
-                                sv.count2 = tc;
-                                uint8_t t0 = gv.r, t1 = gv.g, t2 = gv.b;
-                                gv.r = sv.r2;
-                                gv.g = sv.g2;
-                                gv.b = sv.b2;
-                                sv.r2 = t0;
-                                sv.g2 = t1;
-                                sv.b2 = t2;
-                            }
-                        }
-                    } else {
-                        // w = nl . normalised((pc, 1)) over four components (FuseMap.cu:641)
-                        float n4 = sqrtf(pc.x * pc.x + pc.y * pc.y + pc.z * pc.z + 1.0f * 1.0f);
-                        float q0 = pc.x / n4, q1 = pc.y / n4, q2 = pc.z / n4, q3 = 1.0f / n4;
-                        float wv = nl.x * q0 + nl.y * q1 + nl.z * q2 + nl.w * q3;
-                        if (sv.label != 0) {
-                            if (sv.count < 7) {
-                                sv.label2 = sv.label;
-                                sv.r2 = gv.r;
-                                sv.g2 = gv.g;
-                                sv.b2 = gv.b;
-                                sv.count2 = sv.count;
-                                sv.label = 0;
-                                sv.count = 1;
-                                float aw = wv * 0.2f;
-                                float o0 = (float)gv.r / 255.f, o1 = (float)gv.g / 255.f,
-                                      o2 = (float)gv.b / 255.f;
-                                float r0 = (aw * (val[0] / 255.f) + (1.0f - aw) * o0) * 255.f;
-                                float r1 = (aw * (val[1] / 255.f) + (1.0f - aw) * o1) * 255.f;
-                                float r2 = (aw * (val[2] / 255.f) + (1.0f - aw) * o2) * 255.f;
-                                gv.r = u8i(r0);
-                                gv.g = u8i(r1);
-                                gv.b = u8i(r2);
-                            }
-                        } else {
-                            sv.count = (uint16_t)min(m.max_count, (int)sv.count + 1);
-                        }
+                        r = palette_channel(0, L);
+                        gr = palette_channel(1, L);
+                        b = palette_channel(2, L);
                     }
+                } else if (has_normal && L != 0) {
+                    if (L == label2 || count2 < 7) {
+                        count2 = L == label2 ? min(m.max_count, count2 + 1) : 1;
+                        label2 = L;
+                        r2 = palette_channel(0, L);
+                        g2 = palette_channel(1, L);
+                        b2 = palette_channel(2, L);
+                        labels = blue2 = true;
+                    }
+                    if ((count < count2 && label != 0) || (count < count2 * 2 && label == 0)) {
+                        if (!kHalf && !blue2) b2 = ((const uint8_t*)sp)[8];
+                        int t = label;
+                        label = label2;
+                        label2 = t;
+                        t = count;
+                        count = count2;
+                        count2 = t;
+                        t = r;
+                        r = r2;
+                        r2 = t;
+                        t = gr;
+                        gr = g2;
+                        g2 = t;
+                        t = b;
+                        b = b2;
+                        b2 = t;
+                        labels = blue2 = true;
+                    }
+                } else if (has_normal && count < 7) {
+                    // w = nl . normalised((pc, 1)) over four components (FuseMap.cu:641)
+                    const float4 nl = nmap.at(v, u);
+                    float n4 = sqrtf(pc.x * pc.x + pc.y * pc.y + pc.z * pc.z + 1.0f * 1.0f);
+                    float q0 = pc.x / n4, q1 = pc.y / n4, q2 = pc.z / n4, q3 = 1.0f / n4;
+                    float wv = nl.x * q0 + nl.y * q1 + nl.z * q2 + nl.w * q3;
+                    label2 = label;
+                    r2 = r;
+                    g2 = gr;
+                    b2 = b;
+                    count2 = count;
+                    label = 0;
+                    count = 1;
+                    labels = blue2 = true;
+                    float aw = wv * 0.2f;
+                    float o0 = (float)r / 255.f, o1 = (float)gr / 255.f, o2 = (float)b / 255.f;
+                    r = u8i((aw * ((float)c0 / 255.f) + (1.0f - aw) * o0) * 255.f);
+                    gr = u8i((aw * ((float)c1 / 255.f) + (1.0f - aw) * o1) * 255.f);
+                    b = u8i((aw * ((float)c2 / 255.f) + (1.0f - aw) * o2) * 255.f);
                 }
             }
-            if (m.half) {
+            s0 = (uint32_t)count | (uint32_t)count2 << 16;
+            s1 = (uint32_t)label | (uint32_t)label2 << 8 | (uint32_t)r2 << 16 | (uint32_t)g2 << 24;
+            if (kHalf) {
                 // the sdf rounded to half on the store; the colour in the spare bytes
-                sv.pad[0] = gv.r;
-                sv.pad[1] = gv.g;
-                sv.pad[2] = gv.b;
-                *sp = sv;
-                m.geom_h[kv] = f2h(gv.sdf) | ((uint32_t)gv.weight << 16);
+                sp[0] = s0;
+                sp[1] = s1;
+                sp[2] = (uint32_t)b2 | (uint32_t)r << 8 | (uint32_t)gr << 16 | (uint32_t)b << 24;
+                m.geom_h[kv] = f2h(sdf) | (uint32_t)weight << 16;
             } else {
-                if (semantics || new_voxel) *sp = sv;
-                m.geom[kv] = gv;
+                ((uint2*)m.geom)[kv] =
+                    make_uint2(__float_as_uint(sdf), (uint32_t)weight | (uint32_t)r << 8 |
+                                                         (uint32_t)gr << 16 | (uint32_t)b << 24);
+                if (kSem || new_voxel) sp[0] = s0;
+                if (labels) sp[1] = s1;
+                if (new_voxel)
+                    sp[2] = (uint32_t)b2;
+                else if (blue2)
+                    ((uint8_t*)sp)[8] = (uint8_t)b2;
             }
         }
     }
@@ -863,8 +915,9 @@ int launch_map_reset(MapDev m, MapCounters* ctr, AllocScratch a, hipStream_t s) 
     return SICP_OK;
 }
 
-int launch_allocate(MapDev m, MapCounters* ctr, AllocScratch a, View<float> depth, PoseArg pose,
-                    sicp_intrinsics K, VisFrustum vf, const int* gate, hipStream_t s) {
+int launch_allocate(MapDev m, MapCounters* ctr, AllocScratch a, View<float> depth,
+                    const FuseImages& im, PoseArg pose, sicp_intrinsics K, VisFrustum vf,
+                    const int* gate, hipStream_t s) {
     const int cols = depth.cols, rows = depth.rows;
     if ((uint32_t)(cols * rows) > a.cap_pixels) return invalid("image larger than the map's max_cols x max_rows");
     uint32_t vchunks;
@@ -872,7 +925,7 @@ int launch_allocate(MapDev m, MapCounters* ctr, AllocScratch a, View<float> dept
     if (vchunks > (uint32_t)kScanMaxChunks) return invalid("heap larger than 4M blocks");
     AllocArgs g{(float)(1.0 / (double)K.fx), (float)(1.0 / (double)K.fy), K.cx, K.cy, cols, rows};
     dim3 grid(div_up(cols, 64), div_up(rows, 4));
-    alloc_mark_kernel<<<grid, 256, 0, s>>>(m, ctr, a, depth, pose, g, gate);
+    alloc_mark_kernel<<<grid, 256, 0, s>>>(m, ctr, a, depth, im, pose, g, gate);
     SICP_LAUNCH_CHECK("alloc_mark_kernel");
     // raster chunks of 256 pixels (one per thread) while their sums fit the
     // partial scan, else of 1024
@@ -942,13 +995,13 @@ int launch_visible_compact(MapDev m, MapCounters* ctr, AllocScratch a, sicp_bloc
     return SICP_OK;
 }
 
-int launch_fuse(MapDev m, MapCounters* ctr, const sicp_block* visible, View<float> depth,
-                View<uint8_t> rgb, View<float4> nmap, View<uint8_t> mask, int num_detection,
-                PoseArg pose, sicp_intrinsics K, uint32_t* wave_counts, const int* gate,
-                hipStream_t s) {
-    FuseArgs g{K.fx, K.fy, K.cx, K.cy, depth.cols, depth.rows, num_detection};
-    fuse_kernel<<<kFuseBlocks, 256, 0, s>>>(m, ctr, visible, depth, rgb, nmap, mask, pose, g,
-                                            wave_counts, gate);
+int launch_fuse(MapDev m, MapCounters* ctr, AllocScratch a, const sicp_block* visible, int cols,
+                int rows, const FuseImages& im, PoseArg pose, sicp_intrinsics K,
+                const int* gate, hipStream_t s) {
+    const FuseArgs g{K.fx, K.fy, K.cx, K.cy, cols, rows, 1.0f / m.trunc};
+    auto* k = m.half ? (im.num_detection > 0 ? fuse_kernel<true, true> : fuse_kernel<true, false>)
+                     : (im.num_detection > 0 ? fuse_kernel<false, true> : fuse_kernel<false, false>);
+    k<<<kFuseBlocks, 256, 0, s>>>(m, ctr, visible, a.pixels, im.nmap, pose, g, a.fuse_counts, gate);
     SICP_LAUNCH_CHECK("fuse_kernel");
     return SICP_OK;
 }

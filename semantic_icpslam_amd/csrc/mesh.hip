@@ -15,7 +15,7 @@
 // voxel reading its 8 corners, 24 neighbours and 8 colours itself, and the few
 // voxels on the surface writing up to 15 vertices in turn while the others
 // waited, the passes took 70 and 281 us on 6000 blocks (640x480 / 5 mm); a
-// block's 1331 staged values, and a thread per vertex, take @MESH@.
+// block's 1331 staged values, and a thread per vertex, take 40 and 63.
 #include <cstdio>
 #include <cstring>
 

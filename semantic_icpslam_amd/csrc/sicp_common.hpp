@@ -84,6 +84,23 @@ template <class T> SICP_DEV T early_load(const T* p) {
 SICP_DEV int flag_or_one(const int* flag) { return flag ? early_load(flag) : 1; }
 SICP_DEV bool gate_closed(const int* gate) { return flag_or_one(gate) == 0; }
 
+// --------------------------------------------------------------- division --
+// Correctly rounded quotients from a shared reciprocal (Markstein, "Computation
+// of elementary functions on the IBM RISC System/6000 processor", 1990): with
+// y the correctly rounded 1/b and q = a y, q + y (a - b q) in fused
+// multiply-adds is a/b rounded once. Three instructions a quotient against
+// eleven for the division, whose scaling only numbers near the ends of the
+// exponent range need: quotients outside `fits` take the division.
+// One Newton step from any y0 within an ulp of 1/b gives y for every integer
+// up to 256, two for every mantissa but all ones (every mantissa and y0
+// checked).
+SICP_DEV float rcp_step(float b, float y) { return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y); }
+SICP_DEV float quotient(float a, float b, float y) {
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+SICP_DEV bool fits(float v) { return fabsf(v) >= 0x1p-60f && fabsf(v) <= 0x1p60f; }
+
 // ------------------------------------------------------------------ poses --
 struct PoseF {
     m3 R, Rinv;
@@ -102,11 +119,23 @@ SICP_DEV PoseF to_pose(const sicp_pose_f& p) {
     o.t = v3{p.t[0], p.t[1], p.t[2]};
     return o;
 }
-// One branch on the pointer, each side whole (a select of the two sources
-// becomes a branch and a load per number).
+// Both sources are read through constant-address-space pointers, so the whole
+// pose is a few scalar loads from the chosen one (a select of the numbers
+// becomes a branch and a load for each, a select of plain pointers flat
+// loads). No kernel writes the pose that it is given.
 SICP_DEV PoseF load_pose(const PoseArg& a) {
-    if (a.dev) return to_pose(*a.dev);
-    return to_pose(a.val);
+    typedef const __attribute__((address_space(4))) sicp_pose_f* ConstPose;
+    typedef const __attribute__((address_space(4))) float* ConstFloat;
+    if (!a.dev) return to_pose(a.val);
+    const ConstFloat f = (ConstFloat)(ConstPose)a.dev;
+    sicp_pose_f p;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) p.R[i] = f[i];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) p.Rinv[i] = f[9 + i];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) p.t[i] = f[18 + i];
+    return to_pose(p);
 }
 
 inline PoseArg make_pose_arg(const sicp_pose_f* host, const sicp_pose_f* dev) {

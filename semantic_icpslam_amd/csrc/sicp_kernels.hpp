@@ -263,6 +263,7 @@ struct AllocScratch {
     int32_t* pending_next;     // rank -> next pending rank
     uint8_t* vis_flags;        // per heap slot
     uint32_t* fuse_counts;     // per fusion wavefront: voxels written (kFuseBlocks * 4)
+    uint2* pixels;             // per pixel, what the fusion reads of the frame (pack_pixel)
     uint32_t cap_pixels;
 };
 
@@ -278,18 +279,28 @@ struct VisFrustum {
 // visibility flags of the heap it leaves (CheckBlockVisibility) for the
 // camera `K` and `vf`; launch_visible_compact then completes the
 // visibility pass (the visible list and count).
-int launch_allocate(MapDev m, MapCounters* ctr, AllocScratch a, View<float> depth, PoseArg pose,
-                    sicp_intrinsics K, VisFrustum vf, const int* gate, hipStream_t s);
+// The frame's images that the fusion reads beside the depth: the allocation,
+// which visits every pixel, packs them (AllocScratch::pixels). Normals and
+// labels are read with num_detection > 0 only.
+struct FuseImages {
+    View<uint8_t> rgb;
+    View<float4> nmap;
+    View<uint8_t> mask;
+    int num_detection;
+};
+int launch_allocate(MapDev m, MapCounters* ctr, AllocScratch a, View<float> depth,
+                    const FuseImages& im, PoseArg pose, sicp_intrinsics K, VisFrustum vf,
+                    const int* gate, hipStream_t s);
 int launch_visible_compact(MapDev m, MapCounters* ctr, AllocScratch a, sicp_block* visible,
                            const int* gate, hipStream_t s);
 // A whole visibility pass (flags, then the visible list).
 int launch_visibility(MapDev m, MapCounters* ctr, AllocScratch a, sicp_block* visible,
                       PoseArg pose, sicp_intrinsics K, int cols, int rows, float dmax,
                       float dmin, const int* gate, hipStream_t s);
-int launch_fuse(MapDev m, MapCounters* ctr, const sicp_block* visible, View<float> depth,
-                View<uint8_t> rgb, View<float4> nmap, View<uint8_t> mask, int num_detection,
-                PoseArg pose, sicp_intrinsics K, uint32_t* wave_counts, const int* gate,
-                hipStream_t s);
+// The fusion of the frame that launch_allocate packed before on the stream.
+int launch_fuse(MapDev m, MapCounters* ctr, AllocScratch a, const sicp_block* visible, int cols,
+                int rows, const FuseImages& im, PoseArg pose, sicp_intrinsics K,
+                const int* gate, hipStream_t s);
 // The per-wavefront counts of launch_fuse into the map's counters (always run
 // after it). With `zmin` set, the same launch also clears the zRange images,
 // the rendering-tile count and the raycast queue count (`rq_count`), so the

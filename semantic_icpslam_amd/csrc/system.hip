@@ -500,7 +500,10 @@ static int grab_end(sicp_system* s, const sicp_image& rgb_u8x3, const sicp_image
     // Mapping::FuseColor (Mapping.cc:76-97) -> FuseMapColor (FuseMap.cu:1039-1162)
     ev = stage_begin(s, st);
     // the allocation's last launch also flags the visible blocks
-    if ((rc = launch_allocate(m->dev, m->ctr, m->alloc, f.range.v(), pose, s->K[0],
+    const FuseImages im{view<uint8_t>(rgb_u8x3), f.nmap[0].v(),
+                        labels ? view<uint8_t>(labels_u8) : View<uint8_t>{},
+                        labels ? num_detection : 0};
+    if ((rc = launch_allocate(m->dev, m->ctr, m->alloc, f.range.v(), im, pose, s->K[0],
                               VisFrustum{c, r, m->cfg.depth_max, m->cfg.depth_min}, gate, st)))
         return rc;
     stage_end(s, kStageAlloc, ev, st);
@@ -508,11 +511,8 @@ static int grab_end(sicp_system* s, const sicp_image& rgb_u8x3, const sicp_image
     if ((rc = launch_visible_compact(m->dev, m->ctr, m->alloc, m->visible, gate, st)))
         return rc;
     stage_end(s, kStageVisible, ev, st);
-    View<uint8_t> mask = labels ? view<uint8_t>(labels_u8) : View<uint8_t>{};
     ev = stage_begin(s, st);
-    if ((rc = launch_fuse(m->dev, m->ctr, m->visible, f.range.v(), view<uint8_t>(rgb_u8x3),
-                          f.nmap[0].v(), mask, labels ? num_detection : 0, pose, s->K[0],
-                          m->alloc.fuse_counts, gate, st)))
+    if ((rc = launch_fuse(m->dev, m->ctr, m->alloc, m->visible, c, r, im, pose, s->K[0], gate, st)))
         return rc;
     stage_end(s, kStageFuse, ev, st);
     // The fusion's counts are summed by the render prepass; the zRange images,
