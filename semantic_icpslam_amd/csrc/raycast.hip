@@ -1014,6 +1014,107 @@ SICP_DEV bool coop_normal(const MapDev& m, v3 pt, int k, BlockCache& c, const Po
     return true;
 }
 
+// The march of a ray by its group of lanes, from any state of the loop: on
+// return the state with which the loop ends, or back_face. `k`, `interp` and
+// `steps`: the last sample's voxel index (-1: no block), whether it was an
+// interpolated read, and the sum of the steps taken (the adjoint's).
+struct CoopState {
+    v3 result;
+    float dist_s, sdf, steps;
+    bool back_face, interp;
+    long k;
+    BlockCache cache;
+};
+SICP_DEV void coop_march(const MapDev& m, const Ray& ray, int k, int gbase, CoopState& s) {
+    const v3 dir8 = scale((float)kBlockSide, ray.dir);
+    // After a missing or empty voxel the lanes hold the block-width steps'
+    // samples instead, until one of them is a voxel (which the next turn takes).
+    bool run = false;
+    while (s.dist_s < ray.dist_e) {
+        const v3 d = run ? dir8 : ray.dir;
+        const float step = run ? (float)kBlockSide : 1.0f;
+        v3 P = s.result;
+        float D = s.dist_s;
+#pragma unroll
+        for (int j = 0; j < kRayGroup - 1; ++j)
+            if (j < k) {
+                P = add(P, d);
+                D += step;
+            }
+        const bool inr = D < ray.dist_e;
+        float sv = qnanf();
+        int exists = 0, wok = 0;
+        long idx = -1;
+        if (inr) {
+            bool v;
+            idx = find_voxel_i(m, floor_i(P.x), floor_i(P.y), floor_i(P.z), s.cache, v);
+            if (idx >= 0) {
+                uint32_t wt;
+                vox_load(m, (size_t)idx, sv, wt);
+                exists = 1;
+                wok = wt != 0u;
+            }
+        }
+        float sp = __shfl_up(sv, 1, kRayGroup);
+        if (k == 0) sp = s.sdf;
+        const bool band = wok && sv <= 0.1f && sv >= -0.5f;
+        const bool cross = wok && !band && ((sp < 0.f && sv >= 0.f) || (sp > 0.f && sv <= 0.f));
+        const bool event = run ? !inr || wok : !inr || !wok || band || cross;
+        const uint32_t gm = (uint32_t)(__ballot(event) >> gbase) & ((1u << kRayGroup) - 1u);
+        if (gm == 0u) {  // kRayGroup steps
+            s.result = add(gshfl3(P, kRayGroup - 1), d);
+            s.dist_s = gshfl(D, kRayGroup - 1) + step;
+            s.sdf = gshfl(sv, kRayGroup - 1);
+            s.k = gshfl(idx, kRayGroup - 1);
+            s.steps += step * (float)kRayGroup;
+            s.interp = false;
+            continue;
+        }
+        const int ks = __ffs(gm) - 1;
+        s.result = gshfl3(P, ks);
+        s.dist_s = gshfl(D, ks);
+        s.steps += step * (float)ks;
+        const float prev = gshfl(sp, ks);
+        const long k_prev = gshfl(idx, ks > 0 ? ks - 1 : 0);
+        if (ks > 0) {
+            s.k = k_prev;
+            s.interp = false;
+        }
+        s.sdf = prev;
+        if (!gshfl((int)inr, ks)) break;  // the loop condition fails here
+        if (run) {
+            run = false;
+            continue;
+        }
+        s.k = gshfl(idx, ks);
+        const float sk = gshfl(sv, ks);
+        if (!gshfl(wok, ks)) {  // missing block (NaN) or empty voxel: block-width step
+            s.sdf = gshfl(exists, ks) ? sk : qnanf();
+            s.interp = false;
+            s.result = add(s.result, dir8);
+            s.dist_s += (float)kBlockSide;
+            s.steps += (float)kBlockSide;
+            run = true;
+            continue;
+        }
+        float s1 = sk;
+        s.interp = gshfl((int)band, ks) != 0;
+        if (s.interp) {
+            bool v;
+            s1 = coop_interp(m, s.result, k, s.cache, v);
+        }
+        s.sdf = s1;
+        if (prev < 0.f && s1 >= 0.f) {
+            s.back_face = true;
+            break;
+        }
+        if (prev > 0.f && s1 <= 0.f) break;
+        s.result = add(s.result, ray.dir);
+        s.dist_s += 1.0f;
+        s.steps += 1.0f;
+    }
+}
+
 constexpr int kRayLongThreads = 256;
 __global__ __launch_bounds__(kRayLongThreads) void raycast_long_kernel(
     MapDev m, View<float4> vmap, View<float4> nmap, View<float> zmin, View<float> zmax, PoseArg pa,
@@ -1026,7 +1127,6 @@ __global__ __launch_bounds__(kRayLongThreads) void raycast_long_kernel(
     const RayState st0 = m.rq[i0 < m.rq_cap ? i0 : 0u];
     const int open = early_load(gate);  // gate and nonempty: never null here
     const uint32_t any = early_load(nonempty);
-    const PoseF pose = load_pose(pa);
     if ((open == 0) | (any == 0u)) return;
     const uint32_t n = min(queued, m.rq_cap);
     const int k = threadIdx.x & (kRayGroup - 1);
@@ -1039,87 +1139,23 @@ __global__ __launch_bounds__(kRayLongThreads) void raycast_long_kernel(
         Ray ray;  // the first pass's ray_setup
         ray.dir = v3{st.dx, st.dy, st.dz};
         ray.dist_e = st.dist_e;
-        v3 result{st.rx, st.ry, st.rz};
-        float dist_s = st.dist_s, sdf = st.sdf;
-        bool back_face = false;
-        BlockCache cache{0, 0, 0, -1};
-        while (dist_s < ray.dist_e) {
-            v3 P = result;
-            float D = dist_s;
-#pragma unroll
-            for (int j = 0; j < kRayGroup - 1; ++j)
-                if (j < k) {
-                    P = add(P, scale(1.0f, ray.dir));
-                    D += 1.0f;
-                }
-            const bool inr = D < ray.dist_e;
-            float sv = nan;
-            int exists = 0, wok = 0;
-            if (inr) {
-                bool v;
-                const long idx = find_voxel_i(m, floor_i(P.x), floor_i(P.y), floor_i(P.z), cache, v);
-                if (idx >= 0) {
-                    uint32_t wt;
-                    vox_load(m, (size_t)idx, sv, wt);
-                    exists = 1;
-                    wok = wt != 0u;
-                }
-            }
-            float sp = __shfl_up(sv, 1, kRayGroup);
-            if (k == 0) sp = sdf;
-            const bool band = wok && sv <= 0.1f && sv >= -0.5f;
-            const bool cross = wok && !band && ((sp < 0.f && sv >= 0.f) || (sp > 0.f && sv <= 0.f));
-            const bool event = !inr || !wok || band || cross;
-            const uint32_t gm = (uint32_t)(__ballot(event) >> gbase) & ((1u << kRayGroup) - 1u);
-            if (gm == 0u) {  // kRayGroup one-voxel steps
-                result = add(gshfl3(P, kRayGroup - 1), scale(1.0f, ray.dir));
-                dist_s = gshfl(D, kRayGroup - 1) + 1.0f;
-                sdf = gshfl(sv, kRayGroup - 1);
-                continue;
-            }
-            const int ks = __ffs(gm) - 1;
-            result = gshfl3(P, ks);
-            dist_s = gshfl(D, ks);
-            const float prev = gshfl(sp, ks);
-            if (!gshfl((int)inr, ks)) {  // the loop condition fails here
-                sdf = prev;
-                break;
-            }
-            const float sk = gshfl(sv, ks);
-            if (!gshfl(wok, ks)) {  // missing block (NaN) or empty voxel: block-width step
-                sdf = gshfl(exists, ks) ? sk : nan;
-                result = add(result, scale((float)kBlockSide, ray.dir));
-                dist_s += (float)kBlockSide;
-                continue;
-            }
-            float s1 = sk;
-            if (gshfl((int)band, ks)) {
-                bool v;
-                s1 = coop_interp(m, result, k, cache, v);
-            }
-            if (prev < 0.f && s1 >= 0.f) {
-                back_face = true;
-                break;
-            }
-            if (prev > 0.f && s1 <= 0.f) {
-                sdf = s1;
-                break;
-            }
-            sdf = s1;
-            result = add(result, scale(1.0f, ray.dir));
-            dist_s += 1.0f;
-        }
+        CoopState c{v3{st.rx, st.ry, st.rz}, st.dist_s, st.sdf, 0.f, false, false, -1,
+                    BlockCache{0, 0, 0, -1}};
+        coop_march(m, ray, k, gbase, c);
+        v3 result = c.result;
+        float sdf = c.sdf;
         float4 vout = make_float4(nan, nan, nan, nan);
         float4 nout = vout;
-        if (!back_face && sdf <= 0.0f) {
+        if (!c.back_face && sdf <= 0.0f) {
             float step = sdf * m.step_scale;
             result = add(result, scale(step, ray.dir));
             bool v;
-            sdf = coop_interp(m, result, k, cache, v);
+            sdf = coop_interp(m, result, k, c.cache, v);
             step = sdf * m.step_scale;
             result = add(result, scale(step, ray.dir));
             v3 normal;
-            if (coop_normal(m, result, k, cache, pose, normal)) {
+            const PoseF pose = load_pose(pa);  // here: held through the march it spills
+            if (coop_normal(m, result, k, c.cache, pose, normal)) {
                 v3 r = mv(pose.Rinv, sub(scale(result, m.voxel), pose.t));
                 vout = make_float4(r.x, r.y, r.z, 1.0f);
                 nout = make_float4(normal.x, normal.y, normal.z, 1.0f);
@@ -1148,35 +1184,52 @@ __global__ void ray_queue_reset_kernel(uint32_t* count) { *count = 0u; }
 // T' = T exp(xi), xi = (translation, rotation) in the camera frame:
 // R' = R (I + [w]x), t' = t + R v.
 
-// A trilinear read (readSdfInterped, RenderScene.cu:310-343) with its eight
-// corner voxels, their weights and its gradient in voxel units. The value is
-// formed exactly as the forward read forms it.
+// Eight lanes share a pixel (kRayGroup): they march its ray together, hold a
+// corner each of every trilinear read, and scatter its gradient; the values
+// and derivatives that follow from the corners are formed by every lane alike.
+// One thread per pixel left 160 wavefronts on 1024 SIMDs, each a chain of
+// 32000 instructions and 900 dependent reads: 257 us for 10000 pixels at
+// 1280x720 / 2 mm, 61 now.
+
+// A trilinear read (readSdfInterped, RenderScene.cu:310-343) with this lane's
+// corner voxel and weight and the read's gradient in voxel units. The value
+// is formed exactly as the forward read forms it.
 struct TriRead {
-    long k[8];
-    float w[8];
+    long k;   // -1: missing
+    float w;
     v3 grad;
     float val;
     bool ok;  // every corner exists, the value is not NaN
 };
-SICP_DEV void tri_read(const MapDev& m, v3 p, TriRead& t) {
-    const AxisPair X = axis_pair(p.x), Y = axis_pair(p.y), Z = axis_pair(p.z);
+// The corner's lookup, its bucket's read in flight, then the read's rest.
+struct TriProbe {
+    AxisPair X, Y, Z;
+    Probe p;
+    int local;
+};
+SICP_DEV TriProbe tri_probe(const MapDev& m, v3 q, int k) {
+    TriProbe t{axis_pair(q.x), axis_pair(q.y), axis_pair(q.z), Probe{}, 0};
+    const int vx = (k & 1) ? t.X.v1 : t.X.v0, vy = (k & 2) ? t.Y.v1 : t.Y.v0,
+              vz = (k & 4) ? t.Z.v1 : t.Z.v0;
+    t.p = probe_load(m.table, m.nb, m.nb_mask, vx >> 3, vy >> 3, vz >> 3);
+    t.local = local_of(vx, vy, vz);
+    return t;
+}
+SICP_DEV void tri_corner(const MapDev& m, const TriProbe& t, long& k, float& sd) {
+    const int slot = probe_result(t.p, m.excess);
+    k = slot < 0 ? -1 : (long)slot * kBlockVoxels + t.local;
+    const float v = vox_sdf(m, slot < 0 ? 0 : (size_t)k);
+    sd = slot < 0 ? qnanf() : v;
+}
+SICP_DEV void tri_finish(const TriProbe& q, int k, long kk, float mine, TriRead& t) {
     float sd[8];
-    t.ok = true;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int vx = (i & 1) ? X.v1 : X.v0, vy = (i & 2) ? Y.v1 : Y.v0,
-                  vz = (i & 4) ? Z.v1 : Z.v0;
-        const int slot = map_lookup(m, vx >> 3, vy >> 3, vz >> 3);
-        if (slot < 0) {
-            t.k[i] = -1;
-            sd[i] = qnanf();
-            t.ok = false;
-        } else {
-            t.k[i] = (long)slot * kBlockVoxels + local_of(vx, vy, vz);
-            sd[i] = vox_sdf(m, (size_t)t.k[i]);
-        }
-    }
-    const float fx = X.frac, fy = Y.frac, fz = Z.frac;
+    for (int i = 0; i < 8; ++i) sd[i] = gshfl(mine, i);
+    int missing = kk < 0 ? 1 : 0;
+#pragma unroll
+    for (int o = 1; o < kRayGroup; o <<= 1) missing |= __shfl_xor(missing, o, kRayGroup);
+    t.k = kk;
+    const float fx = q.X.frac, fy = q.Y.frac, fz = q.Z.frac;
     float r0, r1, r2, r3;
     r0 = (1.0f - fx) * sd[0] + fx * sd[1];
     r1 = (1.0f - fx) * sd[2] + fx * sd[3];
@@ -1186,22 +1239,25 @@ SICP_DEV void tri_read(const MapDev& m, v3 p, TriRead& t) {
     r1 = (1.0f - fx) * sd[6] + fx * sd[7];
     r3 = (1.0f - fy) * r0 + fy * r1;
     t.val = (1.0f - fz) * r2 + fz * r3;
-    t.ok = t.ok && !isnan_(t.val);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-        t.w[i] = ((i & 1) ? fx : 1.0f - fx) * ((i & 2) ? fy : 1.0f - fy) * ((i & 4) ? fz : 1.0f - fz);
+    t.ok = missing == 0 && !isnan_(t.val);
+    t.w = ((k & 1) ? fx : 1.0f - fx) * ((k & 2) ? fy : 1.0f - fy) * ((k & 4) ? fz : 1.0f - fz);
     t.grad.x = (1.0f - fz) * ((1.0f - fy) * (sd[1] - sd[0]) + fy * (sd[3] - sd[2])) +
                fz * ((1.0f - fy) * (sd[5] - sd[4]) + fy * (sd[7] - sd[6]));
     t.grad.y = (1.0f - fz) * (a1 - a0) + fz * (r1 - r0);
     t.grad.z = r3 - r2;
 }
+SICP_DEV void tri_read(const MapDev& m, v3 q, int k, TriRead& t) {
+    const TriProbe tp = tri_probe(m, q, k);
+    long kk;
+    float mine;
+    tri_corner(m, tp, kk, mine);
+    tri_finish(tp, k, kk, mine, t);
+}
 
-// dL/d(values) += g * weights.
+// dL/d(values) += g * weights, each lane its corner.
 SICP_DEV void tri_scatter(const TriRead& t, float g, float* grad_sdf) {
     if (!grad_sdf || g == 0.0f) return;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-        if (t.k[i] >= 0 && t.w[i] != 0.0f) atomicAdd(grad_sdf + t.k[i], g * t.w[i]);
+    if (t.k >= 0 && t.w != 0.0f) atomicAdd(grad_sdf + t.k, g * t.w);
 }
 
 struct AdjointArgs {
@@ -1214,76 +1270,60 @@ struct AdjointArgs {
     float* grad_px;        // n x 6 per-pixel pose gradients; may be null
     double* partials;      // 6 x kAdjMaxBlocks
 };
-constexpr int kAdjThreads = 256;
-constexpr int kAdjMaxBlocks = 256;
+constexpr int kAdjThreads = 128;   // 16 pixels: 10000 pixels give each CU two or three
+constexpr int kAdjMaxBlocks = 1024;
 
-// One pixel: false (and no gradient) where the forward pass writes NaN.
+// One pixel, by the lanes k of a group whose first lane is gbase: false (and
+// no gradient) where the forward pass writes NaN. Every lane of the group
+// takes the same branches.
 SICP_DEV bool adjoint_pixel(const MapDev& m, const View<float>& zmin, const View<float>& zmax,
                             const PoseF& pose, const RayArgs& g, int x, int y, v3 gv, v3 gn,
-                            float* grad_sdf, float gxi[6]) {
+                            float* grad_sdf, float gxi[6], int k, int gbase) {
     Ray ray;
     if (!ray_setup(m, zmin, zmax, pose, g, x, y, ray)) return false;
-    // the march of raycast_kernel, uncapped, with its summed step
-    v3 result = ray.start;
-    float dist_s = ray.dist_s, sdf = 1.0f, msum = 0.0f;
-    bool valid_sdf = false, interp0 = false;
-    BlockCache cache{0, 0, 0, -1};
-    long k0 = -1;
-    while (dist_s < ray.dist_e) {
-        const float prev = sdf;
-        const long k = find_voxel_i(m, floor_i(result.x), floor_i(result.y), floor_i(result.z),
-                                    cache, valid_sdf);
-        if (k < 0) {
-            sdf = qnanf();
-        } else {
-            uint32_t wt;
-            vox_load(m, (size_t)k, sdf, wt);
-            if (wt == 0u) valid_sdf = false;
-        }
-        k0 = k;
-        interp0 = false;
-        float step;
-        if (!valid_sdf) {
-            step = (float)kBlockSide;
-        } else {
-            if (sdf <= 0.1f && sdf >= -0.5f) {
-                sdf = read_sdf_interped(m, result, cache, valid_sdf);
-                interp0 = true;
-            }
-            if (prev < 0.f && sdf >= 0.f) return false;  // back face
-            if (prev > 0.f && sdf <= 0.f) break;
-            step = 1.0f;
-        }
-        result = add(result, scale(step, ray.dir));
-        dist_s += step;
-        msum += step;
-    }
+    CoopState c{ray.start, ray.dist_s, 1.0f, 0.0f, false, false, -1, BlockCache{0, 0, 0, -1}};
+    coop_march(m, ray, k, gbase, c);
+    if (c.back_face) return false;
+    const v3 result = c.result;
+    const float sdf = c.sdf, msum = c.steps;
+    const bool interp0 = c.interp;
+    const long k0 = c.k;
     if (!(sdf <= 0.0f)) return false;
     const float ks = m.step_scale;
     const v3 r0 = result;
     TriRead t0;
-    if (interp0) tri_read(m, r0, t0);
+    if (interp0) tri_read(m, r0, k, t0);
     const float s0 = sdf;
     const v3 r1 = add(r0, scale(s0 * ks, ray.dir));
     TriRead t1;
-    tri_read(m, r1, t1);
+    tri_read(m, r1, k, t1);
     const float s1 = t1.val;
     const v3 r2 = add(r1, scale(s1 * ks, ray.dir));
     // readNormal's six reads: pt.a + 1.0f / pt.a + -1.0f on one axis, pt on
-    // the others, in order; the first failing one ends the pixel (the reads
-    // are repeated on the way back rather than kept)
+    // the others; a failing one ends the pixel
     auto normal_point = [&](int a) {
         const float d = (a & 1) ? -1.0f : 1.0f;
         const int ax = a >> 1;
         return v3{ax == 0 ? r2.x + d : r2.x, ax == 1 ? r2.y + d : r2.y, ax == 2 ? r2.z + d : r2.z};
     };
+    // (all six lookups in flight, then all six reads)
+    TriRead tn[6];
+    {
+        TriProbe tp[6];
+        long kk[6];
+        float mine[6];
+#pragma unroll
+        for (int a = 0; a < 6; ++a) tp[a] = tri_probe(m, normal_point(a), k);
+#pragma unroll
+        for (int a = 0; a < 6; ++a) tri_corner(m, tp[a], kk[a], mine[a]);
+#pragma unroll
+        for (int a = 0; a < 6; ++a) tri_finish(tp[a], k, kk[a], mine[a], tn[a]);
+    }
     float sv[6];
-#pragma unroll 1
+#pragma unroll
     for (int a = 0; a < 6; ++a) {
-        TriRead tn;
-        tri_read(m, normal_point(a), tn);
-        sv[a] = tn.val;
-        if (!tn.ok || sv[a] == 1.0f) return false;
+        sv[a] = tn[a].val;
+        if (!tn[a].ok || sv[a] == 1.0f) return false;
     }
     const v3 gvec = mk(sv[0] - sv[1], sv[2] - sv[3], sv[4] - sv[5]);
     const v3 mvec = mv(pose.Rinv, gvec);
@@ -1297,14 +1337,12 @@ SICP_DEV bool adjoint_pixel(const MapDev& m, const View<float>& zmin, const View
     const v3 gm = divs(sub(gn, scale(ndg, nrm)), mlen);
     gw = add(gw, cross(gm, mvec));
     const v3 gg = mv(pose.R, gm);
-#pragma unroll 1
+#pragma unroll
     for (int a = 0; a < 6; ++a) {
         const float ga = (a >> 1) == 0 ? gg.x : ((a >> 1) == 1 ? gg.y : gg.z);
         const float gsa = (a & 1) ? -ga : ga;
-        TriRead tn;
-        tri_read(m, normal_point(a), tn);
-        tri_scatter(tn, gsa, grad_sdf);
-        gr2 = add(gr2, scale(gsa, tn.grad));
+        tri_scatter(tn[a], gsa, grad_sdf);
+        gr2 = add(gr2, scale(gsa, tn[a].grad));
     }
     // vertex: v = R'^T (voxel r2 - t')
     gr2 = add(gr2, scale(m.voxel, mv(pose.R, gv)));
@@ -1323,7 +1361,7 @@ SICP_DEV bool adjoint_pixel(const MapDev& m, const View<float>& zmin, const View
     if (interp0) {
         tri_scatter(t0, gs0, grad_sdf);
         gr0 = add(gr0, scale(gs0, t0.grad));
-    } else if (grad_sdf && k0 >= 0 && gs0 != 0.0f) {
+    } else if (grad_sdf && k == 0 && k0 >= 0 && gs0 != 0.0f) {
         atomicAdd(grad_sdf + k0, gs0);
     }
     // r0 = block_s + M dir
@@ -1350,44 +1388,55 @@ __global__ __launch_bounds__(kAdjThreads) void raycast_adjoint_kernel(MapDev m, 
                                                                       View<float> zmax,
                                                                       PoseArg pa, AdjointArgs a) {
     const PoseF pose = load_pose(pa);
+    constexpr int kGroups = kAdjThreads / kRayGroup;
+    const int k = threadIdx.x & (kRayGroup - 1), gbase = (threadIdx.x & 63) & ~(kRayGroup - 1);
+    const int group = threadIdx.x / kRayGroup;
     double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
+    for (int i = blockIdx.x * kGroups + group; i < a.n; i += gridDim.x * kGroups) {
         const int px = a.pixels[i];
-        if (px < 0 || px >= a.g.cols * a.g.rows) {  // outside the image: no gradient
-            if (a.grad_px)
-                for (int j = 0; j < 6; ++j) a.grad_px[6 * i + j] = 0.f;
-            continue;
-        }
-        const int y = px / a.g.cols, x = px - y * a.g.cols;
-        const v3 gv{a.grad_v[3 * i], a.grad_v[3 * i + 1], a.grad_v[3 * i + 2]};
-        const v3 gn = a.grad_n ? v3{a.grad_n[3 * i], a.grad_n[3 * i + 1], a.grad_n[3 * i + 2]}
-                               : v3{0.f, 0.f, 0.f};
         float gxi[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (!adjoint_pixel(m, zmin, zmax, pose, a.g, x, y, gv, gn, a.grad_sdf, gxi))
-            for (int j = 0; j < 6; ++j) gxi[j] = 0.f;
+        if (px >= 0 && px < a.g.cols * a.g.rows) {  // else outside the image: no gradient
+            const int y = px / a.g.cols, x = px - y * a.g.cols;
+            const v3 gv{a.grad_v[3 * i], a.grad_v[3 * i + 1], a.grad_v[3 * i + 2]};
+            const v3 gn = a.grad_n
+                              ? v3{a.grad_n[3 * i], a.grad_n[3 * i + 1], a.grad_n[3 * i + 2]}
+                              : v3{0.f, 0.f, 0.f};
+            if (!adjoint_pixel(m, zmin, zmax, pose, a.g, x, y, gv, gn, a.grad_sdf, gxi, k, gbase))
+                for (int j = 0; j < 6; ++j) gxi[j] = 0.f;
+        }
 #pragma unroll
         for (int j = 0; j < 6; ++j) acc[j] += (double)gxi[j];
-        if (a.grad_px)
-            for (int j = 0; j < 6; ++j) a.grad_px[6 * i + j] = gxi[j];
-    }
-    // fixed-order workgroup sum: rows through LDS, thread j sums column j
-    __shared__ double tile[kAdjThreads][7];
+        if (a.grad_px && k < 6) {
+            float v = gxi[0];
 #pragma unroll
-    for (int j = 0; j < 6; ++j) tile[threadIdx.x][j] = acc[j];
+            for (int j = 1; j < 6; ++j) v = k == j ? gxi[j] : v;
+            a.grad_px[6 * i + k] = v;
+        }
+    }
+    // fixed-order workgroup sum: one row per group through LDS, thread j sums column j
+    __shared__ double tile[kGroups][7];
+    if (k == 0) {
+#pragma unroll
+        for (int j = 0; j < 6; ++j) tile[group][j] = acc[j];
+    }
     __syncthreads();
     if (threadIdx.x < 6) {
         double s = 0.0;
-        for (int r = 0; r < kAdjThreads; ++r) s += tile[r][threadIdx.x];
+        for (int r = 0; r < kGroups; ++r) s += tile[r][threadIdx.x];
         a.partials[threadIdx.x * kAdjMaxBlocks + blockIdx.x] = s;
     }
 }
 
-__global__ void adjoint_finish_kernel(const double* partials, int nb, double* grad_pose) {
-    if (threadIdx.x < 6) {
-        double s = 0.0;
-        for (int b = 0; b < nb; ++b) s += partials[threadIdx.x * kAdjMaxBlocks + b];
-        grad_pose[threadIdx.x] = s;
-    }
+// The workgroups' partial sums in a fixed order: wavefront j adds column j,
+// lane l rows l, l + 64, ..., then the lanes fold.
+__global__ __launch_bounds__(384) void adjoint_finish_kernel(const double* partials, int nb,
+                                                             double* grad_pose) {
+    const int j = threadIdx.x >> 6, l = threadIdx.x & 63;
+    double s = 0.0;
+    for (int b = l; b < nb; b += 64) s += partials[j * kAdjMaxBlocks + b];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (l == 0) grad_pose[j] = s;
 }
 
 }  // namespace
@@ -1399,11 +1448,11 @@ int launch_raycast_adjoint(MapDev m, View<float> zmin, View<float> zmax, PoseArg
                            double* partials, double* grad_pose, hipStream_t s) {
     AdjointArgs a{RayArgs{invfx, invfy, cx, cy, cols, rows, 0, 0, 0}, pixels, n, grad_v, grad_n,
                   grad_sdf, grad_px, partials};
-    int nb = (int)div_up(n > 0 ? n : 1, kAdjThreads);
+    int nb = (int)div_up(n > 0 ? n : 1, kAdjThreads / kRayGroup);
     if (nb > kAdjMaxBlocks) nb = kAdjMaxBlocks;
     raycast_adjoint_kernel<<<nb, kAdjThreads, 0, s>>>(m, zmin, zmax, pose, a);
     SICP_LAUNCH_CHECK("raycast_adjoint_kernel");
-    adjoint_finish_kernel<<<1, 64, 0, s>>>(partials, nb, grad_pose);
+    adjoint_finish_kernel<<<1, 384, 0, s>>>(partials, nb, grad_pose);
     SICP_LAUNCH_CHECK("adjoint_finish_kernel");
     return SICP_OK;
 }
