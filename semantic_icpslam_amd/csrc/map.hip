@@ -12,9 +12,9 @@
 //   count   per pixel: how many of its flagged steps are their block's first
 //           request;
 //   scan    exclusive scan of those counts -> the rank of every new block;
-//   emit    per pixel: write new blocks at their ranks;
-//   link    per new block: elect the smallest rank of each bucket (atomicMin)
-//           and push the rank onto the bucket's pending list;
+//   emit    per pixel: write new blocks at their ranks, elect the smallest rank
+//           of each bucket (atomicMin) and push the rank onto the bucket's
+//           pending list; other workgroups clear the new blocks' voxels;
 //   insert  per elected bucket: insert its pending blocks in rank order into
 //           the two bucket entries, then the overflow chain (the overflow
 //           entry of a block is the one at its own heap slot, so no counter
@@ -135,6 +135,8 @@ SICP_DEV int req_insert(const AllocScratch& a, uint64_t key) {
     return -1;
 }
 
+constexpr uint32_t kClearBlocks = 512;  // workgroups clearing the new blocks' voxels
+
 struct AllocArgs {
     float invfx, invfy, cx, cy;
     int cols, rows;
@@ -231,7 +233,10 @@ SICP_DEV uint2 chunk_offset(const uint32_t* sums, uint32_t w, uint32_t n);
 // scan that ranks the requests in raster order: the count kernel leaves
 // each chunk's sum in `partials`, and the emit kernel forms every pixel's
 // first rank itself (the sum of the earlier chunks plus the prefix within
-// the chunk) and stores the total — no separate scan launches.
+// the chunk) and stores the total — no separate scan launches. A rank's
+// linking and the clearing of the new blocks need no more than the rank and
+// the total, so they ride in the same launch (as a launch of their own they
+// took 4.7 us a frame, nearly all of it the launch).
 template <int P>
 __global__ __launch_bounds__(256) void alloc_count_kernel(MapDev m, AllocScratch a,
                                                           View<float> depth, PoseArg pa,
@@ -260,6 +265,32 @@ __global__ __launch_bounds__(256) void alloc_count_kernel(MapDev m, AllocScratch
     if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
+// Clears the voxels of the `created` blocks from heap slot `base` on (empty
+// sdf, weight 0, zero semantic record: Voxel::release,
+// Mapping/DeviceMap.h:76-87), as workgroup `wg` of `nwg`.
+SICP_DEV void clear_new_blocks(const MapDev& m, uint32_t created, uint32_t base, uint32_t wg,
+                               uint32_t nwg) {
+    const uint2 g = make_uint2(0x7fffffffu, 0u);
+    const uint3 z = make_uint3(0u, 0u, 0u);
+    for (uint32_t r = wg; r < created; r += nwg) {
+        size_t off = (size_t)(base + r) * kBlockVoxels;
+        for (int v = threadIdx.x; v < kBlockVoxels; v += blockDim.x) {
+            if (m.half)
+                m.geom_h[off + v] = kEmptyHalfVoxel;
+            else
+                ((uint2*)m.geom)[off + v] = g;
+            ((uint3*)m.sem)[off + v] = z;
+        }
+    }
+}
+
+// The blocks this frame creates: the heap's room bounds them; the rest are
+// counted as dropped.
+SICP_DEV uint32_t blocks_created(const MapDev& m, uint32_t total, uint32_t base) {
+    const uint32_t room = base < (uint32_t)m.num_blocks ? (uint32_t)m.num_blocks - base : 0u;
+    return min(total, room);
+}
+
 template <int P>
 __global__ __launch_bounds__(256) void alloc_emit_kernel(MapDev m, MapCounters* ctr,
                                                          AllocScratch a, View<float> depth,
@@ -268,6 +299,14 @@ __global__ __launch_bounds__(256) void alloc_emit_kernel(MapDev m, MapCounters* 
                                                          uint32_t nchunks, const int* gate) {
     if (gate && *gate == 0) {
         if (blockIdx.x == 0 && threadIdx.x == 0) ctr->new_total = 0u;
+        return;
+    }
+    // the first slot of this frame's new blocks (the insertion advances it)
+    const uint32_t heap = ctr->heap_used;
+    if (blockIdx.x >= nchunks) {
+        const uint32_t total = chunk_offset(partials, 0u, nchunks).y;
+        clear_new_blocks(m, blocks_created(m, total, heap), heap, blockIdx.x - nchunks,
+                         gridDim.x - nchunks);
         return;
     }
     const int n = g.cols * g.rows;
@@ -283,7 +322,7 @@ __global__ __launch_bounds__(256) void alloc_emit_kernel(MapDev m, MapCounters* 
         ctr->new_total = off.y;
         // the first slot of this frame's new blocks, kept apart from
         // heap_used, which the insertion advances while others still read it
-        ctr->alloc_base = ctr->heap_used;
+        ctr->alloc_base = heap;
     }
     uint32_t tot;
     uint32_t r = off.x + block_exclusive_scan(s, &tot);
@@ -297,69 +336,21 @@ __global__ __launch_bounds__(256) void alloc_emit_kernel(MapDev m, MapCounters* 
         for_owned_steps(m, a, depth, x, y, i, mask, pose, g, [&](uint64_t key, int slot) {
             a.new_keys[r] = key;
             a.new_req_slot[r] = (uint32_t)slot;
+            const uint32_t hs = heap + r;
+            if (hs < (uint32_t)m.num_blocks) {  // else the heap is exhausted
+                const i3 p = unpack_key(key);
+                const uint32_t b = bucket_of(p.x, p.y, p.z, m);
+                atomicMin(&a.bucket_leader[b], (int)r);
+                a.pending_next[r] = atomicExch(&a.bucket_head[b], (int)r);
+                m.blocks[hs] = sicp_block{p.x, p.y, p.z, (int)hs};
+            }
             ++r;
         });
     }
 }
 
-// Clears the voxels of the blocks this frame creates (empty sdf, weight 0,
-// zero semantic record: Voxel::release, Mapping/DeviceMap.h:76-87), over
-// `nwg` workgroups starting at `wg`.
-SICP_DEV void clear_new_blocks(const MapDev& m, const MapCounters* ctr, uint32_t wg,
-                               uint32_t nwg) {
-    const uint32_t total = ctr->new_total;
-    const uint32_t base = ctr->alloc_base;
-    uint32_t created = 0;
-    if (base < (uint32_t)m.num_blocks) created = min(total, (uint32_t)m.num_blocks - base);
-    const uint2 g = make_uint2(0x7fffffffu, 0u);
-    const uint3 z = make_uint3(0u, 0u, 0u);
-    for (uint32_t r = wg; r < created; r += nwg) {
-        size_t off = (size_t)(base + r) * kBlockVoxels;
-        for (int v = threadIdx.x; v < kBlockVoxels; v += blockDim.x) {
-            if (m.half)
-                m.geom_h[off + v] = kEmptyHalfVoxel;
-            else
-                ((uint2*)m.geom)[off + v] = g;
-            ((uint3*)m.sem)[off + v] = z;
-        }
-    }
-}
-
-// Workgroups below kLinkBlocks link the new requests into their buckets'
-// pending lists and write the block records; the others clear the new
-// blocks' voxels (disjoint memory, so one launch serves both).
-constexpr int kLinkBlocks = 512, kClearBlocks = 1024;
-__global__ __launch_bounds__(256) void alloc_link_kernel(MapDev m, const MapCounters* ctr,
-                                                         AllocScratch a, const int* gate) {
-    if (gate && *gate == 0) return;
-    if (blockIdx.x >= kLinkBlocks) {
-        clear_new_blocks(m, ctr, blockIdx.x - kLinkBlocks, gridDim.x - kLinkBlocks);
-        return;
-    }
-    const uint32_t total = ctr->new_total;
-    const uint32_t base = ctr->alloc_base;
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < total;
-         r += kLinkBlocks * blockDim.x) {
-        uint32_t slot = base + r;
-        if (slot >= (uint32_t)m.num_blocks) continue;  // heap exhausted
-        i3 p = unpack_key(a.new_keys[r]);
-        uint32_t b = bucket_of(p.x, p.y, p.z, m);
-        atomicMin(&a.bucket_leader[b], (int)r);
-        int prev = atomicExch(&a.bucket_head[b], (int)r);
-        a.pending_next[r] = prev;
-        m.blocks[slot] = sicp_block{p.x, p.y, p.z, (int)slot};
-    }
-}
-
 SICP_DEV void store_entry(sicp_hash_entry* e, uint64_t key, int slot, int next) {
     *(uint4*)e = make_uint4((uint32_t)key, (uint32_t)(key >> 32), (uint32_t)slot, (uint32_t)next);
-}
-
-// The blocks this frame creates: the heap's room bounds them; the rest are
-// counted as dropped.
-SICP_DEV uint32_t blocks_created(const MapDev& m, uint32_t total, uint32_t base) {
-    const uint32_t room = base < (uint32_t)m.num_blocks ? (uint32_t)m.num_blocks - base : 0u;
-    return min(total, room);
 }
 
 // The insertion of the frame's new blocks into the table, over the launch's
@@ -940,15 +931,10 @@ int launch_allocate(MapDev m, MapCounters* ctr, AllocScratch a, View<float> dept
         alloc_count_kernel<kScanPerThread><<<nchunks, kScanThreads, 0, s>>>(
             m, a, depth, pose, g, a.scan_partials, gate);
     SICP_LAUNCH_CHECK("alloc_count_kernel");
-    if (one)
-        alloc_emit_kernel<1><<<nchunks, kScanThreads, 0, s>>>(m, ctr, a, depth, pose, g,
-                                                              a.scan_partials, nchunks, gate);
-    else
-        alloc_emit_kernel<kScanPerThread><<<nchunks, kScanThreads, 0, s>>>(
-            m, ctr, a, depth, pose, g, a.scan_partials, nchunks, gate);
+    auto* emit = one ? alloc_emit_kernel<1> : alloc_emit_kernel<kScanPerThread>;
+    emit<<<nchunks + kClearBlocks, kScanThreads, 0, s>>>(m, ctr, a, depth, pose, g,
+                                                         a.scan_partials, nchunks, gate);
     SICP_LAUNCH_CHECK("alloc_emit_kernel");
-    alloc_link_kernel<<<kLinkBlocks + kClearBlocks, 256, 0, s>>>(m, ctr, a, gate);
-    SICP_LAUNCH_CHECK("alloc_link_kernel");
     // the insertion with the visibility flags (chunks as launch_visibility
     // forms them)
     const VisArgs vg{K.fx, K.fy, K.cx, K.cy, vf.cols, vf.rows, vf.dmin, vf.dmax};
