@@ -33,14 +33,28 @@ constexpr int kPixPerThread = 4;
 // Images of at most this many pixels take one pixel per thread instead (four
 // times the workgroups, each lane a quarter of the arithmetic).
 constexpr int kIcpSpreadPixels = 320 * kIcpThreads;
-// Every kernel here runs kIcpThreads threads per workgroup; the constant is
-// used instead of blockDim, whose value the kernel would otherwise load from
+// The kernels here run kIcpThreads threads per workgroup (the tracking loop in
+// the FP64 form kWideThreads); the constant is used instead of blockDim, whose value the kernel would otherwise load from
 // the dispatch packet (a memory round trip before the first address).
 
 struct IcpGeom {
     int cols, rows, n;
     float fx, fy, cx, cy;
+    int chunk;  // kWideThreads launches: pixels of a workgroup (0 elsewhere)
 };
+
+// The tracking loop in the FP64 form runs workgroups of 512 threads, at most
+// one per compute unit, each on consecutive pixels. With 256 threads and four
+// pixels each, 640x480 makes 300 workgroups on 256 compute units: 44 of them
+// run two, and the launch lasts as long as those. Larger workgroups also leave
+// fewer partial rows (256, 150 and 38 against 300, 300 and 75), which 16 lanes
+// a column fetch in one round trip instead of two, before the pixels' loads
+// (wide_rows_load). At 640x480 a level-0 launch spans 9.0 us against 11.6, a
+// level-1 one 7.2 against 8.5, a level-2 one 7.5 to 8.8 against 7.1 to 8.5;
+// the frame takes 410 us against 442.
+// The compensated form keeps the 256-thread layout: its rounding depends on
+// the order of the sums.
+constexpr int kWideThreads = 512, kWideMaxBlocks = 256;
 
 // A workgroup's place among the workgroups that share one image: the launch
 // grid itself, or, in a launch serving several sequences, the sequence's own
@@ -101,6 +115,21 @@ struct FinishBatchArgs {
     FinishSeqArgs seq[kMaxBatch];
 };
 
+// The distance and sine tests without their square roots: the correctly
+// rounded root is monotonic, so each test is one of the squared value against
+// the largest float whose root passes it (sqrtf(s) <= 0.1f, sqrtf(s) < 0.6f,
+// sqrtf(s) < 0.1f).
+constexpr float kDistSq = 0x1.47ae16p-7f, kSineSq = 0x1.70a3d6p-2f, kRgbDistSq = 0x1.47ae12p-7f;
+
+// (float)(1.0 / (double)z). A quotient in 53 bits is not rounded onto a
+// different 24-bit one (53 >= 2 x 24 + 1), so this is 1 / z rounded once; the
+// double division remains for the z that two reciprocal steps do not cover.
+SICP_DEV float inverse(float z) {
+    float y = rcp_step(z, rcp_step(z, __builtin_amdgcn_rcpf(z)));
+    if (!(fits(z) && (__float_as_uint(z) & 0x7fffffu) != 0x7fffffu)) y = (float)(1.0 / (double)z);
+    return y;
+}
+
 // ICPReduce::searchPoint up to the gather (Tracking/Reduction.cu:231-243):
 // current vertex to world, into the last camera, projected with the
 // reference's FP64 promotions (invz = 1.0 / z in double stored to float,
@@ -117,7 +146,7 @@ SICP_DEV IcpProj icp_project(float4 vc4, const PoseF& cur, const PoseF& last, co
     p.vcurr_g = add(mv(cur.R, vcurr_c), cur.t);
     const v3 vcurr_p = mv(last.Rinv, sub(p.vcurr_g, last.t));
     p.vcurr_p = vcurr_p;
-    float invz = (float)(1.0 / (double)vcurr_p.z);
+    const float invz = inverse(vcurr_p.z);
     p.u = (int)((double)(vcurr_p.x * invz * g.fx + g.cx) + 0.5);
     p.v = (int)((double)(vcurr_p.y * invz * g.fy + g.cy) + 0.5);
     p.ok = p.ok && !(p.u < 0 || p.v < 0 || p.u >= g.cols || p.v >= g.rows);
@@ -134,9 +163,10 @@ SICP_DEV bool icp_finish(const IcpProj& p, float4 nc4, float4 vl4, float4 nl4, c
     v3 ncurr_g = mv(cur.R, ncurr_c);
     v3 nlast_c = xyz(nl4);
     v3 nlast_g = mv(last.R, nlast_c);
-    float dist = norm(sub(vlast_g, p.vcurr_g));
-    float sine = norm(cross(ncurr_g, nlast_g));
-    if (!(sine < 0.6f && dist <= 0.1f && !isnan_(ncurr_c.x) && !isnan_(nlast_c.x))) return false;
+    const v3 gap = sub(vlast_g, p.vcurr_g), turn = cross(ncurr_g, nlast_g);
+    if (!(dot(turn, turn) <= kSineSq && dot(gap, gap) <= kDistSq && !isnan_(ncurr_c.x) &&
+          !isnan_(nlast_c.x)))
+        return false;
     v3 nl = mv(last.Rinv, nlast_g);
     v3 vcl = mv(last.Rinv, sub(p.vcurr_g, last.t));
     v3 vll = mv(last.Rinv, sub(vlast_g, last.t));
@@ -170,8 +200,8 @@ SICP_DEV bool rgb_project(v3 p, const IcpGeom& g, int& u, int& v) {
 // {-1, 0} without a correspondence.
 SICP_DEV int2 rgb_record(int key, float4 vc, float4 vl, int li, int u, int v, int cols) {
     const float d0 = vl.x - vc.x, d1 = vl.y - vc.y, d2 = vl.z - vc.z, d3 = vl.w - vc.w;
-    const float dist = sqrtf(d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3);
-    if (isnan_(vl.x) || !(dist < 0.1f) || li == 0) return make_int2(-1, 0);
+    const float dist_sq = d0 * d0 + d1 * d1 + d2 * d2 + d3 * d3;
+    if (isnan_(vl.x) || !(dist_sq <= kRgbDistSq) || li == 0) return make_int2(-1, 0);
     return make_int2(v * cols + u, key - li);
 }
 
@@ -216,17 +246,18 @@ struct IcpBatch {
     int key[kPixPerThread];
 };
 template <bool kRgb, int NP>
-SICP_DEV void icp_load_batch(IcpBatch& bt, int base, int stride, const View<float4>& vcurr,
-                             const View<float4>& ncurr, const RgbPass& rp, const IcpGeom& g) {
+SICP_DEV void icp_load_batch(IcpBatch& bt, int base, int stride, int end,
+                             const View<float4>& vcurr, const View<float4>& ncurr,
+                             const RgbPass& rp, const IcpGeom& g) {
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
         const int i = base + k * stride;
-        const int ii = i < g.n ? i : 0;
+        const int ii = i < end ? i : 0;
         const int y = ii / g.cols, x = ii - y * g.cols;
         bt.vc[k] = vcurr.at(y, x);
         bt.nc[k] = ncurr.at(y, x);
         if (kRgb) bt.key[k] = rp.key.at(y, x);
-        if (i >= g.n) {
+        if (i >= end) {
             bt.vc[k].x = qnanf();
             bt.key[k] = -1;
         }
@@ -235,8 +266,8 @@ SICP_DEV void icp_load_batch(IcpBatch& bt, int base, int stride, const View<floa
 
 // Sum of two u32 values over the workgroup (wrapping, so any order gives the
 // same result, as the reference's int sums). Every thread gets the totals.
-SICP_DEV uint2 block_sum_u32x2(uint32_t a, uint32_t b) {
-    __shared__ uint32_t red[2][kIcpThreads / 64];
+template <int NT> SICP_DEV uint2 block_sum_u32x2(uint32_t a, uint32_t b) {
+    __shared__ uint32_t red[2][NT / 64];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         a += __shfl_xor(a, o, 64);
@@ -249,7 +280,7 @@ SICP_DEV uint2 block_sum_u32x2(uint32_t a, uint32_t b) {
     __syncthreads();
     uint2 r = make_uint2(0u, 0u);
 #pragma unroll
-    for (int w = 0; w < kIcpThreads / 64; ++w) {
+    for (int w = 0; w < NT / 64; ++w) {
         r.x += red[0][w];
         r.y += red[1][w];
     }
@@ -305,25 +336,25 @@ static_assert(sizeof(SumF64) == 8 && sizeof(SumK32) == 8, "one 8-byte partial pe
 // Workgroup reduction of every thread's NS sums into this workgroup's
 // partial row (column-major: partials[j * kIcpMaxBlocks + workgroup]), by
 // transposition through LDS: every thread stores its sums as one row; thread
-// (j, k) then adds rows k, k+8, ... of column j and eight lanes fold with
-// three butterflies. Fixed order; much cheaper than folding 29 doubles
-// across 64 lanes with cross-lane permutes.
-template <int NS, class Acc>
+// (j, k) then adds rows k, k + NT / 32, ... of column j and the column's NT / 32
+// lanes fold with butterflies. Fixed order; much cheaper than folding 29
+// doubles across 64 lanes with cross-lane permutes.
+template <int NT, int NS, class Acc>
 SICP_DEV void block_rows_to_partials(const Acc (&acc)[NS], double* partials, Wg wg) {
-    __shared__ Acc tile[kIcpThreads][NS + 1];
+    constexpr int kLanes = NT / 32;
+    __shared__ Acc tile[NT][NS + 1];
 #pragma unroll
     for (int j = 0; j < NS; ++j) tile[threadIdx.x][j] = acc[j];
     __syncthreads();
     const int t = threadIdx.x;
-    if (t < NS * 8) {
-        const int j = t >> 3, k = t & 7;
+    if (t < NS * kLanes) {
+        const int j = t / kLanes, k = t % kLanes;
         Acc s;
         s.zero();
 #pragma unroll 8
-        for (int r = k; r < kIcpThreads; r += 8) s.merge(tile[r][j]);
-        s.merge(s.shfl_xor(1));
-        s.merge(s.shfl_xor(2));
-        s.merge(s.shfl_xor(4));
+        for (int r = k; r < NT; r += kLanes) s.merge(tile[r][j]);
+#pragma unroll
+        for (int o = 1; o < kLanes; o <<= 1) s.merge(s.shfl_xor(o));
         // column-major: sum j of every workgroup is contiguous
         if (k == 0) reinterpret_cast<Acc*>(partials)[j * kIcpMaxBlocks + wg.id] = s;
     }
@@ -340,29 +371,38 @@ SICP_DEV void add_row(Acc acc[kIcpSums], const float row[7]) {
 }
 
 // Per-thread accumulation + workgroup reduction into this workgroup's
-// partial row. `get_pose(cur, last)` is called by every thread once the first
-// pixels' loads are in flight; it returns false when there is nothing to do.
+// partial row. `get_pose(cur, last, loads)` is called by every thread; it calls
+// `loads`, which issues the first pixels' loads, before it waits for anything
+// of its own, and returns false when there is nothing to do.
 // kRgb: the same pass also runs RGBStep's correspondence test
 // (FindCorresp, Reduction.cu:409-461) on every pixel, writing its record and
 // the workgroup's int count and sum of squared differences.
-template <bool kRgb, class Acc, class PoseFn>
+template <int NT, bool kRgb, class Acc, class PoseFn>
 SICP_DEV void icp_accumulate(const View<float4>& vcurr, const View<float4>& vlast,
                              const View<float4>& ncurr, const View<float4>& nlast,
                              const IcpGeom& g, double* partials, const RgbPass& rp, Wg wg,
                              PoseFn get_pose) {
-    const int stride = wg.n * kIcpThreads;
-    int base = wg.id * kIcpThreads + threadIdx.x;
+    constexpr bool kWide = NT == kWideThreads;
+    const int stride = kWide ? NT : wg.n * NT;
+    const int end = kWide ? min(g.n, (wg.id + 1) * g.chunk) : g.n;
+    int base = wg.id * (kWide ? g.chunk : NT) + threadIdx.x;
     // A launch of one pixel per thread runs a one-slot copy of the pass (a
     // uniform choice), so neither copy carries per-slot branches that would
-    // split the slots' loads and arithmetic into separate blocks.
-    const bool single = stride >= g.n;
+    // split the slots' loads and arithmetic into separate blocks; a wide one of
+    // up to three a three-slot copy.
+    const bool single = kWide ? g.chunk <= NT : stride >= g.n;
+    const bool three = kWide && g.chunk <= 3 * NT;
     IcpBatch bt;
-    if (single)
-        icp_load_batch<kRgb, 1>(bt, base, stride, vcurr, ncurr, rp, g);
-    else
-        icp_load_batch<kRgb, kPixPerThread>(bt, base, stride, vcurr, ncurr, rp, g);
+    auto first_loads = [&] {
+        if (single)
+            icp_load_batch<kRgb, 1>(bt, base, stride, end, vcurr, ncurr, rp, g);
+        else if (three)
+            icp_load_batch<kRgb, 3>(bt, base, stride, end, vcurr, ncurr, rp, g);
+        else
+            icp_load_batch<kRgb, kPixPerThread>(bt, base, stride, end, vcurr, ncurr, rp, g);
+    };
     PoseF cur, last;
-    if (!get_pose(cur, last)) {
+    if (!get_pose(cur, last, first_loads)) {
         phase_mark(4);
         return;
     }
@@ -372,7 +412,7 @@ SICP_DEV void icp_accumulate(const View<float4>& vcurr, const View<float4>& vlas
     uint32_t cnt = 0, sq = 0;
     auto pass = [&](auto slots) {
         constexpr int NP = decltype(slots)::value;
-        while (base < g.n) {
+        while (base < end) {
             float4 vl[NP], nl[NP], rvl[NP];
             IcpProj pr[NP];
             int ru[NP], rv[NP], rli[NP];
@@ -397,7 +437,7 @@ SICP_DEV void icp_accumulate(const View<float4>& vcurr, const View<float4>& vlas
                     add_row(acc, row);
                 if (kRgb) {
                     const int i = base + k * stride;
-                    if (i < g.n) {
+                    if (i < end) {
                         const int2 rc = rok[k] ? rgb_record(bt.key[k], bt.vc[k], rvl[k], rli[k],
                                                             ru[k], rv[k], g.cols)
                                                : make_int2(-1, 0);
@@ -410,22 +450,24 @@ SICP_DEV void icp_accumulate(const View<float4>& vcurr, const View<float4>& vlas
                 }
             }
             base += stride * NP;
-            if (base < g.n) icp_load_batch<kRgb, NP>(bt, base, stride, vcurr, ncurr, rp, g);
+            if (base < end) icp_load_batch<kRgb, NP>(bt, base, stride, end, vcurr, ncurr, rp, g);
         }
     };
     if (single)
         pass(std::integral_constant<int, 1>{});
+    else if (three)
+        pass(std::integral_constant<int, 3>{});
     else
         pass(std::integral_constant<int, kPixPerThread>{});
     phase_mark(4);
     if (kRgb) {
-        const uint2 r = block_sum_u32x2(cnt, sq);
+        const uint2 r = block_sum_u32x2<NT>(cnt, sq);
         if (threadIdx.x == 0) {
             rp.ipart[wg.id] = r.x;
             rp.ipart[kIcpMaxBlocks + wg.id] = r.y;
         }
     }
-    block_rows_to_partials(acc, partials, wg);
+    block_rows_to_partials<NT>(acc, partials, wg);
 }
 
 // RGBStep's row pass over the records of the correspondence pass of
@@ -433,35 +475,40 @@ SICP_DEV void icp_accumulate(const View<float4>& vcurr, const View<float4>& vlas
 // int sums (RGBStep, Reduction.cu:618-620; every workgroup forms the same
 // value), then GetRow of every record into this workgroup's partial row.
 // Workgroup 0 also stores the count, the sum and sigma in `rs.totals`.
-template <class Acc, class PoseFn>
+template <int NT, class Acc, class PoseFn>
 SICP_DEV void rgb_rows(const View<float4>& vlast, const View<int16_t>& dx,
                        const View<int16_t>& dy, const IcpGeom& g, const RgbScratch& rs,
                        int nb_match, PoseFn get_pose) {
     const Wg wg = grid_wg();
-    const int stride = wg.n * kIcpThreads;
-    int base = wg.id * kIcpThreads + threadIdx.x;
-    // One-slot or four-slot copy of the pass, as in icp_accumulate.
-    const bool single = stride >= g.n;
+    constexpr bool kWide = NT == kWideThreads;
+    const int stride = kWide ? NT : wg.n * NT;
+    const int end = kWide ? min(g.n, (wg.id + 1) * g.chunk) : g.n;
+    int base = wg.id * (kWide ? g.chunk : NT) + threadIdx.x;
+    // One-, three- or four-slot copy of the pass, as in icp_accumulate.
+    const bool single = kWide ? g.chunk <= NT : stride >= g.n;
+    const bool three = kWide && g.chunk <= 3 * NT;
     int2 rc[kPixPerThread];
     auto load_records = [&](auto slots) {
 #pragma unroll
         for (int k = 0; k < decltype(slots)::value; ++k) {
             const int i = base + k * stride;
-            rc[k] = i < g.n ? rs.rec[i] : make_int2(-1, 0);
+            rc[k] = i < end ? rs.rec[i] : make_int2(-1, 0);
         }
     };
     if (single)
         load_records(std::integral_constant<int, 1>{});
+    else if (three)
+        load_records(std::integral_constant<int, 3>{});
     else
         load_records(std::integral_constant<int, kPixPerThread>{});
     uint32_t c = 0, q = 0;
-    for (int b = threadIdx.x; b < nb_match; b += kIcpThreads) {
+    for (int b = threadIdx.x; b < nb_match; b += NT) {
         c += rs.ipart[b];
         q += rs.ipart[kIcpMaxBlocks + b];
     }
     PoseF cur, last;
     if (!get_pose(cur, last)) return;
-    const uint2 r = block_sum_u32x2(c, q);
+    const uint2 r = block_sum_u32x2<NT>(c, q);
     const int count = (int)r.x, sum_sq = (int)r.y;
     const float sigma = sqrtf((float)sum_sq / (float)(count == 0 ? 1 : count));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -474,7 +521,7 @@ SICP_DEV void rgb_rows(const View<float4>& vlast, const View<int16_t>& dx,
     for (int j = 0; j < kIcpSums; ++j) acc[j].zero();
     auto pass = [&](auto slots) {
         constexpr int NP = decltype(slots)::value;
-        while (base < g.n) {
+        while (base < end) {
             float4 vl[NP];
             int gx[NP], gy[NP];
 #pragma unroll
@@ -496,48 +543,51 @@ SICP_DEV void rgb_rows(const View<float4>& vlast, const View<int16_t>& dx,
                 }
             }
             base += stride * NP;
-            if (base < g.n) load_records(slots);
+            if (base < end) load_records(slots);
         }
     };
     if (single)
         pass(std::integral_constant<int, 1>{});
+    else if (three)
+        pass(std::integral_constant<int, 3>{});
     else
         pass(std::integral_constant<int, kPixPerThread>{});
-    block_rows_to_partials(acc, rs.partials, wg);
+    block_rows_to_partials<NT>(acc, rs.partials, wg);
 }
 
 // Sum of the partial rows of `nb` workgroups into totals (LDS), in a fixed
-// order: thread (j, k) adds rows k, k+8, ... (below nb) of column j, then
-// eight lanes fold. NS sums per row. Above kFoldPairRows rows the thread
-// adds the row pairs (2p, 2p + 1), p = k, k+8, ... instead, a pair being one
+// order: of the kLanes = NT / 32 lanes of column j, lane k adds rows k,
+// k + kLanes, ... (below nb), then the lanes fold. NS sums per row. Above kFoldPairRows rows the thread
+// adds the row pairs (2p, 2p + 1), p = k, k + kLanes, ... instead, a pair being one
 // 16-byte load (column j starts 16-byte aligned). Measured per launch at
-// 640x480 (launch span, single rows against pairs): 75 rows 6.9-8.0 against
+// 640x480 by eight lanes (launch span, single rows against pairs): 75 rows 6.9-8.0 against
 // 7.6-8.7 us, 300 rows 11.9 against 11.6 us.
 constexpr int kFoldPairRows = 128;
-template <int NS = kIcpSums, class Acc = SumF64>
+template <int NT, int NS = kIcpSums, class Acc = SumF64>
 SICP_DEV void icp_totals_issue(const double* partials, int nb, Acc& s) {
+    constexpr int kLanes = NT / 32;
     const int t = threadIdx.x;
     s.zero();
-    if (t < NS * 8 && nb <= kFoldPairRows) {
-        const int j = t >> 3, k = t & 7;
+    if (t < NS * kLanes && nb <= kFoldPairRows) {
+        const int j = t / kLanes, k = t % kLanes;
         const Acc* col = reinterpret_cast<const Acc*>(partials) + j * kIcpMaxBlocks;
         // Rows below nb only: sixteen loads in flight per step while sixteen
         // complete rows remain, then eight with predicates. A fixed 64-row
         // unroll with predicated loads cost every launch the full sequence
         // of loads and merges (3.2 against 1.5 us at 19 rows).
         int r0 = 0;
-        for (; k + 8 * (r0 + 15) < nb; r0 += 16) {
+        for (; k + kLanes * (r0 + 15) < nb; r0 += 16) {
             Acc v[16];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) v[r] = col[k + 8 * (r0 + r)];
+            for (int r = 0; r < 16; ++r) v[r] = col[k + kLanes * (r0 + r)];
 #pragma unroll
             for (int r = 0; r < 16; ++r) s.merge(v[r]);
         }
-        for (; k + 8 * r0 < nb; r0 += 8) {
+        for (; k + kLanes * r0 < nb; r0 += 8) {
             Acc v[8];
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
-                const int bi = k + 8 * (r0 + r);
+                const int bi = k + kLanes * (r0 + r);
                 if (bi < nb)
                     v[r] = col[bi];
                 else
@@ -546,8 +596,8 @@ SICP_DEV void icp_totals_issue(const double* partials, int nb, Acc& s) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) s.merge(v[r]);
         }
-    } else if (t < NS * 8) {
-        const int j = t >> 3, k = t & 7;
+    } else if (t < NS * kLanes) {
+        const int j = t / kLanes, k = t % kLanes;
         struct alignas(16) Pair {
             Acc a, b;
         };
@@ -555,21 +605,21 @@ SICP_DEV void icp_totals_issue(const double* partials, int nb, Acc& s) {
         const int full = nb >> 1, pairs = (nb + 1) >> 1;
         // As above by pairs; the second row of a last, odd pair counts as zero.
         int r0 = 0;
-        for (; k + 8 * (r0 + 15) < full; r0 += 16) {
+        for (; k + kLanes * (r0 + 15) < full; r0 += 16) {
             Pair v[16];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) v[r] = col[k + 8 * (r0 + r)];
+            for (int r = 0; r < 16; ++r) v[r] = col[k + kLanes * (r0 + r)];
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 s.merge(v[r].a);
                 s.merge(v[r].b);
             }
         }
-        for (; k + 8 * r0 < pairs; r0 += 8) {
+        for (; k + kLanes * r0 < pairs; r0 += 8) {
             Pair v[8];
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
-                const int p = k + 8 * (r0 + r);
+                const int p = k + kLanes * (r0 + r);
                 if (p < pairs) {
                     v[r] = col[p];
                     if (p >= full) v[r].b.zero();
@@ -586,28 +636,80 @@ SICP_DEV void icp_totals_issue(const double* partials, int nb, Acc& s) {
         }
     }
 }
-template <int NS = kIcpSums, class Acc = SumF64>
+template <int NT, int NS = kIcpSums, class Acc = SumF64>
 SICP_DEV void icp_totals_fold(Acc s, double* totals) {
+    constexpr int kLanes = NT / 32;
     const int t = threadIdx.x;
-    s.merge(s.shfl_xor(1));
-    s.merge(s.shfl_xor(2));
-    s.merge(s.shfl_xor(4));
-    if (t < NS * 8 && (t & 7) == 0) totals[t >> 3] = s.value();
+#pragma unroll
+    for (int o = 1; o < kLanes; o <<= 1) s.merge(s.shfl_xor(o));
+    if (t < NS * kLanes && t % kLanes == 0) totals[t / kLanes] = s.value();
 }
-template <int NS = kIcpSums, class Acc = SumF64>
+template <int NT, int NS = kIcpSums, class Acc = SumF64>
 SICP_DEV void icp_totals(const double* partials, int nb, double* totals) {
     Acc s;
-    icp_totals_issue<NS, Acc>(partials, nb, s);
-    icp_totals_fold<NS, Acc>(s, totals);
+    icp_totals_issue<NT, NS, Acc>(partials, nb, s);
+    icp_totals_fold<NT, NS, Acc>(s, totals);
     __syncthreads();
+}
+
+// The fold of the wide launches, whose rows are at most kWideMaxBlocks: every
+// load at once (a lane's eight row pairs, or eight single rows up to
+// kFoldPairRows), and the merging apart, so that the pixels' loads can be
+// issued between the two: the rows come first, and the pixels' data arrives
+// during the fold and the update. Behind the pixels' loads, which fill the
+// same path, the fold of 256 rows took 4.0 us; before them it takes 2.2, and
+// the pixel pass is no longer for it (level 0 of 640x480).
+template <class Acc> struct alignas(16) RowPair {
+    Acc a, b;
+};
+constexpr int kWideRows = 8;
+static_assert(kWideMaxBlocks <= 2 * kWideRows * (kWideThreads / 32) &&
+                  kFoldPairRows <= kWideRows * (kWideThreads / 32),
+              "one step of loads covers every row");
+template <class Acc>
+SICP_DEV void wide_rows_load(const double* partials, int nb, RowPair<Acc> (&v)[kWideRows]) {
+    constexpr int kLanes = kWideThreads / 32;
+    const int j = min((int)threadIdx.x / kLanes, kIcpSums - 1), k = threadIdx.x % kLanes;
+    if (nb > kFoldPairRows) {
+        const RowPair<Acc>* col =
+            reinterpret_cast<const RowPair<Acc>*>(partials + j * kIcpMaxBlocks);
+        const int full = nb >> 1, pairs = (nb + 1) >> 1;
+#pragma unroll
+        for (int r = 0; r < kWideRows; ++r) {
+            const int p = k + kLanes * r;
+            v[r] = col[p < pairs ? p : 0];
+            if (p >= pairs) v[r].a.zero();
+            if (p >= full) v[r].b.zero();
+        }
+    } else {
+        const Acc* col = reinterpret_cast<const Acc*>(partials) + j * kIcpMaxBlocks;
+#pragma unroll
+        for (int r = 0; r < kWideRows; ++r) {
+            const int row = k + kLanes * r;
+            v[r].a = col[row < nb ? row : 0];
+            if (row >= nb) v[r].a.zero();
+            v[r].b.zero();
+        }
+    }
+}
+template <class Acc> SICP_DEV Acc wide_rows_merge(const RowPair<Acc> (&v)[kWideRows]) {
+    Acc s;
+    s.zero();
+#pragma unroll
+    for (int r = 0; r < kWideRows; ++r) {
+        s.merge(v[r].a);
+        s.merge(v[r].b);
+    }
+    return s;
 }
 
 template <class Acc>
 __global__ __launch_bounds__(kIcpThreads) void icp_partials_kernel(
     View<float4> vcurr, View<float4> vlast, View<float4> ncurr, View<float4> nlast, PoseArg pc,
     PoseArg pl, IcpGeom g, double* partials) {
-    icp_accumulate<false, Acc>(vcurr, vlast, ncurr, nlast, g, partials, RgbPass{}, grid_wg(),
-                          [&](PoseF& cur, PoseF& last) {
+    icp_accumulate<kIcpThreads, false, Acc>(vcurr, vlast, ncurr, nlast, g, partials, RgbPass{}, grid_wg(),
+                          [&](PoseF& cur, PoseF& last, auto loads) {
+                              loads();
                               cur = load_pose(pc);
                               last = load_pose(pl);
                               return true;
@@ -619,7 +721,7 @@ __global__ __launch_bounds__(kIcpThreads) void icp_sums_finalize_kernel(const do
                                                                         int nb,
                                                                         float* sums_out) {
     __shared__ double totals[NS];
-    icp_totals<NS, Acc>(partials, nb, totals);
+    icp_totals<kIcpThreads, NS, Acc>(partials, nb, totals);
     if (threadIdx.x < NS) sums_out[threadIdx.x] = (float)totals[threadIdx.x];
 }
 
@@ -661,7 +763,7 @@ __global__ __launch_bounds__(kIcpThreads) void so3_partials_kernel(
             for (int b = a; b < 4; ++b) acc[q++].add(row[a] * row[b]);
         acc[10].add(1.0f);
     }
-    block_rows_to_partials(acc, partials, grid_wg());
+    block_rows_to_partials<kIcpThreads>(acc, partials, grid_wg());
 }
 
 SICP_DEV void copy16(double* d, const double* s) {
@@ -901,26 +1003,39 @@ static_assert(kStateWords <= kIcpThreads, "TrackState copied one word per thread
 // workgroup waits for another; workgroup 0 publishes it to `st_out`.
 // With `rgb_prev` (the previous iteration's photometric partial rows) the
 // update folds those too; `totals` then holds 2 * kIcpSums values.
-template <bool kFirst, class Acc>
+template <int NT, bool kFirst, class Acc, class Loads>
 SICP_DEV void icp_state(TrackState* S, double* totals, const TrackState* st_in,
                         const FrameMeta* last, const TrackParams& tp,
                         const double* partials_prev, const double* rgb_prev, int nb_prev,
-                        int min_count_prev, TrackState* st_out, Wg wg) {
+                        int min_count_prev, TrackState* st_out, Wg wg, Loads loads) {
     if (kFirst) {
+        loads();
         phase_mark(1);
         if (threadIdx.x == 0) track_begin_state(S, last, tp);
         __syncthreads();
         phase_mark(2);
     } else {
         const unsigned long long* src = reinterpret_cast<const unsigned long long*>(st_in);
-        unsigned long long w = threadIdx.x < kStateWords ? src[threadIdx.x] : 0ull;
         Acc s, sr;
         sr.zero();
-        icp_totals_issue<kIcpSums, Acc>(partials_prev, nb_prev, s);
-        if (rgb_prev) icp_totals_issue<kIcpSums, Acc>(rgb_prev, nb_prev, sr);
+        unsigned long long w;
+        if constexpr (NT == kWideThreads) {
+            RowPair<Acc> v[kWideRows], vr[kWideRows];
+            wide_rows_load(partials_prev, nb_prev, v);
+            if (rgb_prev) wide_rows_load(rgb_prev, nb_prev, vr);
+            w = threadIdx.x < kStateWords ? src[threadIdx.x] : 0ull;
+            loads();
+            s = wide_rows_merge(v);
+            if (rgb_prev) sr = wide_rows_merge(vr);
+        } else {
+            loads();
+            w = threadIdx.x < kStateWords ? src[threadIdx.x] : 0ull;
+            icp_totals_issue<NT, kIcpSums, Acc>(partials_prev, nb_prev, s);
+            if (rgb_prev) icp_totals_issue<NT, kIcpSums, Acc>(rgb_prev, nb_prev, sr);
+        }
         if (threadIdx.x < kStateWords) reinterpret_cast<unsigned long long*>(S)[threadIdx.x] = w;
-        icp_totals_fold<kIcpSums, Acc>(s, totals);
-        if (rgb_prev) icp_totals_fold<kIcpSums, Acc>(sr, totals + kIcpSums);
+        icp_totals_fold<NT, kIcpSums, Acc>(s, totals);
+        if (rgb_prev) icp_totals_fold<NT, kIcpSums, Acc>(sr, totals + kIcpSums);
         __syncthreads();
         phase_mark(1);
         __shared__ double gn_tmp[32];
@@ -940,7 +1055,7 @@ SICP_DEV void icp_state(TrackState* S, double* totals, const TrackState* st_in,
 // kRgb: the photometric term is on; its correspondence pass runs here and
 // the previous iteration's photometric rows (`rgb_prev`) join the update.
 // Acc: the arithmetic of the sums (SumF64, or SumK32 in the precision form).
-template <bool kFirst, bool kRgb, class Acc>
+template <int NT, bool kFirst, bool kRgb, class Acc>
 SICP_DEV void icp_iteration_body(const View<float4>& vcurr, const View<float4>& vlast,
                                  const View<float4>& ncurr, const View<float4>& nlast,
                                  const IcpGeom& g, const TrackState* st_in, const FrameMeta* last,
@@ -950,11 +1065,12 @@ SICP_DEV void icp_iteration_body(const View<float4>& vcurr, const View<float4>& 
     __shared__ TrackState S;
     __shared__ double totals[2 * kIcpSums];
     phase_mark(0);
-    icp_accumulate<kRgb, Acc>(vcurr, vlast, ncurr, nlast, g, partials, rp, wg,
-                              [&](PoseF& cur, PoseF& lst) {
-                                  icp_state<kFirst, Acc>(&S, totals, st_in, last, tp,
-                                                         partials_prev, kRgb ? rgb_prev : nullptr,
-                                                         nb_prev, min_count_prev, st_out, wg);
+    icp_accumulate<NT, kRgb, Acc>(vcurr, vlast, ncurr, nlast, g, partials, rp, wg,
+                              [&](PoseF& cur, PoseF& lst, auto loads) {
+                                  icp_state<NT, kFirst, Acc>(
+                                      &S, totals, st_in, last, tp, partials_prev,
+                                      kRgb ? rgb_prev : nullptr, nb_prev, min_count_prev, st_out,
+                                      wg, loads);
                                   phase_mark(3);
                                   if (S.done) return false;
                                   cur = to_pose(S.curr_f);
@@ -969,13 +1085,13 @@ SICP_DEV void icp_iteration_body(const View<float4>& vcurr, const View<float4>& 
 #endif
 }
 
-template <bool kFirst, bool kRgb, class Acc>
-__global__ __launch_bounds__(kIcpThreads) void icp_iteration_kernel(
+template <int NT, bool kFirst, bool kRgb, class Acc>
+__global__ __launch_bounds__(NT) void icp_iteration_kernel(
     View<float4> vcurr, View<float4> vlast, View<float4> ncurr, View<float4> nlast, IcpGeom g,
     const TrackState* st_in, const FrameMeta* last, TrackParams tp, const double* partials_prev,
     const double* rgb_prev, int nb_prev, int min_count_prev, TrackState* st_out,
     double* partials, RgbPass rp) {
-    icp_iteration_body<kFirst, kRgb, Acc>(vcurr, vlast, ncurr, nlast, g, st_in, last, tp,
+    icp_iteration_body<NT, kFirst, kRgb, Acc>(vcurr, vlast, ncurr, nlast, g, st_in, last, tp,
                                           partials_prev, rgb_prev, nb_prev, min_count_prev,
                                           st_out, partials, rp, grid_wg());
 }
@@ -983,24 +1099,24 @@ __global__ __launch_bounds__(kIcpThreads) void icp_iteration_kernel(
 // One Gauss-Newton iteration of several sequences in one launch: sequence q
 // owns workgroups wg0[q] .. wg0[q + 1] - 1 and runs exactly the arithmetic of
 // its own icp_iteration_kernel launch on them (the point-to-plane term).
-template <bool kFirst, class Acc>
-__global__ __launch_bounds__(kIcpThreads) void icp_iteration_batch_kernel(IcpBatchArgs a) {
+template <int NT, bool kFirst, class Acc>
+__global__ __launch_bounds__(NT) void icp_iteration_batch_kernel(IcpBatchArgs a) {
     int q = 0;
     while (q + 1 < a.n && (int)blockIdx.x >= a.wg0[q + 1]) ++q;
     const IcpSeqArgs& e = a.seq[q];
     const Wg wg{(int)blockIdx.x - a.wg0[q], a.wg0[q + 1] - a.wg0[q]};
-    icp_iteration_body<kFirst, false, Acc>(e.vcurr, e.vlast, e.ncurr, e.nlast, e.g, e.st_in,
+    icp_iteration_body<NT, kFirst, false, Acc>(e.vcurr, e.vlast, e.ncurr, e.nlast, e.g, e.st_in,
                                            e.last, e.tp, e.partials_prev, nullptr, e.nb_prev,
                                            e.min_count_prev, e.st_out, e.partials, RgbPass{}, wg);
 }
 
 // RGBStep's row pass. The pose is the iteration state's (`st`, published by
 // the iteration's pixel pass) or, without a state, `pc` / `pl`.
-template <class Acc>
-__global__ __launch_bounds__(kIcpThreads) void rgb_rows_kernel(
+template <int NT, class Acc>
+__global__ __launch_bounds__(NT) void rgb_rows_kernel(
     View<float4> vlast, View<int16_t> dx, View<int16_t> dy, IcpGeom g, RgbScratch rs,
     int nb_match, const TrackState* st, PoseArg pc, PoseArg pl) {
-    rgb_rows<Acc>(vlast, dx, dy, g, rs, nb_match, [&](PoseF& cur, PoseF& lst) {
+    rgb_rows<NT, Acc>(vlast, dx, dy, g, rs, nb_match, [&](PoseF& cur, PoseF& lst) {
         if (st) {
             if (st->done) return false;
             cur = to_pose(st->curr_f);
@@ -1036,7 +1152,7 @@ __global__ __launch_bounds__(kIcpThreads) void rgb_match_kernel(View<float4> vcu
             sq += (uint32_t)(rc.y * rc.y);
         }
     }
-    const uint2 r = block_sum_u32x2(cnt, sq);
+    const uint2 r = block_sum_u32x2<kIcpThreads>(cnt, sq);
     if (threadIdx.x == 0) {
         rp.ipart[blockIdx.x] = r.x;
         rp.ipart[kIcpMaxBlocks + blockIdx.x] = r.y;
@@ -1054,8 +1170,8 @@ SICP_DEV void track_finish_body(const TrackState* st_in, const FrameMeta* last,
                                 const View<float4>& nnext, const FrameImages& images, Wg wg) {
     __shared__ TrackState S;
     __shared__ double totals[2 * kIcpSums];
-    icp_state<kFirst, Acc>(&S, totals, st_in, last, tp, partials_prev, rgb_prev, nb_prev,
-                           min_count_prev, nullptr, wg);
+    icp_state<kIcpThreads, kFirst, Acc>(&S, totals, st_in, last, tp, partials_prev, rgb_prev, nb_prev,
+                           min_count_prev, nullptr, wg, [] {});
     if (threadIdx.x == 0) track_end_state(&S);
     __syncthreads();
     if (wg.id == 0) {
@@ -1148,12 +1264,20 @@ inline int icp_blocks(int n, bool spread) {
     return b < 1 ? 1 : (b > kIcpMaxBlocks ? kIcpMaxBlocks : b);
 }
 
+// The tracking loop's workgroups: wide ones in FP64, one pixel per thread as
+// far as they go (four without `spread`).
+inline int icp_iteration_blocks(int n, bool k32, bool spread) {
+    if (k32) return icp_blocks(n, spread);
+    const int b = (int)div_up(n, spread ? kWideThreads : kWideThreads * kPixPerThread);
+    return b < kWideMaxBlocks ? b : kWideMaxBlocks;
+}
+
 }  // namespace
 
 int launch_icp_sums(View<float4> vcurr, View<float4> vlast, View<float4> ncurr,
                     View<float4> nlast, PoseArg curr, PoseArg last, sicp_intrinsics K,
                     IcpScratch scratch, float* sums_out, bool k32, hipStream_t s) {
-    IcpGeom g{vcurr.cols, vcurr.rows, vcurr.cols * vcurr.rows, K.fx, K.fy, K.cx, K.cy};
+    IcpGeom g{vcurr.cols, vcurr.rows, vcurr.cols * vcurr.rows, K.fx, K.fy, K.cx, K.cy, 0};
     const int nb = icp_blocks(g.n, true);
     if (k32) {
         icp_partials_kernel<SumK32><<<nb, kIcpThreads, 0, s>>>(vcurr, vlast, ncurr, nlast, curr,
@@ -1175,18 +1299,21 @@ namespace {
 IcpGeom geom_of(const IcpLevel& l) {
     return IcpGeom{l.vcurr.cols, l.vcurr.rows, l.vcurr.cols * l.vcurr.rows,
                    l.K.fx,       l.K.fy,       l.K.cx,
-                   l.K.cy};
+                   l.K.cy,       0};
 }
 }  // namespace
 
-template <class Acc>
+template <int NT, class Acc>
 static void icp_iteration_launch(const IcpLevel& cur, const IcpLevel* prev,
                                  const FrameMeta* last, TrackParams tp, const TrackState* st_in,
                                  TrackState* st_out, const double* partials_prev,
                                  double* partials, const RgbScratch* rgb, hipStream_t s) {
-    const IcpGeom g = geom_of(cur);
-    const int nb = icp_blocks(g.n, tp.spread);
-    const int nb_prev = prev ? icp_blocks(prev->vcurr.cols * prev->vcurr.rows, tp.spread) : 0;
+    IcpGeom g = geom_of(cur);
+    const int nb = icp_iteration_blocks(g.n, tp.sums_k32, tp.spread);
+    if (NT == kWideThreads) g.chunk = (int)div_up(g.n, nb);
+    const int nb_prev = prev ? icp_iteration_blocks(prev->vcurr.cols * prev->vcurr.rows,
+                                                    tp.sums_k32, tp.spread)
+                             : 0;
     const int min_prev = prev ? prev->min_count : 0;
     RgbPass rp{};
     const double* rgb_prev = nullptr;
@@ -1195,19 +1322,19 @@ static void icp_iteration_launch(const IcpLevel& cur, const IcpLevel* prev,
         rgb_prev = rgb->partials;
     }
     if (prev && rgb)
-        icp_iteration_kernel<false, true, Acc><<<nb, kIcpThreads, 0, s>>>(
+        icp_iteration_kernel<NT, false, true, Acc><<<nb, NT, 0, s>>>(
             cur.vcurr, cur.vlast, cur.ncurr, cur.nlast, g, st_in, last, tp, partials_prev,
             rgb_prev, nb_prev, min_prev, st_out, partials, rp);
     else if (prev)
-        icp_iteration_kernel<false, false, Acc><<<nb, kIcpThreads, 0, s>>>(
+        icp_iteration_kernel<NT, false, false, Acc><<<nb, NT, 0, s>>>(
             cur.vcurr, cur.vlast, cur.ncurr, cur.nlast, g, st_in, last, tp, partials_prev,
             nullptr, nb_prev, min_prev, st_out, partials, rp);
     else if (rgb)
-        icp_iteration_kernel<true, true, Acc><<<nb, kIcpThreads, 0, s>>>(
+        icp_iteration_kernel<NT, true, true, Acc><<<nb, NT, 0, s>>>(
             cur.vcurr, cur.vlast, cur.ncurr, cur.nlast, g, nullptr, last, tp, nullptr, nullptr,
             0, 0, st_out, partials, rp);
     else
-        icp_iteration_kernel<true, false, Acc><<<nb, kIcpThreads, 0, s>>>(
+        icp_iteration_kernel<NT, true, false, Acc><<<nb, NT, 0, s>>>(
             cur.vcurr, cur.vlast, cur.ncurr, cur.nlast, g, nullptr, last, tp, nullptr, nullptr,
             0, 0, st_out, partials, rp);
 }
@@ -1216,12 +1343,9 @@ int launch_icp_iteration(const IcpLevel& cur, const IcpLevel* prev, const FrameM
                          TrackParams tp, const TrackState* st_in, TrackState* st_out,
                          const double* partials_prev, double* partials, const RgbScratch* rgb,
                          hipStream_t s) {
-    if (tp.sums_k32)
-        icp_iteration_launch<SumK32>(cur, prev, last, tp, st_in, st_out, partials_prev, partials,
-                                     rgb, s);
-    else
-        icp_iteration_launch<SumF64>(cur, prev, last, tp, st_in, st_out, partials_prev, partials,
-                                     rgb, s);
+    auto* launch = tp.sums_k32 ? icp_iteration_launch<kIcpThreads, SumK32>
+                               : icp_iteration_launch<kWideThreads, SumF64>;
+    launch(cur, prev, last, tp, st_in, st_out, partials_prev, partials, rgb, s);
     SICP_LAUNCH_CHECK("icp_iteration_kernel");
     return SICP_OK;
 }
@@ -1236,9 +1360,11 @@ int launch_icp_iteration_batch(const IcpBatchEntry* e, int n, hipStream_t s) {
     for (int q = 0; q < n; ++q) {
         if ((e[q].prev == nullptr) != first || e[q].tp.sums_k32 != k32 || e[q].tp.rgb)
             return invalid("icp batch: sequences at different iterations or forms");
-        const IcpGeom g = geom_of(e[q].cur);
+        IcpGeom g = geom_of(e[q].cur);
+        const int nb = icp_iteration_blocks(g.n, k32 != 0, e[q].tp.spread);
+        if (!k32) g.chunk = (int)div_up(g.n, nb);
         a.wg0[q] = wg;
-        wg += icp_blocks(g.n, e[q].tp.spread);
+        wg += nb;
         const IcpLevel* p = e[q].prev;
         a.seq[q] = IcpSeqArgs{e[q].cur.vcurr,
                               e[q].cur.vlast,
@@ -1251,18 +1377,20 @@ int launch_icp_iteration_batch(const IcpBatchEntry* e, int n, hipStream_t s) {
                               e[q].st_out,
                               e[q].partials_prev,
                               e[q].partials,
-                              p ? icp_blocks(p->vcurr.cols * p->vcurr.rows, e[q].tp.spread) : 0,
+                              p ? icp_iteration_blocks(p->vcurr.cols * p->vcurr.rows, k32 != 0,
+                                                       e[q].tp.spread)
+                                : 0,
                               p ? p->min_count : 0};
     }
     a.wg0[n] = wg;
     if (first && k32)
-        icp_iteration_batch_kernel<true, SumK32><<<wg, kIcpThreads, 0, s>>>(a);
+        icp_iteration_batch_kernel<kIcpThreads, true, SumK32><<<wg, kIcpThreads, 0, s>>>(a);
     else if (first)
-        icp_iteration_batch_kernel<true, SumF64><<<wg, kIcpThreads, 0, s>>>(a);
+        icp_iteration_batch_kernel<kWideThreads, true, SumF64><<<wg, kWideThreads, 0, s>>>(a);
     else if (k32)
-        icp_iteration_batch_kernel<false, SumK32><<<wg, kIcpThreads, 0, s>>>(a);
+        icp_iteration_batch_kernel<kIcpThreads, false, SumK32><<<wg, kIcpThreads, 0, s>>>(a);
     else
-        icp_iteration_batch_kernel<false, SumF64><<<wg, kIcpThreads, 0, s>>>(a);
+        icp_iteration_batch_kernel<kWideThreads, false, SumF64><<<wg, kWideThreads, 0, s>>>(a);
     SICP_LAUNCH_CHECK("icp_iteration_batch_kernel");
     return SICP_OK;
 }
@@ -1283,7 +1411,8 @@ int launch_track_finish_batch(const FinishBatchEntry* e, int n, hipStream_t s) {
         a.seq[q] = FinishSeqArgs{e[q].tp,       e[q].st_in,  e[q].last,  e[q].partials_prev,
                                  e[q].st_final, e[q].next,   e[q].vlast, e[q].nlast,
                                  e[q].vnext,    e[q].nnext,
-                                 icp_blocks(p->vcurr.cols * p->vcurr.rows, e[q].tp.spread),
+                                 icp_iteration_blocks(p->vcurr.cols * p->vcurr.rows, k32 != 0,
+                                                      e[q].tp.spread),
                                  p->min_count};
     }
     a.wg0[n] = wg;
@@ -1297,14 +1426,16 @@ int launch_track_finish_batch(const FinishBatchEntry* e, int n, hipStream_t s) {
 
 int launch_rgb_rows(const IcpLevel& cur, const TrackState* st, RgbScratch rgb, bool k32,
                     bool spread, hipStream_t s) {
-    const IcpGeom g = geom_of(cur);
-    const int nb = icp_blocks(g.n, spread);
-    if (k32)
-        rgb_rows_kernel<SumK32><<<nb, kIcpThreads, 0, s>>>(cur.vlast, cur.rgb.dx, cur.rgb.dy, g,
-                                                           rgb, nb, st, PoseArg{}, PoseArg{});
-    else
-        rgb_rows_kernel<SumF64><<<nb, kIcpThreads, 0, s>>>(cur.vlast, cur.rgb.dx, cur.rgb.dy, g,
-                                                           rgb, nb, st, PoseArg{}, PoseArg{});
+    IcpGeom g = geom_of(cur);
+    const int nb = icp_iteration_blocks(g.n, k32, spread);
+    if (k32) {
+        rgb_rows_kernel<kIcpThreads, SumK32><<<nb, kIcpThreads, 0, s>>>(
+            cur.vlast, cur.rgb.dx, cur.rgb.dy, g, rgb, nb, st, PoseArg{}, PoseArg{});
+    } else {
+        g.chunk = (int)div_up(g.n, nb);
+        rgb_rows_kernel<kWideThreads, SumF64><<<nb, kWideThreads, 0, s>>>(
+            cur.vlast, cur.rgb.dx, cur.rgb.dy, g, rgb, nb, st, PoseArg{}, PoseArg{});
+    }
     SICP_LAUNCH_CHECK("rgb_rows_kernel");
     return SICP_OK;
 }
@@ -1321,7 +1452,8 @@ int launch_track_finish(const IcpLevel* prev, const FrameMeta* last, TrackParams
     FrameImages im{};
     if (images) im = *images;
     if (prev) {
-        const int nb_prev = icp_blocks(prev->vcurr.cols * prev->vcurr.rows, tp.spread);
+        const int nb_prev = icp_iteration_blocks(prev->vcurr.cols * prev->vcurr.rows,
+                                                 tp.sums_k32, tp.spread);
         if (tp.sums_k32)
             track_finish_kernel<false, SumK32><<<blocks, kIcpThreads, 0, s>>>(
                 st_in, last, tp, partials_prev, rgb ? rgb->partials : nullptr, nb_prev,
@@ -1357,8 +1489,8 @@ int launch_rgb_sums(View<uint8_t> inext, View<uint8_t> ilast, View<float4> vnext
     rgb_match_kernel<<<nb, kIcpThreads, 0, s>>>(vnext, vlast, g, curr, last,
                                                  RgbPass{kv, ilast, rgb.rec, rgb.ipart});
     SICP_LAUNCH_CHECK("rgb_match_kernel");
-    rgb_rows_kernel<SumF64><<<nb, kIcpThreads, 0, s>>>(vlast, dx, dy, g, rgb, nb, nullptr, curr,
-                                                       last);
+    rgb_rows_kernel<kIcpThreads, SumF64><<<nb, kIcpThreads, 0, s>>>(vlast, dx, dy, g, rgb, nb,
+                                                                    nullptr, curr, last);
     SICP_LAUNCH_CHECK("rgb_rows_kernel");
     icp_sums_finalize_kernel<><<<1, kIcpThreads, 0, s>>>(rgb.partials, nb, sums_out);
     SICP_LAUNCH_CHECK("icp_sums_finalize_kernel");
@@ -1368,7 +1500,7 @@ int launch_rgb_sums(View<uint8_t> inext, View<uint8_t> ilast, View<float4> vnext
 int launch_so3_sums(View<uint8_t> inext, View<uint8_t> ilast, View<int16_t> dx,
                     View<int16_t> dy, PoseArg curr, PoseArg last, sicp_intrinsics K,
                     IcpScratch scratch, float* sums_out, hipStream_t s) {
-    const IcpGeom g{inext.cols, inext.rows, inext.cols * inext.rows, K.fx, K.fy, K.cx, K.cy};
+    const IcpGeom g{inext.cols, inext.rows, inext.cols * inext.rows, K.fx, K.fy, K.cx, K.cy, 0};
     const int nb = icp_blocks(g.n, true);
     so3_partials_kernel<<<nb, kIcpThreads, 0, s>>>(inext, ilast, dx, dy, curr, last, g,
                                                      scratch.partials);

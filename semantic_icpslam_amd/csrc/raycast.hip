@@ -1122,7 +1122,7 @@ __global__ __launch_bounds__(kRayLongThreads) void raycast_long_kernel(
     constexpr uint32_t kGroupsPerWg = kRayLongThreads / kRayGroup;
     const uint32_t i0 = blockIdx.x * kGroupsPerWg + (threadIdx.x / kRayGroup);
     // the queue's count, this group's first entry (at a clamped index, used
-    // only below the count), the pose and the gates, loaded together
+    // only below the count) and the gates, loaded together
     const uint32_t queued = early_load(m.rq_count);
     const RayState st0 = m.rq[i0 < m.rq_cap ? i0 : 0u];
     const int open = early_load(gate);  // gate and nonempty: never null here
