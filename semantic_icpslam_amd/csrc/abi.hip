@@ -3,6 +3,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -30,6 +31,62 @@ bool image_ok(const sicp_image& im, size_t elem, int cols, int rows) {
     if (!im.ptr || im.cols != cols || im.rows != rows || cols <= 0 || rows <= 0) return false;
     if (im.pitch < (size_t)cols * elem) return false;
     return true;
+}
+
+namespace {
+std::mutex g_loans_mu;
+void* g_loans[kHostLoansKept];
+int g_loans_free = 0;
+}  // namespace
+
+void HostLoan::take() {
+    {
+        std::lock_guard<std::mutex> lock(g_loans_mu);
+        if (g_loans_free > 0) ptr = g_loans[--g_loans_free];
+    }
+    if (ptr) return;
+    // Another thread may be capturing a graph in the mode that forbids
+    // allocations elsewhere; this one concerns no stream.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (hipHostMalloc(&ptr, kHostLoanBytes, hipHostMallocPortable) != hipSuccess) {
+        ptr = nullptr;
+        (void)hipGetLastError();
+    }
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
+int HostLoan::wait(void* dst, size_t bytes, hipStream_t s) {
+    hipError_t e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+        ptr = nullptr;  // a kernel may still write it: given up, not lent again
+        return hip_fail(e, "hipStreamSynchronize(host results)");
+    }
+    std::memcpy(dst, ptr, bytes);
+    return SICP_OK;
+}
+
+HostLoan::~HostLoan() {
+    if (!ptr) return;
+    {
+        std::lock_guard<std::mutex> lock(g_loans_mu);
+        if (g_loans_free < kHostLoansKept) {
+            g_loans[g_loans_free++] = ptr;
+            return;
+        }
+    }
+    (void)hipHostFree(ptr);
+}
+
+void host_loans_release() {
+    void* idle[kHostLoansKept];
+    int n = 0;
+    {
+        std::lock_guard<std::mutex> lock(g_loans_mu);
+        std::swap(n, g_loans_free);
+        std::memcpy(idle, g_loans, sizeof(idle));
+    }
+    for (int i = 0; i < n; ++i) (void)hipHostFree(idle[i]);
 }
 
 static bool pow2(uint32_t v) { return v && !(v & (v - 1)); }
@@ -168,6 +225,7 @@ void map_free(sicp_map* m) {
     for (void* p : m->owned) (void)hipFree(p);
     if (m->mesh_counts) (void)hipFree(m->mesh_counts);
     if (m->mesh_total) (void)hipHostFree(m->mesh_total);
+    host_loans_release();
     delete m;
 }
 
@@ -293,10 +351,21 @@ size_t sicp_icp_partials_size(void) { return sizeof(double) * kIcpMaxBlocks * kI
 }  // extern "C"
 
 namespace sicp {
+// A step's host results: what its last kernel wrote to the loan, or a copy of
+// the device's sums where there is none.
+static int step_results(HostLoan& loan, float* h, size_t bytes, const float* sums_dev,
+                        hipStream_t s) {
+    if (loan.ptr) return loan.wait(h, bytes, s);
+    SICP_HIP(hipMemcpyAsync(h, sums_dev, bytes, hipMemcpyDeviceToHost, s));
+    SICP_HIP(hipStreamSynchronize(s));
+    return SICP_OK;
+}
+
 int icp_step(sicp_image vcurr, sicp_image vlast, sicp_image ncurr, sicp_image nlast,
                     const sicp_pose_f* curr, const sicp_pose_f* last, sicp_intrinsics K,
                     void* partials_dev, float* sums_dev, float* host_sums, double* A_host,
-                    double* b_host, float* residual_host, bool k32, void* stream) {
+                    double* b_host, float* residual_host, bool k32, void* stream,
+                    bool allocates) {
     const int c = vcurr.cols, r = vcurr.rows;
     if (!image_ok(vcurr, 16, c, r) || !image_ok(vlast, 16, c, r) || !image_ok(ncurr, 16, c, r) ||
         !image_ok(nlast, 16, c, r))
@@ -306,14 +375,20 @@ int icp_step(sicp_image vcurr, sicp_image vlast, sicp_image ncurr, sicp_image nl
         return invalid("icp_step: partials not 16-byte aligned");
     IcpScratch sc{(double*)partials_dev};
     hipStream_t s = (hipStream_t)stream;
+    const bool host = host_sums || A_host || b_host || residual_host;
+    HostLoan loan;
+    if (host && allocates) loan.take();
     int rc = launch_icp_sums(view<float4>(vcurr), view<float4>(vlast), view<float4>(ncurr),
                              view<float4>(nlast), make_pose_arg(curr, nullptr),
-                             make_pose_arg(last, nullptr), K, sc, sums_dev, k32, s);
-    if (rc) return rc;
-    if (host_sums || A_host || b_host || residual_host) {
+                             make_pose_arg(last, nullptr), K, sc, sums_dev, (float*)loan.ptr, k32,
+                             s);
+    if (rc) {
+        loan.ptr = nullptr;  // as in wait()
+        return rc;
+    }
+    if (host) {
         float h[kIcpSums];
-        SICP_HIP(hipMemcpyAsync(h, sums_dev, sizeof(h), hipMemcpyDeviceToHost, s));
-        SICP_HIP(hipStreamSynchronize(s));
+        if ((rc = step_results(loan, h, sizeof(h), sums_dev, s))) return rc;
         if (host_sums) std::memcpy(host_sums, h, sizeof(h));
         double A[36], b[6];
         create_matrix(h, A, b);
@@ -359,14 +434,19 @@ int sicp_so3_step(sicp_image next_image, sicp_image last_image, sicp_image didx,
         return invalid("so3_step: partials not 16-byte aligned");
     IcpScratch sc{(double*)partials_dev};
     hipStream_t s = (hipStream_t)stream;
+    const bool host = host_sums || A_host || b_host || residual_host;
+    HostLoan loan;
+    if (host) loan.take();
     int rc = launch_so3_sums(view<uint8_t>(next_image), view<uint8_t>(last_image),
                              view<int16_t>(didx), view<int16_t>(didy), make_pose_arg(curr, nullptr),
-                             make_pose_arg(last, nullptr), K, sc, sums_dev, s);
-    if (rc) return rc;
-    if (host_sums || A_host || b_host || residual_host) {
+                             make_pose_arg(last, nullptr), K, sc, sums_dev, (float*)loan.ptr, s);
+    if (rc) {
+        loan.ptr = nullptr;  // as in wait()
+        return rc;
+    }
+    if (host) {
         float h[11];
-        SICP_HIP(hipMemcpyAsync(h, sums_dev, sizeof(h), hipMemcpyDeviceToHost, s));
-        SICP_HIP(hipStreamSynchronize(s));
+        if ((rc = step_results(loan, h, sizeof(h), sums_dev, s))) return rc;
         if (host_sums) std::memcpy(host_sums, h, sizeof(h));
         // CreateMatrix<3,4> (Reduction.cu:6-16)
         double A[9], b[3];
@@ -427,19 +507,29 @@ int sicp_rgb_step(sicp_image next_image, sicp_image last_image, sicp_image next_
     rs.totals = (int32_t*)(b + pr + n * sizeof(int2) + ip);
     int16_t* key = (int16_t*)(b + pr + n * sizeof(int2) + ip + 16);
     hipStream_t s = (hipStream_t)stream;
+    const bool host =
+        host_sums || corresp_host || sigma_host || A_host || b_host || residual_host;
+    HostLoan loan;
+    if (host) loan.take();
     int rc = launch_rgb_sums(view<uint8_t>(next_image), view<uint8_t>(last_image),
                              view<float4>(next_vmap), view<float4>(last_vmap),
                              view<int16_t>(didx), view<int16_t>(didy),
                              make_pose_arg(curr, nullptr), make_pose_arg(last, nullptr), K, key,
-                             rs, sums_dev, s);
-    if (rc) return rc;
-    if (host_sums || corresp_host || sigma_host || A_host || b_host || residual_host) {
-        float h[kIcpSums];
+                             rs, sums_dev, (float*)loan.ptr, s);
+    if (rc) {
+        loan.ptr = nullptr;  // as in wait()
+        return rc;
+    }
+    if (host) {
+        float h[kIcpSums + 3];
         int32_t t[3];
-        SICP_HIP(hipMemcpyAsync(h, sums_dev, sizeof(h), hipMemcpyDeviceToHost, s));
-        SICP_HIP(hipMemcpyAsync(t, rs.totals, sizeof(t), hipMemcpyDeviceToHost, s));
-        SICP_HIP(hipStreamSynchronize(s));
-        if (host_sums) std::memcpy(host_sums, h, sizeof(h));
+        if (!loan.ptr)
+            SICP_HIP(hipMemcpyAsync(t, rs.totals, sizeof(t), hipMemcpyDeviceToHost, s));
+        if ((rc = step_results(loan, h, (loan.ptr ? kIcpSums + 3 : kIcpSums) * sizeof(float),
+                               sums_dev, s)))
+            return rc;
+        if (loan.ptr) std::memcpy(t, h + kIcpSums, sizeof(t));
+        if (host_sums) std::memcpy(host_sums, h, kIcpSums * sizeof(float));
         if (corresp_host) {
             corresp_host[0] = t[0];
             corresp_host[1] = t[1];

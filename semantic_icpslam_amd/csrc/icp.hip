@@ -719,10 +719,18 @@ __global__ __launch_bounds__(kIcpThreads) void icp_partials_kernel(
 template <int NS = kIcpSums, class Acc = SumF64>
 __global__ __launch_bounds__(kIcpThreads) void icp_sums_finalize_kernel(const double* partials,
                                                                         int nb,
-                                                                        float* sums_out) {
+                                                                        float* sums_out,
+                                                                        float* sums_host,
+                                                                        const int32_t* extra) {
     __shared__ double totals[NS];
     icp_totals<kIcpThreads, NS, Acc>(partials, nb, totals);
-    if (threadIdx.x < NS) sums_out[threadIdx.x] = (float)totals[threadIdx.x];
+    if (threadIdx.x < NS) {
+        const float v = (float)totals[threadIdx.x];
+        sums_out[threadIdx.x] = v;
+        if (sums_host) sums_host[threadIdx.x] = v;
+    }
+    if (sums_host && extra && threadIdx.x < 3)
+        ((int32_t*)sums_host)[NS + threadIdx.x] = extra[threadIdx.x];
 }
 
 // SO3Reduce::GetRow (Tracking/Reduction.cu:96-131): the last frame's pixel
@@ -1276,20 +1284,22 @@ inline int icp_iteration_blocks(int n, bool k32, bool spread) {
 
 int launch_icp_sums(View<float4> vcurr, View<float4> vlast, View<float4> ncurr,
                     View<float4> nlast, PoseArg curr, PoseArg last, sicp_intrinsics K,
-                    IcpScratch scratch, float* sums_out, bool k32, hipStream_t s) {
+                    IcpScratch scratch, float* sums_out, float* sums_host, bool k32,
+                    hipStream_t s) {
     IcpGeom g{vcurr.cols, vcurr.rows, vcurr.cols * vcurr.rows, K.fx, K.fy, K.cx, K.cy, 0};
     const int nb = icp_blocks(g.n, true);
     if (k32) {
         icp_partials_kernel<SumK32><<<nb, kIcpThreads, 0, s>>>(vcurr, vlast, ncurr, nlast, curr,
                                                                last, g, scratch.partials);
         SICP_LAUNCH_CHECK("icp_partials_kernel");
-        icp_sums_finalize_kernel<kIcpSums, SumK32><<<1, kIcpThreads, 0, s>>>(scratch.partials,
-                                                                              nb, sums_out);
+        icp_sums_finalize_kernel<kIcpSums, SumK32><<<1, kIcpThreads, 0, s>>>(
+            scratch.partials, nb, sums_out, sums_host, nullptr);
     } else {
         icp_partials_kernel<SumF64><<<nb, kIcpThreads, 0, s>>>(vcurr, vlast, ncurr, nlast, curr,
                                                                last, g, scratch.partials);
         SICP_LAUNCH_CHECK("icp_partials_kernel");
-        icp_sums_finalize_kernel<><<<1, kIcpThreads, 0, s>>>(scratch.partials, nb, sums_out);
+        icp_sums_finalize_kernel<><<<1, kIcpThreads, 0, s>>>(scratch.partials, nb, sums_out,
+                                                             sums_host, nullptr);
     }
     SICP_LAUNCH_CHECK("icp_sums_finalize_kernel");
     return SICP_OK;
@@ -1474,7 +1484,7 @@ int launch_track_finish(const IcpLevel* prev, const FrameMeta* last, TrackParams
 int launch_rgb_sums(View<uint8_t> inext, View<uint8_t> ilast, View<float4> vnext,
                     View<float4> vlast, View<int16_t> dx, View<int16_t> dy, PoseArg curr,
                     PoseArg last, sicp_intrinsics K, int16_t* key, RgbScratch rgb,
-                    float* sums_out, hipStream_t s) {
+                    float* sums_out, float* sums_host, hipStream_t s) {
     const int cols = inext.cols, rows = inext.rows;
     View<int16_t> kv{(char*)key, (size_t)cols * sizeof(int16_t), cols, rows};
     int rc = launch_rgb_keys(inext, dx, dy, vnext, kv, s);
@@ -1492,20 +1502,22 @@ int launch_rgb_sums(View<uint8_t> inext, View<uint8_t> ilast, View<float4> vnext
     rgb_rows_kernel<kIcpThreads, SumF64><<<nb, kIcpThreads, 0, s>>>(vlast, dx, dy, g, rgb, nb,
                                                                     nullptr, curr, last);
     SICP_LAUNCH_CHECK("rgb_rows_kernel");
-    icp_sums_finalize_kernel<><<<1, kIcpThreads, 0, s>>>(rgb.partials, nb, sums_out);
+    icp_sums_finalize_kernel<><<<1, kIcpThreads, 0, s>>>(rgb.partials, nb, sums_out, sums_host,
+                                                         rgb.totals);
     SICP_LAUNCH_CHECK("icp_sums_finalize_kernel");
     return SICP_OK;
 }
 
 int launch_so3_sums(View<uint8_t> inext, View<uint8_t> ilast, View<int16_t> dx,
                     View<int16_t> dy, PoseArg curr, PoseArg last, sicp_intrinsics K,
-                    IcpScratch scratch, float* sums_out, hipStream_t s) {
+                    IcpScratch scratch, float* sums_out, float* sums_host, hipStream_t s) {
     const IcpGeom g{inext.cols, inext.rows, inext.cols * inext.rows, K.fx, K.fy, K.cx, K.cy, 0};
     const int nb = icp_blocks(g.n, true);
     so3_partials_kernel<<<nb, kIcpThreads, 0, s>>>(inext, ilast, dx, dy, curr, last, g,
                                                      scratch.partials);
     SICP_LAUNCH_CHECK("so3_partials_kernel");
-    icp_sums_finalize_kernel<kSo3Sums><<<1, kIcpThreads, 0, s>>>(scratch.partials, nb, sums_out);
+    icp_sums_finalize_kernel<kSo3Sums><<<1, kIcpThreads, 0, s>>>(scratch.partials, nb, sums_out,
+                                                                 sums_host, nullptr);
     SICP_LAUNCH_CHECK("icp_sums_finalize_kernel");
     return SICP_OK;
 }

@@ -57,7 +57,7 @@ int sicp_icp_step_static(sicp_image vcurr, sicp_image vlast, sicp_image ncurr, s
     const int rc = scratch_address(&partials);
     if (rc) return rc;
     return sicp::icp_step(vcurr, vlast, ncurr, nlast, curr, last, K, partials, sums_dev,
-                          host_sums, A_host, b_host, residual_host, false, stream);
+                          host_sums, A_host, b_host, residual_host, false, stream, false);
 }
 
 }  // extern "C"

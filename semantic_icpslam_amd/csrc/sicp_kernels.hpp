@@ -91,10 +91,13 @@ struct IcpScratch {
 };
 
 // ICPStep: the 29 sums of one level into `sums_out` (device); `k32`: the
-// precision form's FP32 compensated sums instead of FP64 accumulation.
+// precision form's FP32 compensated sums instead of FP64 accumulation. The
+// steps' `sums_host` (may be null) is pinned host memory that gets the sums
+// too (RGBStep: then the match count, sum and sigma).
 int launch_icp_sums(View<float4> vcurr, View<float4> vlast, View<float4> ncurr,
                     View<float4> nlast, PoseArg curr, PoseArg last, sicp_intrinsics K,
-                    IcpScratch scratch, float* sums_out, bool k32, hipStream_t s);
+                    IcpScratch scratch, float* sums_out, float* sums_host, bool k32,
+                    hipStream_t s);
 
 // The photometric inputs of one level (RGBStep, Reduction.h:81-90): the
 // current frame's candidate key (its intensity where the pose-independent
@@ -184,7 +187,7 @@ int launch_track_finish_batch(const FinishBatchEntry* e, int n, hipStream_t s);
 int launch_rgb_sums(View<uint8_t> inext, View<uint8_t> ilast, View<float4> vnext,
                     View<float4> vlast, View<int16_t> dx, View<int16_t> dy, PoseArg curr,
                     PoseArg last, sicp_intrinsics K, int16_t* key, RgbScratch rgb,
-                    float* sums_out, hipStream_t s);
+                    float* sums_out, float* sums_host, hipStream_t s);
 int launch_track_init(FrameMeta* next, FrameMeta* last, TrackState* st, hipStream_t s);
 
 // SO3Step: the 11 sums of the rotation-only photometric alignment (the 6
@@ -192,7 +195,7 @@ int launch_track_init(FrameMeta* next, FrameMeta* last, TrackState* st, hipStrea
 // `sums_out`.
 int launch_so3_sums(View<uint8_t> inext, View<uint8_t> ilast, View<int16_t> dx,
                     View<int16_t> dy, PoseArg curr, PoseArg last, sicp_intrinsics K,
-                    IcpScratch scratch, float* sums_out, hipStream_t s);
+                    IcpScratch scratch, float* sums_out, float* sums_host, hipStream_t s);
 
 // Host FP64 solve + SE(3) update (same code path as the device).
 void se3_update_host(const double* A, const double* b, double* delta, const double* last_pose,

@@ -72,6 +72,7 @@ struct FrameBuf {
 struct sicp_system {
     sicp_system_config cfg;
     sicp_map* map = nullptr;
+    int device = -1;  // the one that was current at its creation
     sicp::FrameBuf fa, fb;
     sicp::FrameBuf* next = &fa;
     sicp::FrameBuf* last = &fb;
@@ -232,6 +233,28 @@ __global__ __launch_bounds__(kStageThreads) void stage_copy_kernel(StageArgs a) 
     }
 }
 
+// What sicp_system_last_result reads, gathered into pinned host memory by one
+// launch (three copies to pageable memory took 30 us of host time a frame).
+struct ResultWords {
+    TrackState track;
+    MapCounters counters;
+    FrameMeta meta;
+};
+static_assert(sizeof(ResultWords) <= kHostLoanBytes, "a host loan holds the result");
+static_assert(sizeof(TrackState) % 4 == 0 && sizeof(MapCounters) % 4 == 0 &&
+                  sizeof(FrameMeta) % 4 == 0,
+              "copied by words");
+template <class T> __device__ __forceinline__ void copy_words(T* d, const T* s) {
+    for (unsigned i = threadIdx.x; i < sizeof(T) / 4; i += 64)
+        reinterpret_cast<uint32_t*>(d)[i] = reinterpret_cast<const uint32_t*>(s)[i];
+}
+__global__ __launch_bounds__(64) void result_kernel(const TrackState* t, const MapCounters* c,
+                                                    const FrameMeta* m, ResultWords* out) {
+    copy_words(&out->track, t);
+    copy_words(&out->counters, c);
+    copy_words(&out->meta, m);
+}
+
 // Adds the copy of `src` into `dst` (same shape, `elem` bytes per element).
 static void stage_add(StageArgs& a, uint32_t& wgs, const sicp_image& src, const sicp_image& dst,
                       size_t elem) {
@@ -327,6 +350,7 @@ int sicp_system_create(const sicp_system_config* cfg, sicp_system** out) {
     const bool rgb = !cfg->icp_only;
     sicp_system* s = new sicp_system();
     s->cfg = *cfg;
+    (void)hipGetDevice(&s->device);
     int rc = map_alloc(cfg->map, &s->map);
     if (rc) {
         delete s;
@@ -734,13 +758,28 @@ int sicp_system_read_timing_detail(sicp_system* s, int stage, double* ms_out, in
 int sicp_system_last_result(sicp_system* s, sicp_frame_result* out, void* stream) {
     if (!s || !out) return invalid("system_last_result: null argument");
     hipStream_t st = (hipStream_t)stream;
-    TrackState t;
-    MapCounters c;
-    FrameMeta fm;
-    SICP_HIP(hipMemcpyAsync(&t, s->st, sizeof(t), hipMemcpyDeviceToHost, st));
-    SICP_HIP(hipMemcpyAsync(&c, s->map->ctr, sizeof(c), hipMemcpyDeviceToHost, st));
-    SICP_HIP(hipMemcpyAsync(&fm, s->last->meta, sizeof(fm), hipMemcpyDeviceToHost, st));
-    SICP_HIP(hipStreamSynchronize(st));
+    ResultWords r;
+    HostLoan loan;
+    int device = -1;
+    // a copy is also right from another device's stream, a kernel is not
+    if (hipGetDevice(&device) == hipSuccess && device == s->device) loan.take();
+    if (loan.ptr) {
+        result_kernel<<<1, 64, 0, st>>>(s->st, s->map->ctr, s->last->meta,
+                                        (ResultWords*)loan.ptr);
+        SICP_LAUNCH_CHECK("result_kernel");
+        const int rc = loan.wait(&r, sizeof(r), st);
+        if (rc) return rc;
+    } else {
+        SICP_HIP(hipMemcpyAsync(&r.track, s->st, sizeof(r.track), hipMemcpyDeviceToHost, st));
+        SICP_HIP(hipMemcpyAsync(&r.counters, s->map->ctr, sizeof(r.counters),
+                                hipMemcpyDeviceToHost, st));
+        SICP_HIP(hipMemcpyAsync(&r.meta, s->last->meta, sizeof(r.meta), hipMemcpyDeviceToHost,
+                                st));
+        SICP_HIP(hipStreamSynchronize(st));
+    }
+    const TrackState& t = r.track;
+    const MapCounters& c = r.counters;
+    const FrameMeta& fm = r.meta;
     std::memset(out, 0, sizeof(*out));
     out->frame_index = s->frame_index - 1;
     out->tracked = t.tracked;
