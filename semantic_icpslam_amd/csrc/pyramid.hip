@@ -1,8 +1,9 @@
 // pyramid.hip — depth / intensity pyramid kernels for gfx950.
 //
 // One thread per output pixel; 64x4 workgroups so each wavefront covers 64
-// consecutive pixels of a row (coalesced row loads and stores). Every kernel
-// is a bandwidth-bound stencil; the 5x5 windows are served from L1/L2.
+// consecutive pixels of a row (coalesced row loads and stores). The stencils'
+// windows are served from L1/L2; the 5x5 ones are bound by their arithmetic,
+// the others by bandwidth.
 #include "sicp_kernels.hpp"
 
 namespace sicp {
@@ -22,9 +23,68 @@ inline dim3 grid2d(int cols, int rows) { return dim3(div_up(cols, kTX), div_up(r
 // The 5x5 window is unrolled: every tap's load is issued at a clamped
 // address first, then the taps inside the clipped window are summed in the
 // reference's row-major order.
+//
+// Bound by its 25 exponentials per pixel. expf_cw's cases (NaN, overflow,
+// underflow, a denormal result) are a branch or two per tap and keep the taps
+// apart, so a wavefront whose depths are within kNearTaps of each other uses
+// the one case that is left, in straight code, and one away from the image's
+// edges also drops the window's selects. 640x480: 13.4 us with every case,
+// 9.3 us so.
+
+// 2 x 6.5^2 + 8 / 32 = 84.75: exp of no less than -84.75, a normal float.
+constexpr float kNearTaps = 6.5f;
+
+// expf_cw for x in [-84.75, 0]: the same operations (x <= 0 makes the rounding
+// offset -0.5; at 0 both give k = 0), with the factor 2^k, k >= -123, added to
+// the exponent of p in [0.7, 1.42], which is the same normal product.
+SICP_DEV float exp_near(float x) {
+    const float kf = x * 1.44269504088896341f;
+    const int k = (int)(kf - 0.5f);
+    const float fk = (float)k;
+    const float r = (x - fk * 0.693359375f) - fk * -2.12194440e-4f;
+    float p = 1.0f / 5040.0f;
+    p = p * r + 1.0f / 720.0f;
+    p = p * r + 1.0f / 120.0f;
+    p = p * r + 1.0f / 24.0f;
+    p = p * r + 1.0f / 6.0f;
+    p = p * r + 0.5f;
+    p = p * r + 1.0f;
+    p = p * r + 1.0f;
+    return __uint_as_float(__float_as_uint(p) + ((unsigned)k << 23));
+}
+
+// The window's two sums. kNear: every depth is within kNearTaps of the
+// centre's; kInner: the whole window is inside the clipped one.
+template <bool kNear, bool kInner>
+SICP_DEV void filter_sums(const uint16_t (&tap)[25], float scale_inv, int x, int y, int tx, int ty,
+                          float& sum1, float& sum2) {
+    const float sig_space = 0.03125f, sig_range = 2.0f;
+    const float center = (float)tap[12] * scale_inv;
+#pragma unroll
+    for (int dy = 0; dy < 5; ++dy) {
+        const int cy = y - 2 + dy;
+#pragma unroll
+        for (int dx = 0; dx < 5; ++dx) {
+            const int cx = x - 2 + dx;
+            // Every tap is computed; one outside the clipped window adds +0
+            // through a select (the sums are never -0, so their bits do not
+            // change). One straight block lets the compiler interleave the
+            // 25 taps' exponentials; a branch per tap kept them apart.
+            const bool in = kInner || (cy >= 0 && cy < ty && cx >= 0 && cx < tx);
+            const float val = (float)tap[dy * 5 + dx] * scale_inv;
+            const float space2 = (float)((2 - dx) * (2 - dx) + (2 - dy) * (2 - dy));
+            const float color2 = (center - val) * (center - val);
+            const float arg = -(space2 * sig_space + color2 * sig_range);
+            // exp(-0) is 1
+            const float weight = !kNear ? expf_cw(arg) : dy == 2 && dx == 2 ? 1.f : exp_near(arg);
+            sum1 += in ? val * weight : 0.f;
+            sum2 += in ? weight : 0.f;
+        }
+    }
+}
+
 SICP_DEV void filter_px(const View<uint16_t>& depth, const View<float>& raw,
                         const View<float>& filtered, float scale_inv, float cutoff, int x, int y) {
-    const float sig_space = 0.03125f, sig_range = 2.0f;
     const int tx = min(x + 3, depth.cols - 1);
     const int ty = min(y + 3, depth.rows - 1);
     uint16_t tap[25];
@@ -36,26 +96,17 @@ SICP_DEV void filter_px(const View<uint16_t>& depth, const View<float>& raw,
     }
     float center = (float)tap[12] * scale_inv;
     raw.at(y, x) = center < cutoff ? center : qnanf();
+    // (a factor this large, or NaN, could make a depth infinite or NaN)
+    float far = fabsf(scale_inv) <= 1e30f ? 0.f : 2.f * kNearTaps;
+#pragma unroll
+    for (int i = 0; i < 25; ++i) far = fmaxf(far, fabsf(center - (float)tap[i] * scale_inv));
     float sum1 = 0.f, sum2 = 0.f;
-#pragma unroll
-    for (int dy = 0; dy < 5; ++dy) {
-        const int cy = y - 2 + dy;
-#pragma unroll
-        for (int dx = 0; dx < 5; ++dx) {
-            const int cx = x - 2 + dx;
-            // Every tap is computed; one outside the clipped window adds +0
-            // through a select (the sums are never -0, so their bits do not
-            // change). One straight block lets the compiler interleave the
-            // 25 taps' exponentials; a branch per tap kept them apart.
-            const bool in = cy >= 0 && cy < ty && cx >= 0 && cx < tx;
-            float val = (float)tap[dy * 5 + dx] * scale_inv;
-            float space2 = (float)((x - cx) * (x - cx) + (y - cy) * (y - cy));
-            float color2 = (center - val) * (center - val);
-            float weight = expf_cw(-(space2 * sig_space + color2 * sig_range));
-            sum1 += in ? val * weight : 0.f;
-            sum2 += in ? weight : 0.f;
-        }
-    }
+    if (!__all(far <= kNearTaps))
+        filter_sums<false, false>(tap, scale_inv, x, y, tx, ty, sum1, sum2);
+    else if (__all(x >= 2 && y >= 2 && tx == x + 3 && ty == y + 3))
+        filter_sums<true, true>(tap, scale_inv, x, y, tx, ty, sum1, sum2);
+    else
+        filter_sums<true, false>(tap, scale_inv, x, y, tx, ty, sum1, sum2);
     float fin = sum1 / sum2;
     filtered.at(y, x) = fin < cutoff ? fin : qnanf();
 }
@@ -130,6 +181,31 @@ template <class T> SICP_DEV T out_cast(float v);
 template <> SICP_DEV float out_cast<float>(float v) { return v; }
 template <> SICP_DEV uint8_t out_cast<uint8_t>(float v) { return (uint8_t)(int)v; }
 
+// The window's weighted sum and its weight, a whole number of at most 256 and
+// so exact in float. kInner: the window is not clipped, so that a tap's weight
+// is a constant; a wavefront away from the edges uses it (both levels of a
+// 1280x720 frame: 13.4 us, 17.0 with each tap's weight worked out).
+template <bool kInner, class T>
+SICP_DEV void pyrdown_sums(const T (&tap)[25], int x, int y, int tx, int ty, float& sum,
+                           float& count) {
+#pragma unroll
+    for (int dy = 0; dy < 5; ++dy) {
+        const int cy = 2 * y - 2 + dy;
+#pragma unroll
+        for (int dx = 0; dx < 5; ++dx) {
+            const int cx = 2 * x - 2 + dx;
+            // Selects instead of branches, as in filter_sums.
+            const float s = (float)tap[dy * 5 + dx];
+            const bool in = kInner || (cy >= 0 && cy < ty && cx >= 0 && cx < tx);
+            const bool use = in && !isnan_(s);
+            const float g = kInner ? binom5(4 - dy) * binom5(4 - dx)
+                                   : binom5(ty - cy - 1) * binom5(tx - cx - 1);
+            sum += use ? s * g : 0.f;
+            count += use ? g : 0.f;
+        }
+    }
+}
+
 // One output pixel from a source read through `src(y, x)` (global memory or
 // an LDS tile) of size scols x srows.
 template <class T, class Src>
@@ -143,23 +219,13 @@ SICP_DEV T pyrdown_px(const Src& src, int scols, int srows, int x, int y) {
 #pragma unroll
         for (int dx = 0; dx < 5; ++dx) tap[dy * 5 + dx] = src(cy, min(max(2 * x - 2 + dx, 0), scols - 1));
     }
-    float sum = 0.f;
-    int count = 0;
-#pragma unroll
-    for (int dy = 0; dy < 5; ++dy) {
-        const int cy = 2 * y - 2 + dy;
-#pragma unroll
-        for (int dx = 0; dx < 5; ++dx) {
-            const int cx = 2 * x - 2 + dx;
-            // Selects instead of branches, as in filter_px.
-            const float s = (float)tap[dy * 5 + dx];
-            const bool use = cy >= 0 && cy < ty && cx >= 0 && cx < tx && !isnan_(s);
-            const float g = binom5(ty - cy - 1) * binom5(tx - cx - 1);
-            sum += use ? s * g : 0.f;
-            count = use ? (int)((float)count + g) : count;
-        }
-    }
-    return out_cast<T>(sum / (float)count);
+    float sum = 0.f, count = 0.f;
+    const bool inner = x >= 1 && y >= 1 && tx == 2 * x + 3 && ty == 2 * y + 3;
+    if (__all(inner))
+        pyrdown_sums<true>(tap, x, y, tx, ty, sum, count);
+    else
+        pyrdown_sums<false>(tap, x, y, tx, ty, sum, count);
+    return out_cast<T>(sum / count);
 }
 
 template <class T> struct GlobalSrc {
@@ -194,6 +260,31 @@ __global__ __launch_bounds__(256) void intensity_kernel(View<uint8_t> rgb, View<
 // Sobel pair of the reference, {1,0,-1, 2,0,-2, 1,0,-1} and its transpose,
 // written as closed forms of the tap index below.
 
+// A wavefront away from the image's edges takes the constant tap indexes of
+// kInner (as in pyrdown_sums).
+template <bool kInner>
+SICP_DEV void derivative_sums(const uint8_t (&tap)[9], int cols, int rows, int x, int y,
+                              float& dxv, float& dyv) {
+    int k = 8;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            // Selects instead of branches, as in filter_sums; k counts the
+            // taps inside the image, as the reference's index does.
+            const int cy = y - 1 + j, cx = x - 1 + i;
+            const bool in = kInner || (cy >= 0 && cy < rows && cx >= 0 && cx < cols);
+            const float p = (float)tap[j * 3 + i];
+            const int r = k / 3, c = k - 3 * r;
+            const float wx = p * ((float)(1 - c) * (r == 1 ? 2.f : 1.f));
+            const float wy = p * ((float)(1 - r) * (c == 1 ? 2.f : 1.f));
+            dxv += in ? wx : 0.f;
+            dyv += in ? wy : 0.f;
+            k -= in ? 1 : 0;
+        }
+    }
+}
+
 SICP_DEV int2 derivative_px(const View<uint8_t>& img, const View<int16_t>& dx,
                             const View<int16_t>& dy, int x, int y) {
     uint8_t tap[9];
@@ -204,24 +295,10 @@ SICP_DEV int2 derivative_px(const View<uint8_t>& img, const View<int16_t>& dx,
         for (int i = 0; i < 3; ++i) tap[j * 3 + i] = row[min(max(x - 1 + i, 0), img.cols - 1)];
     }
     float dxv = 0.f, dyv = 0.f;
-    int k = 8;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            // Selects instead of branches, as in filter_px; k counts the
-            // taps inside the image, as the reference's index does.
-            const int cy = y - 1 + j, cx = x - 1 + i;
-            const bool in = cy >= 0 && cy < img.rows && cx >= 0 && cx < img.cols;
-            const float p = (float)tap[j * 3 + i];
-            const int r = k / 3, c = k - 3 * r;
-            const float wx = p * ((float)(1 - c) * (r == 1 ? 2.f : 1.f));
-            const float wy = p * ((float)(1 - r) * (c == 1 ? 2.f : 1.f));
-            dxv += in ? wx : 0.f;
-            dyv += in ? wy : 0.f;
-            k -= in ? 1 : 0;
-        }
-    }
+    if (__all(x >= 1 && y >= 1 && x + 1 < img.cols && y + 1 < img.rows))
+        derivative_sums<true>(tap, img.cols, img.rows, x, y, dxv, dyv);
+    else
+        derivative_sums<false>(tap, img.cols, img.rows, x, y, dxv, dyv);
     const int16_t gx = (int16_t)(int)dxv, gy = (int16_t)(int)dyv;
     dx.at(y, x) = gx;
     dy.at(y, x) = gy;
@@ -316,9 +393,8 @@ __global__ __launch_bounds__(256) void resize_map_kernel(View<float4> vsrc, View
 // functions as the single-image kernels above, so the results are
 // identical; what changes is only which launch computes which pixel.
 //
-//  1. level 0: bilateral filter + intensity of the new frame, and the model
-//     pyramid of the last frame (levels 1 and 2, the latter straight from
-//     level 0 through the same 2x2 means);
+//  1. level 0: the model pyramid of the last frame (levels 1 and 2), and the
+//     bilateral filter and intensity of the new one;
 //  2. PyrDown to levels 1 and 2 of depth and intensity: a workgroup owns an
 //     8x4 tile of level 2, computes the 20x12 level-1 window it needs into
 //     LDS (writing the level-1 pixels it owns), then its level-2 pixels;
@@ -343,13 +419,6 @@ __global__ __launch_bounds__(256) void frame_level0_kernel(View<uint16_t> d16, V
                                                            float cutoff, ModelPyramid mp,
                                                            FrameReset fr) {
     int b = blockIdx.x, x, y;
-    if (take_tile(b, d16.cols, d16.rows, x, y)) {
-        if (x < d16.cols && y < d16.rows) {
-            filter_px(d16, range, depth0, scale_inv, cutoff, x, y);
-            intensity_px(rgb, gray0, x, y);
-        }
-        return;
-    }
     // The model pyramid in tiles of 64 x 8 level-1 pixels (kept in LDS) and
     // the 32 x 4 level-2 pixels made of them, so level 0 is read once.
     __shared__ float4 lv[8][kModelTX], ln[8][kModelTX];
@@ -389,6 +458,16 @@ __global__ __launch_bounds__(256) void frame_level0_kernel(View<uint16_t> d16, V
         return;
     }
     b -= nx1 * ny1;
+    // (after the model's tiles, whose loads are then in flight during the
+    // filter: the launch took 12.7 us at 640x480 and takes 11.5; at 320x240 7.9
+    // with the filter first, 6.8 so)
+    if (take_tile(b, d16.cols, d16.rows, x, y)) {
+        if (x < d16.cols && y < d16.rows) {
+            filter_px(d16, range, depth0, scale_inv, cutoff, x, y);
+            intensity_px(rgb, gray0, x, y);
+        }
+        return;
+    }
     // the frame's resets, in the workgroups after the tiles
     const int nz = fr.zmin.cols * fr.zmin.rows;
     const int i = b * 256 + (int)(threadIdx.y * kTX + threadIdx.x);
