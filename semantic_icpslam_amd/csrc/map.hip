@@ -609,10 +609,14 @@ struct FuseArgs {
     float trunc_rcp;  // 1 / truncation, rounded to nearest
 };
 
+// Channel c of label L's colour (FuseMap.cu:18,570-572): (palette x label) % 255
+// in wrapping int arithmetic, which may be negative, narrowed to the byte that
+// the voxel keeps: the records are packed into words, where a sign would fill
+// the bytes above.
 SICP_DEV int palette_channel(int c, int L) {
     const int pal = c == 0 ? (1 << 25) - 1 : (c == 1 ? (1 << 15) - 1 : (1 << 21) - 1);
     int prod = (int)((uint32_t)pal * (uint32_t)L);
-    return prod % 255;
+    return prod % 255 & 0xff;
 }
 
 SICP_DEV int u8i(float v) { return (int)(uint8_t)(uint32_t)(int)v; }
