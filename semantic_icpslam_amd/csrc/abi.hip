@@ -178,18 +178,9 @@ int map_alloc(const sicp_map_config& cfg, sicp_map** out) {
         }
         d.one = one;
     }
-    if (cfg.unify_labels) {
-        // scratch of the neighbour label pass, here so that no later call allocates
-        if ((rc = dmalloc(m, &m->unify_snap, nblk * kBlockVoxels)) ||
-            (rc = dmalloc(m, &m->unify_mark, nblk))) {
-            map_free(m);
-            return rc;
-        }
-        hipError_t e = hipMemset(m->unify_mark, 0, nblk * sizeof(uint32_t));
-        if (e != hipSuccess) {
-            map_free(m);
-            return hip_fail(e, "hipMemset(unify marks)");
-        }
+    if (cfg.unify_labels && (rc = unify_scratch(m))) {
+        map_free(m);
+        return rc;
     }
     a.req_mask = (uint32_t)(q - 1);
     a.cap_pixels = (uint32_t)px;

@@ -13,8 +13,8 @@ struct sicp_map {
     sicp::AllocScratch alloc{};
     sicp_block* visible = nullptr;     // device, num_blocks
     uint32_t* unify_snap = nullptr;    // neighbour label pass: label snapshot, num_blocks * 512
-    uint32_t* unify_mark = nullptr;    // per heap slot: epoch of the last snapshot
-    uint32_t unify_epoch = 0;
+    uint32_t* unify_mark = nullptr;    // per heap slot: the pass of its last snapshot; then the
+                                       // pass under way and the last one that ended
     std::atomic<bool> mesh_lent{false};  // mesh extraction: the memory below is in a call's use
     uint32_t* mesh_counts = nullptr;   // device
     uint32_t* mesh_total = nullptr;    // pinned host
@@ -48,7 +48,10 @@ void host_loans_release();
 
 int map_alloc(const sicp_map_config& cfg, sicp_map** out);
 void map_free(sicp_map* m);
-// The neighbour label pass over the map's visible list (unify.hip).
+// The neighbour label pass over the map's visible list (unify.hip), and its
+// scratch, allocated with the map where every fusion runs the pass (no later
+// call allocates then), else by the first pass.
+int unify_scratch(sicp_map* map);
 int launch_unify(sicp_map* map, const int* gate, hipStream_t s);
 // `queue_cleared`: the hand-over queue count was cleared by launch_fuse_count
 // on the same stream.

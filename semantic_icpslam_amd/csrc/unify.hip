@@ -45,9 +45,12 @@ SICP_DEV uint32_t pack_label(const MapDev& m, size_t k) {
 __global__ __launch_bounds__(256) void unify_snapshot_kernel(MapDev m, const MapCounters* ctr,
                                                              const sicp_block* visible,
                                                              uint32_t* snap, uint32_t* mark,
-                                                             uint32_t epoch, const int* gate) {
+                                                             uint32_t* passes,
+                                                             const int* gate) {
     if (gate && *gate == 0) return;
     const uint32_t nv = ctr->visible;
+    const uint32_t epoch = passes[1] + 1u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) passes[0] = epoch;
     for (uint32_t b = blockIdx.x; b < nv; b += gridDim.x) {
         const int slot = visible[b].slot;
         if (threadIdx.x == 0) mark[slot] = epoch;
@@ -122,9 +125,11 @@ SICP_DEV void tally(Tallies& t, uint32_t w) {
 __global__ __launch_bounds__(64, 4) void unify_kernel(MapDev m, const MapCounters* ctr,
                                                    const sicp_block* visible,
                                                    const uint32_t* snap, const uint32_t* mark,
-                                                   uint32_t epoch, uint32_t count_mask,
+                                                   uint32_t* passes, uint32_t count_mask,
                                                    const int* gate) {
     if (gate && *gate == 0) return;
+    const uint32_t epoch = passes[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) passes[1] = epoch;
     __shared__ int nslot[27];
     __shared__ int nsnap[27];
     __shared__ uint32_t words[kWords];
@@ -296,25 +301,42 @@ __global__ __launch_bounds__(64, 4) void unify_kernel(MapDev m, const MapCounter
 
 }  // namespace
 
+int unify_scratch(sicp_map* map) {
+    const size_t n = (size_t)map->cfg.num_blocks;
+    uint32_t *snap = nullptr, *mark = nullptr;
+    hipError_t e = hipMalloc((void**)&snap, n * kBlockVoxels * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMalloc((void**)&mark, (n + 2) * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemset(mark, 0, (n + 2) * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) {
+        if (snap) (void)hipFree(snap);
+        if (mark) (void)hipFree(mark);
+        return hip_fail(e, "hipMalloc(unify scratch)");
+    }
+    map->unify_snap = snap;
+    map->unify_mark = mark;
+    map->owned.push_back(snap);
+    map->owned.push_back(mark);
+    return SICP_OK;
+}
+
 int launch_unify(sicp_map* map, const int* gate, hipStream_t s) {
     if (!map->unify_snap) {
-        const size_t n = (size_t)map->cfg.num_blocks;
-        hipError_t e = hipMalloc((void**)&map->unify_snap, n * 512 * sizeof(uint32_t));
-        if (e == hipSuccess) e = hipMalloc((void**)&map->unify_mark, n * sizeof(uint32_t));
-        if (e == hipSuccess) e = hipMemset(map->unify_mark, 0, n * sizeof(uint32_t));
-        if (e != hipSuccess) return hip_fail(e, "hipMalloc(unify scratch)");
-        map->owned.push_back(map->unify_snap);
-        map->owned.push_back(map->unify_mark);
+        const int rc = unify_scratch(map);
+        if (rc) return rc;
     }
-    // Epochs distinguish the blocks stamped by this call from earlier ones;
-    // the mark array starts at 0 and the first epoch is 1.
-    const uint32_t epoch = ++map->unify_epoch;
+    // The pass's number tells the blocks that it stamped from those of earlier
+    // passes. It is kept on the device, so that a replayed graph counts on: the
+    // snapshot forms it from the passes that ended, [1], and leaves it in [0];
+    // the update takes it from there and stores it in [1], so neither launch
+    // reads the word that it writes. The marks start at 0, the first pass is 1.
+    uint32_t* passes = map->unify_mark + map->cfg.num_blocks;
     const uint32_t mask = map->cfg.max_label_count <= 255 ? 0xffu : 0xffffu;
     unify_snapshot_kernel<<<4096, 256, 0, s>>>(map->dev, map->ctr, map->visible, map->unify_snap,
-                                                map->unify_mark, epoch, gate);
+                                                map->unify_mark, passes, gate);
     SICP_LAUNCH_CHECK("unify_snapshot_kernel");
     unify_kernel<<<8192, 64, 0, s>>>(map->dev, map->ctr, map->visible, map->unify_snap,
-                                      map->unify_mark, epoch, mask, gate);
+                                      map->unify_mark, passes, mask, gate);
     SICP_LAUNCH_CHECK("unify_kernel");
     return SICP_OK;
 }
