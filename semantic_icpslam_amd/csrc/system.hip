@@ -763,10 +763,21 @@ int sicp_system_last_result(sicp_system* s, sicp_frame_result* out, void* stream
     int device = -1;
     // a copy is also right from another device's stream, a kernel is not
     if (hipGetDevice(&device) == hipSuccess && device == s->device) loan.take();
+    bool gathered = false;
     if (loan.ptr) {
-        result_kernel<<<1, 64, 0, st>>>(s->st, s->map->ctr, s->last->meta,
-                                        (ResultWords*)loan.ptr);
-        SICP_LAUNCH_CHECK("result_kernel");
+        // The launch's own status: hipGetLastError would also report an error
+        // that another call of the thread left. Refused, it has queued nothing,
+        // and the words are copied.
+        const TrackState* track = s->st;
+        const MapCounters* ctr = s->map->ctr;
+        const FrameMeta* meta = s->last->meta;
+        ResultWords* words = (ResultWords*)loan.ptr;
+        void* args[] = {&track, &ctr, &meta, &words};
+        gathered = hipLaunchKernel((const void*)result_kernel, dim3(1), dim3(64), args, 0, st) ==
+                   hipSuccess;
+        if (!gathered) (void)hipGetLastError();
+    }
+    if (gathered) {
         const int rc = loan.wait(&r, sizeof(r), st);
         if (rc) return rc;
     } else {
