@@ -368,13 +368,18 @@ __global__ __launch_bounds__(kMeshThreads) void mesh_emit_kernel(MapDev m,
 
 // The counts' device memory and the host word, kept with the map from the
 // first call on and lent to one call at a time; a call that finds them lent
-// (another thread's) allocates its own for its duration.
+// (another thread's) allocates its own for its duration. A call that fails once
+// something is queued waits for its stream before it gives them back; where
+// that fails too, a kernel may still write them and they are given up.
 struct MeshLoan {
     sicp_map* map;
+    hipStream_t stream;
     bool kept;
+    bool queued = false;  // launches that have not been waited for
     uint32_t* dev = nullptr;
     uint32_t* host = nullptr;
-    explicit MeshLoan(sicp_map* m) : map(m), kept(!m->mesh_lent.exchange(true)) {}
+    MeshLoan(sicp_map* m, hipStream_t s)
+        : map(m), stream(s), kept(!m->mesh_lent.exchange(true)) {}
     int take(size_t words) {
         if (kept) {
             dev = map->mesh_counts;
@@ -393,10 +398,13 @@ struct MeshLoan {
         return SICP_OK;
     }
     ~MeshLoan() {
+        const bool lost = queued && hipStreamSynchronize(stream) != hipSuccess;
         if (kept) {
+            if (lost) map->mesh_counts = map->mesh_total = nullptr;
             map->mesh_lent.store(false);
             return;
         }
+        if (lost) return;
         if (dev) (void)hipFree(dev);
         if (host) (void)hipHostFree(host);
     }
@@ -406,10 +414,11 @@ int launch_mesh(sicp_map* map, float* vertices, float* normals, uint8_t* colors,
                 uint32_t max_triangles, uint32_t* n_out, uint32_t* total_out, hipStream_t s) {
     const uint32_t cap = (uint32_t)map->cfg.num_blocks;
     const uint32_t nchunks = div_up(cap, kMeshChunk);
-    MeshLoan mem(map);
+    MeshLoan mem(map, s);
     const int rc = mem.take((size_t)cap + nchunks);
     if (rc) return rc;
     const MeshCounts ct{mem.dev, mem.dev + cap, nchunks};
+    mem.queued = true;
     mesh_reset_kernel<<<div_up(nchunks, 256), 256, 0, s>>>(ct);
     SICP_LAUNCH_CHECK("mesh_reset_kernel");
     const int grid = (int)(cap < kMeshGrid ? cap : kMeshGrid);
@@ -420,6 +429,7 @@ int launch_mesh(sicp_map* map, float* vertices, float* normals, uint8_t* colors,
         map->dev, map->ctr, ct, map->cfg.voxel_size, out, mem.host);
     SICP_LAUNCH_CHECK("mesh_emit_kernel");
     SICP_HIP(hipStreamSynchronize(s));
+    mem.queued = false;
     const uint32_t tot = *mem.host;
     *n_out = tot < max_triangles ? tot : max_triangles;
     if (total_out) *total_out = tot;
