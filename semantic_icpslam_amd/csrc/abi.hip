@@ -37,6 +37,22 @@ namespace {
 std::mutex g_loans_mu;
 void* g_loans[kHostLoansKept];
 int g_loans_free = 0;
+
+// Another thread may be capturing a graph in the mode that forbids allocations
+// and frees elsewhere, and would lose its capture to them; the loans' concern
+// no stream.
+struct BesideCaptures {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~BesideCaptures() {
+        if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+void free_loan(void* p) {
+    const BesideCaptures scope;
+    if (hipHostFree(p) != hipSuccess) (void)hipGetLastError();
+}
 }  // namespace
 
 void HostLoan::take() {
@@ -45,15 +61,11 @@ void HostLoan::take() {
         if (g_loans_free > 0) ptr = g_loans[--g_loans_free];
     }
     if (ptr) return;
-    // Another thread may be capturing a graph in the mode that forbids
-    // allocations elsewhere; this one concerns no stream.
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const BesideCaptures scope;
     if (hipHostMalloc(&ptr, kHostLoanBytes, hipHostMallocPortable) != hipSuccess) {
         ptr = nullptr;
         (void)hipGetLastError();
     }
-    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 
 int HostLoan::wait(void* dst, size_t bytes, hipStream_t s) {
@@ -75,7 +87,7 @@ HostLoan::~HostLoan() {
             return;
         }
     }
-    (void)hipHostFree(ptr);
+    free_loan(ptr);
 }
 
 void host_loans_release() {
@@ -86,7 +98,7 @@ void host_loans_release() {
         std::swap(n, g_loans_free);
         std::memcpy(idle, g_loans, sizeof(idle));
     }
-    for (int i = 0; i < n; ++i) (void)hipHostFree(idle[i]);
+    for (int i = 0; i < n; ++i) free_loan(idle[i]);
 }
 
 static bool pow2(uint32_t v) { return v && !(v & (v - 1)); }
