@@ -232,7 +232,9 @@ size_t sicp_raycast_backward_scratch_size(void);
  * Triangles past `max_triangles` are dropped (MaxTriangles,
  * DeviceMap.h:181); `n_triangles` gets the number written and `n_total`
  * (may be NULL) the number found. With max_triangles = 0 the call only
- * counts. Synchronises `stream`. */
+ * counts. Synchronises `stream`. The map's first extraction allocates scratch of
+ * about num_blocks x 4 bytes, kept with the map; one that runs while another
+ * thread's is under way on the same map allocates its own for its duration. */
 int sicp_mesh_scene(sicp_map* map, float* vertices_dev, float* normals_dev, uint8_t* colors_dev,
                     uint32_t max_triangles, uint32_t* n_triangles, uint32_t* n_total,
                     void* stream);
@@ -258,7 +260,13 @@ int sicp_mesh_write_ply(const char* path, const float* vertices, const float* no
  * synchronises `stream` and copies the 29 sums to the host; when `A_host`,
  * `b_host`, `residual_host` are non-NULL it also expands them exactly like
  * the reference's CreateMatrix<6,7> (Reduction.cu:6-16): A row-major 6x6
- * (mirrored), b[6], residual = {sum r^2, count}. */
+ * (mirrored), b[6], residual = {sum r^2, count}. Host results (of this step,
+ * its variants but the static one, RGBStep, SO3Step and the frame result) pass
+ * through a 2 KiB pinned buffer of a process-wide pool: a call that finds none
+ * idle allocates one (hipHostMalloc), and without memory for it copies instead.
+ * At most 16 idle ones are kept, and freed when the last map is destroyed. A
+ * call whose wait for `stream` fails does not give its buffer back, since a
+ * kernel may still write it. */
 int sicp_icp_step(sicp_image vcurr, sicp_image vlast, sicp_image ncurr, sicp_image nlast,
                   const sicp_pose_f* curr, const sicp_pose_f* last, sicp_intrinsics K,
                   void* partials_dev, float* sums_dev, float* host_sums,

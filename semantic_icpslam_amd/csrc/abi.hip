@@ -37,6 +37,7 @@ namespace {
 std::mutex g_loans_mu;
 void* g_loans[kHostLoansKept];
 int g_loans_free = 0;
+int g_loans_maps = 0;  // maps alive
 
 // Another thread may be capturing a graph in the mode that forbids allocations
 // and frees elsewhere, and would lose its capture to them; the loans' concern
@@ -90,11 +91,17 @@ HostLoan::~HostLoan() {
     free_loan(ptr);
 }
 
+void host_loans_retain() {
+    std::lock_guard<std::mutex> lock(g_loans_mu);
+    ++g_loans_maps;
+}
+
 void host_loans_release() {
     void* idle[kHostLoansKept];
     int n = 0;
     {
         std::lock_guard<std::mutex> lock(g_loans_mu);
+        if (--g_loans_maps > 0) return;
         std::swap(n, g_loans_free);
         std::memcpy(idle, g_loans, sizeof(idle));
     }
@@ -148,6 +155,7 @@ int map_alloc(const sicp_map_config& cfg, sicp_map** out) {
     if (cfg.unify_labels != 0 && cfg.unify_labels != 1) return invalid("unify_labels must be 0 or 1");
     if (cfg.tsdf_half != 0 && cfg.tsdf_half != 1) return invalid("tsdf_half must be 0 or 1");
     sicp_map* m = new sicp_map();
+    host_loans_retain();
     m->cfg = cfg;
     int rc = SICP_OK;
     const size_t nb = (size_t)cfg.num_buckets, nblk = (size_t)cfg.num_blocks;
