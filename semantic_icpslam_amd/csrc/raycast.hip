@@ -409,6 +409,7 @@ struct RayArgs {
     int cols, rows;
     int tcols, trows;        // raycast_kernel: 8x8-pixel tiles across and down
     int first_pass_samples;  // the first pass's hand-over point (raycast_kernel only)
+    int cube_margin;         // ray_cube_margin of it
 };
 
 // The ray of pixel (x, y) (RenderScene.cu:393-421): start point and unit
@@ -463,11 +464,13 @@ SICP_DEV bool ray_setup(const MapDev& m, const View<float>& zmin, const View<flo
 // (10 bits an axis: a neighbour's tag is one addition away, and one compare
 // tests the lane's cached block), and a missing block by the heap slot
 // num_blocks, whose voxels are kept empty (NaN, weight 0), so that no read
-// tests for it. Rays that leave the 1024-block cube around the wavefront's
-// middle (16 m long at 2 mm voxels) are handed to the second pass.
+// tests for it. Rays whose ends do not lie well inside the 1024-block cube around
+// the wavefront's middle (16 m long at 2 mm voxels) are handed to the second
+// pass from their first sample on (raycasts of such ranges, 640x480 / 2 mm: 1.6
+// ms with depths to 12 m and 7.6 to 60 m; 10.4 and 54.6 as the reference's loop
+// over both passes).
 constexpr int kRayLdsEntries = 256;  // one 64-bit word each: tag + 1, slot
 constexpr uint32_t kTagX = 1u, kTagY = 1u << 10, kTagZ = 1u << 20;
-constexpr int kTagSpan = 1024;
 constexpr uint32_t kNoTag = 0xffffffffu;
 // Samples of a one-voxel run read together, and the waiting lanes' share that
 // has them served: measured at 640x480 / 5 mm, 2 mm, 1280x720 / 4 mm and
@@ -484,15 +487,15 @@ constexpr int kRayAhead = 2, kRayServe = 3;
 constexpr int kRaySuper = 8;
 
 // The tag of block b relative to the wavefront's origin, and whether a point
-// lies well inside the cube that tags can name.
+// lies inside the cube that tags can name, `margin` blocks from its faces.
 SICP_DEV uint32_t block_tag(i3 b, uint32_t otag) {
     return (uint32_t)b.x * kTagX + (uint32_t)b.y * kTagY + (uint32_t)b.z * kTagZ - otag;
 }
-SICP_DEV bool in_cube(v3 p, i3 o) {
-    const uint32_t x = (uint32_t)((floor_i(p.x) >> 3) - o.x - 4),
-                   y = (uint32_t)((floor_i(p.y) >> 3) - o.y - 4),
-                   z = (uint32_t)((floor_i(p.z) >> 3) - o.z - 4);
-    const uint32_t n = (uint32_t)(kTagSpan - 8);
+SICP_DEV bool in_cube(v3 p, i3 o, int margin) {
+    const uint32_t x = (uint32_t)((floor_i(p.x) >> 3) - o.x - margin),
+                   y = (uint32_t)((floor_i(p.y) >> 3) - o.y - margin),
+                   z = (uint32_t)((floor_i(p.z) >> 3) - o.z - margin);
+    const uint32_t n = (uint32_t)(kTagSpan - 2 * margin);
     return (x < n) & (y < n) & (z < n);
 }
 
@@ -727,7 +730,8 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(MapDev map, View<float4>
     v3 result{0.f, 0.f, 0.f};
     float dist_s = 0.f, sdf = 1.0f, prev_sdf = 1.0f;
     // The tags' origin: the block in the middle of the first ray, less half
-    // the span. A ray whose ends lie in the cube stays in it.
+    // the span. A ray whose ends lie ray_cube_margin from the faces stays in
+    // the cube for its samples of this pass.
     uint32_t otag = 0;
     i3 o{0, 0, 0};
     {
@@ -746,7 +750,7 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(MapDev map, View<float4>
             otag = (uint32_t)o.x * kTagX + (uint32_t)o.y * kTagY + (uint32_t)o.z * kTagZ;
             if (hits) {
                 const v3 e = add(ray.start, scale(ray.dist_e - ray.dist_s, ray.dir));
-                if (!in_cube(ray.start, o) || !in_cube(e, o)) {
+                if (!in_cube(ray.start, o, g.cube_margin) || !in_cube(e, o, g.cube_margin)) {
                     deferred = true;
                     status = kEnd;
                 }
@@ -880,13 +884,13 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(MapDev map, View<float4>
         const v3 at = result;
         const float sdf_in = crossed ? prev_sdf : sdf;
         result = add(result, scale(sdf * m.step_scale, ray.dir));
-        bool ok = in_cube(result, o);
+        bool ok = in_cube(result, o, kTagReach);
         if (ok) {
             sdf = ray_interp<kTable>(m, lds, result, otag, false, 0u);
             result = add(result, scale(sdf * m.step_scale, ray.dir));
             // (a NaN position has no normal: its reads would be NaN)
             const bool number = !isnan_(result.x) && !isnan_(result.y) && !isnan_(result.z);
-            ok = !number || in_cube(result, o);
+            ok = !number || in_cube(result, o, kTagReach);
             v3 normal;
             if (ok && number && ray_normal<kTable>(m, lds, result, otag, pose, normal)) {
                 v3 r = mv(pose.Rinv, sub(scale(result, m.voxel), pose.t));
@@ -1446,7 +1450,7 @@ int launch_raycast_adjoint(MapDev m, View<float> zmin, View<float> zmax, PoseArg
                            const int32_t* pixels, int n, const float* grad_v,
                            const float* grad_n, float* grad_sdf, float* grad_px,
                            double* partials, double* grad_pose, hipStream_t s) {
-    AdjointArgs a{RayArgs{invfx, invfy, cx, cy, cols, rows, 0, 0, 0}, pixels, n, grad_v, grad_n,
+    AdjointArgs a{RayArgs{invfx, invfy, cx, cy, cols, rows, 0, 0, 0, 0}, pixels, n, grad_v, grad_n,
                   grad_sdf, grad_px, partials};
     int nb = (int)div_up(n > 0 ? n : 1, kAdjThreads / kRayGroup);
     if (nb > kAdjMaxBlocks) nb = kAdjMaxBlocks;
@@ -1494,7 +1498,9 @@ int launch_raycast_gated(MapDev m, View<float4> vmap, View<float4> nmap, View<fl
         tune.second_pass_workgroups < 1 || tune.second_pass_workgroups > kRayTuneMaxWorkgroups ||
         (tune.lds_block_table != 0 && tune.lds_block_table != 1))
         return invalid("raycast: tuning outside 1..4096 samples, 1..65536 workgroups, table 0/1");
-    RayArgs g{invfx, invfy, cx, cy, vmap.cols, vmap.rows, (int)div_up(vmap.cols, 8), (int)div_up(vmap.rows, 8), tune.first_pass_samples};
+    const RayArgs g{invfx, invfy, cx, cy, vmap.cols, vmap.rows, (int)div_up(vmap.cols, 8),
+                    (int)div_up(vmap.rows, 8), tune.first_pass_samples,
+                    ray_cube_margin(tune.first_pass_samples)};
     if (!gate) gate = m.one;
     if (!nonempty) nonempty = reinterpret_cast<const uint32_t*>(m.one);
     if (!queue_cleared) {

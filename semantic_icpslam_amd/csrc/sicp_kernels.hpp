@@ -329,6 +329,16 @@ struct RayTuning {
 };
 constexpr int kRayTuneMaxSamples = 4096;
 constexpr int kRayTuneMaxWorkgroups = 65536;
+// The first pass names blocks inside a cube of kTagSpan blocks a side. A point
+// kTagReach from its faces may be read around: the block-width step's next
+// sample (two blocks at most, rounded) and the reads of a normal. A ray's
+// samples keep that distance if both its ends keep ray_cube_margin: a sample's
+// position is the last one's plus a step, rounded, which below 2^24 voxels moves
+// it by half a voxel at most. (Further out every block is beyond the keys' range
+// on that axis, for all the rays of the cube, and so missing whatever its name.)
+constexpr int kTagSpan = 1024, kTagReach = 4;
+constexpr int ray_cube_margin(int samples) { return kTagReach + (samples + 15) / 16; }
+static_assert(2 * ray_cube_margin(kRayTuneMaxSamples) < kTagSpan, "some rays fit the cube");
 int launch_raycast(MapDev m, View<float4> vmap, View<float4> nmap, View<float> zmin,
                    View<float> zmax, PoseArg pose, float invfx, float invfy, float cx, float cy,
                    const int* gate, hipStream_t s);
