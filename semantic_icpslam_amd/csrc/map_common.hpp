@@ -37,15 +37,6 @@ SICP_DEV i3 voxel_to_block(i3 v) {
     return i3{v.x / kBlockSide, v.y / kBlockSide, v.z / kBlockSide};
 }
 
-// voxelPosToLocalIdx (DeviceMap.cu:186-201,218-220).
-SICP_DEV int voxel_local_idx(i3 v) {
-    int x = v.x % kBlockSide, y = v.y % kBlockSide, z = v.z % kBlockSide;
-    if (x < 0) x += kBlockSide;
-    if (y < 0) y += kBlockSide;
-    if (z < 0) z += kBlockSide;
-    return z * kBlockSide * kBlockSide + y * kBlockSide + x;
-}
-
 // ---------------------------------------------------------- voxel storage --
 // The FP32 form keeps sicp_voxel_geom records; the half form one 32-bit word
 // per voxel (sdf as IEEE half in bits 0-15, weight in bits 16-23) and the

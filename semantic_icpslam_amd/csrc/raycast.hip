@@ -7,10 +7,11 @@
 // atomicMin / atomicMax on the float bits (all depths are positive, where the
 // IEEE bit order is the numeric order) — no rendering-block list, no
 // host round trip.
-// Raycast (Rendering::operator(), RenderScene.cu:380-488): one thread per
-// pixel, 8x8-pixel workgroups (one wavefront) so neighbouring rays march
-// through the same voxel blocks; each ray keeps the reference's one-entry
-// block cache.
+// Raycast (Rendering::operator(), RenderScene.cu:380-488): a first pass of one
+// lane per pixel, 8x8-pixel workgroups (one wavefront) so that neighbouring rays
+// march through the same voxel blocks, whose lookups they share in LDS; a second
+// pass of eight lanes per ray for the rays still marching then. The adjoint runs
+// the second pass's march.
 #include "map_common.hpp"
 
 namespace sicp {
@@ -293,92 +294,8 @@ struct AxisPair {
 };
 SICP_DEV AxisPair axis_pair(float q) { return AxisPair{floor_i(q), floor_i(q + 1.0f), q - floorf(q)}; }
 
-// Slots of the (up to) eight blocks the corners of an interpolated read touch:
-// per axis the blocks of v0 and v1 (equal, or neighbours). One lookup site,
-// looped, instead of one per corner.
-struct CornerBlocks {
-    int s[8];  // [dx + 2 dy + 4 dz]; dx = 1 only when the x blocks differ, etc.
-};
-SICP_DEV void corner_blocks(const MapDev& m, const AxisPair& X, const AxisPair& Y,
-                            const AxisPair& Z, const BlockCache& c, CornerBlocks& cb) {
-    const int bx0 = X.v0 >> 3, by0 = Y.v0 >> 3, bz0 = Z.v0 >> 3;
-    const int nx = (X.v1 >> 3) != bx0, ny = (Y.v1 >> 3) != by0, nz = (Z.v1 >> 3) != bz0;
-    int s0 = -1, s1 = -1, s2 = -1, s3 = -1, s4 = -1, s5 = -1, s6 = -1, s7 = -1;
-#pragma unroll 1
-    for (int b = 0; b < 8; ++b) {
-        const int dx = b & 1, dy = (b >> 1) & 1, dz = b >> 2;
-        if (dx > nx || dy > ny || dz > nz) continue;
-        const int bx = dx ? (X.v1 >> 3) : bx0, by = dy ? (Y.v1 >> 3) : by0,
-                  bz = dz ? (Z.v1 >> 3) : bz0;
-        const int sl = cache_has(c, bx, by, bz) ? c.slot : map_lookup(m, bx, by, bz);
-        s0 = b == 0 ? sl : s0;
-        s1 = b == 1 ? sl : s1;
-        s2 = b == 2 ? sl : s2;
-        s3 = b == 3 ? sl : s3;
-        s4 = b == 4 ? sl : s4;
-        s5 = b == 5 ? sl : s5;
-        s6 = b == 6 ? sl : s6;
-        s7 = b == 7 ? sl : s7;
-    }
-    cb.s[0] = s0;
-    cb.s[1] = s1;
-    cb.s[2] = s2;
-    cb.s[3] = s3;
-    cb.s[4] = s4;
-    cb.s[5] = s5;
-    cb.s[6] = s6;
-    cb.s[7] = s7;
-}
-
-// The slot of corner (cx, cy, cz) in {0,1}^3 (selected without indexing, so
-// the slots stay in registers).
-SICP_DEV int corner_slot(const CornerBlocks& cb, const AxisPair& X, const AxisPair& Y,
-                         const AxisPair& Z, int cx, int cy, int cz) {
-    const int dx = cx && ((X.v1 >> 3) != (X.v0 >> 3));
-    const int dy = cy && ((Y.v1 >> 3) != (Y.v0 >> 3));
-    const int dz = cz && ((Z.v1 >> 3) != (Z.v0 >> 3));
-    const int a0 = dx ? cb.s[1] : cb.s[0], a1 = dx ? cb.s[3] : cb.s[2];
-    const int a2 = dx ? cb.s[5] : cb.s[4], a3 = dx ? cb.s[7] : cb.s[6];
-    const int b0 = dy ? a1 : a0, b1 = dy ? a3 : a2;
-    return dz ? b1 : b0;
-}
-
-// Rendering::readSdfInterped (RenderScene.cu:310-343) in three parts: the
-// voxel indices of the eight corners (-1 for a missing block) with `valid`
-// of the last corner's lookup, the eight loads, the blend. Corner order,
-// NaN for a missing block and the blend order are the reference's. When all
-// eight corners lie in the cached block (the common case) no lookup is made.
-SICP_DEV void interp_corners(const MapDev& m, const AxisPair& X, const AxisPair& Y,
-                             const AxisPair& Z, const BlockCache& c, int (&idx)[8], bool& valid) {
-    if (cache_has(c, X.v0 >> 3, Y.v0 >> 3, Z.v0 >> 3) && (X.v1 >> 3) == c.x &&
-        (Y.v1 >> 3) == c.y && (Z.v1 >> 3) == c.z) {
-        const int base = c.slot * kBlockVoxels;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            idx[i] = base + local_of((i & 1) ? X.v1 : X.v0, (i & 2) ? Y.v1 : Y.v0,
-                                     (i & 4) ? Z.v1 : Z.v0);
-        valid = true;
-    } else {
-        CornerBlocks cb;
-        corner_blocks(m, X, Y, Z, c, cb);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int sl = corner_slot(cb, X, Y, Z, i & 1, (i >> 1) & 1, i >> 2);
-            idx[i] = sl < 0 ? -1
-                            : sl * kBlockVoxels + local_of((i & 1) ? X.v1 : X.v0,
-                                                           (i & 2) ? Y.v1 : Y.v0,
-                                                           (i & 4) ? Z.v1 : Z.v0);
-        }
-        valid = corner_slot(cb, X, Y, Z, 1, 1, 1) >= 0;
-    }
-}
-// Every load issued (a missing corner reads voxel 0 and is replaced by NaN).
-SICP_DEV void interp_loads(const MapDev& m, const int (&idx)[8], float (&sd)[8]) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sd[i] = vox_sdf(m, (size_t)(idx[i] < 0 ? 0 : idx[i]));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) sd[i] = idx[i] < 0 ? qnanf() : sd[i];
-}
+// Rendering::readSdfInterped (RenderScene.cu:310-343) from its eight corners, NaN
+// for a missing block's, in the reference's order.
 SICP_DEV float interp_blend(const float (&sd)[8], const AxisPair& X, const AxisPair& Y,
                             const AxisPair& Z) {
     const float fx = X.frac, fy = Y.frac, fz = Z.frac;
@@ -391,19 +308,6 @@ SICP_DEV float interp_blend(const float (&sd)[8], const AxisPair& X, const AxisP
     r3 = (1.0f - fy) * r0 + fy * r1;
     return (1.0f - fz) * r2 + fz * r3;
 }
-SICP_DEV float interp_axes(const MapDev& m, AxisPair X, AxisPair Y, AxisPair Z, BlockCache& c,
-                           bool& valid) {
-    int idx[8];
-    float sd[8];
-    interp_corners(m, X, Y, Z, c, idx, valid);
-    interp_loads(m, idx, sd);
-    return interp_blend(sd, X, Y, Z);
-}
-
-SICP_DEV float read_sdf_interped(const MapDev& m, v3 pt, BlockCache& c, bool& valid) {
-    return interp_axes(m, axis_pair(pt.x), axis_pair(pt.y), axis_pair(pt.z), c, valid);
-}
-
 struct RayArgs {
     float invfx, invfy, cx, cy;
     int cols, rows;

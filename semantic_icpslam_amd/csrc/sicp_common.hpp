@@ -82,7 +82,6 @@ template <class T> SICP_DEV T early_load(const T* p) {
 // A device flag written by an earlier launch (a gate: 0 skips the launch's
 // work), or 1 when there is none.
 SICP_DEV int flag_or_one(const int* flag) { return flag ? early_load(flag) : 1; }
-SICP_DEV bool gate_closed(const int* gate) { return flag_or_one(gate) == 0; }
 
 // --------------------------------------------------------------- division --
 // Correctly rounded quotients from a shared reciprocal (Markstein, "Computation
