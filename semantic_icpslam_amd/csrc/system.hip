@@ -760,9 +760,12 @@ int sicp_system_last_result(sicp_system* s, sicp_frame_result* out, void* stream
     hipStream_t st = (hipStream_t)stream;
     ResultWords r;
     HostLoan loan;
-    int device = -1;
-    // a copy is also right from another device's stream, a kernel is not
-    if (hipGetDevice(&device) == hipSuccess && device == s->device) loan.take();
+    // A copy is also right on another device's stream; a kernel would run there
+    // and read this device's memory.
+    int current = -1, streams = -1;
+    if (hipGetDevice(&current) == hipSuccess && current == s->device &&
+        (!st || (hipStreamGetDevice(st, &streams) == hipSuccess && streams == s->device)))
+        loan.take();
     bool gathered = false;
     if (loan.ptr) {
         // The launch's own status: hipGetLastError would also report an error
