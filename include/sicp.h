@@ -432,16 +432,17 @@ typedef struct sicp_system_config {
                                 sums in plain FP32 (BlockReduce / Reduce<float,
                                 29>, Reduction.cu:29-60, 315, 374). */
     int32_t icp_spread;      /* 1 (default): the ICP reduction takes one pixel
-                                per thread while that makes at most a
-                                workgroup per compute unit (in the FP32
-                                compensated form, on levels of at most 320 x
-                                256 pixels), since one level alone would
-                                leave the GPU mostly idle; 0: four pixels per
-                                thread at every level, for systems run
-                                together (sicp_batch_*) whose launches
-                                already fill the GPU. The sums' order
-                                depends on it, so runs compared bit for bit
-                                use the same value. */
+                                per thread on levels of at most 131072 pixels
+                                (a 512-thread workgroup per compute unit; in
+                                the FP32 compensated form, of at most 320 x
+                                256), since one level alone would leave the
+                                GPU mostly idle; 0: four pixels per thread,
+                                for systems run together (sicp_batch_*) whose
+                                launches already fill the GPU. Levels above
+                                131072 pixels (524288 with 0) take more per
+                                thread; in the compensated form, four up to
+                                524288. The sums' order depends on it, so runs
+                                compared bit for bit use the same value. */
 } sicp_system_config;
 
 typedef struct sicp_system sicp_system;

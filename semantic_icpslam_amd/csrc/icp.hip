@@ -51,7 +51,10 @@ struct IcpGeom {
 // a column fetch in one round trip instead of two, before the pixels' loads
 // (wide_rows_load). At 640x480 a level-0 launch spans 9.0 us against 11.6, a
 // level-1 one 7.2 against 8.5, a level-2 one 7.5 to 8.8 against 7.1 to 8.5;
-// the frame takes 410 us against 442.
+// the frame takes 410 us against 442. The tracking of larger frames, this form
+// against the 256-thread one: 1280x720 327 us against 378, 1920x1080 439 and 506,
+// 2304x1728 654 and 729; with the photometric term 601 and 690, 887 and 961, 1464
+// and 1447, the one size found where it is not the faster.
 // The compensated form keeps the 256-thread layout: its rounding depends on
 // the order of the sums.
 constexpr int kWideThreads = 512, kWideMaxBlocks = 256;
@@ -389,7 +392,10 @@ SICP_DEV void icp_accumulate(const View<float4>& vcurr, const View<float4>& vlas
     // A launch of one pixel per thread runs a one-slot copy of the pass (a
     // uniform choice), so neither copy carries per-slot branches that would
     // split the slots' loads and arithmetic into separate blocks; a wide one of
-    // up to three a three-slot copy.
+    // up to three a three-slot copy (a frame with 14 iterations at level 0, that
+    // copy against the four-slot one: chunks of 516 pixels 234 us against 237, 675
+    // 248 and 252, 919 251 and 256, 1020 251 and 256, 1200 255 and 260, 1519 259
+    // and 263; with the photometric term 385 and 389 to 457 and 465).
     const bool single = kWide ? g.chunk <= NT : stride >= g.n;
     const bool three = kWide && g.chunk <= 3 * NT;
     IcpBatch bt;
@@ -1272,8 +1278,9 @@ inline int icp_blocks(int n, bool spread) {
     return b < 1 ? 1 : (b > kIcpMaxBlocks ? kIcpMaxBlocks : b);
 }
 
-// The tracking loop's workgroups: wide ones in FP64, one pixel per thread as
-// far as they go (four without `spread`).
+// The tracking loop's workgroups: wide ones in FP64, one pixel per thread up to
+// 131072 pixels (kWideMaxBlocks of them), or four up to 524288 without `spread`;
+// larger images take more per thread.
 inline int icp_iteration_blocks(int n, bool k32, bool spread) {
     if (k32) return icp_blocks(n, spread);
     const int b = (int)div_up(n, spread ? kWideThreads : kWideThreads * kPixPerThread);

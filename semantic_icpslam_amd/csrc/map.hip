@@ -236,7 +236,7 @@ SICP_DEV uint2 chunk_offset(const uint32_t* sums, uint32_t w, uint32_t n);
 // the chunk) and stores the total — no separate scan launches. A rank's
 // linking and the clearing of the new blocks need no more than the rank and
 // the total, so they ride in the same launch (as a launch of their own they
-// took 4.7 us a frame, nearly all of it the launch).
+// took 4.9 us a frame, nearly all of it the launch).
 template <int P>
 __global__ __launch_bounds__(256) void alloc_count_kernel(MapDev m, AllocScratch a,
                                                           View<float> depth, PoseArg pa,
@@ -639,8 +639,8 @@ SICP_DEV int mean_channel(int c, int w, int c0, float y) {
 // changes, forms its quotients from shared reciprocals, and takes a new voxel
 // down the same path (one code for eight z steps: unrolled it did not stay in
 // the instruction cache). 640x480 / 5 mm 35.5 to 23.3 us a launch, at 2 mm
-// 307 to 172, 1280x720 / 4 mm (half) 53.7 to 32.4, 320x240 / 1 cm 25 to 16.3;
-// the packing adds 0.5 to 2 us to the allocation's first launch.
+// 287 to 157, 1280x720 / 4 mm (half) 57 to 32.5, 320x240 / 1 cm 25 to 16.6;
+// the packing adds up to 2 us to the allocation's first launch.
 template <bool kHalf, bool kSem>
 __global__ __launch_bounds__(256) void fuse_kernel(MapDev map, const MapCounters* ctr,
                                                    const sicp_block* visible,

@@ -14,8 +14,8 @@
 // What bounds it: memory round trips and instructions, not bytes. With every
 // voxel reading its 8 corners, 24 neighbours and 8 colours itself, and the few
 // voxels on the surface writing up to 15 vertices in turn while the others
-// waited, the passes took 70 and 281 us on 6000 blocks (640x480 / 5 mm); a
-// block's 1331 staged values, and a thread per vertex, take 40 and 63.
+// waited, the passes took 68 and 302 us on 6000 blocks (640x480 / 5 mm); a
+// block's 1331 staged values, and a thread per vertex, take 45 and 67.
 #include <cstdio>
 #include <cstring>
 

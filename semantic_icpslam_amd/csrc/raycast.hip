@@ -361,8 +361,8 @@ SICP_DEV bool ray_setup(const MapDev& m, const View<float>& zmin, const View<flo
 // a lane that needs a table probe or an interpolated read waits while the
 // others march on, and the waiting lanes are served together when enough of
 // them wait: the same samples, each ray's in the same order. First pass at
-// 640x480 / 5 mm 122 to 92 us, at 2 mm 186 to 149, 1280x720 / 4 mm (half)
-// 224 to 152, 320x240 / 1 cm 95 to 64.
+// 640x480 / 5 mm 122 to 92 us, at 2 mm 174 to 134, 1280x720 / 4 mm (half)
+// 221 to 143, 320x240 / 1 cm 95 to 59.
 //
 // Blocks are named by a 30-bit tag relative to the wavefront's own origin
 // (10 bits an axis: a neighbour's tag is one addition away, and one compare
@@ -1096,8 +1096,9 @@ __global__ void ray_queue_reset_kernel(uint32_t* count) { *count = 0u; }
 // corner each of every trilinear read, and scatter its gradient; the values
 // and derivatives that follow from the corners are formed by every lane alike.
 // One thread per pixel left 160 wavefronts on 1024 SIMDs, each a chain of
-// 32000 instructions and 900 dependent reads: 257 us for 10000 pixels at
-// 1280x720 / 2 mm, 61 now.
+// 32000 instructions and 900 dependent reads: 226 us for 10000 pixels at
+// 1280x720 / 2 mm, 51 now (500 pixels with the launch's own time 161 and 48,
+// 200000 827 and 470, every pixel 2918 and 1969).
 
 // A trilinear read (readSdfInterped, RenderScene.cu:310-343) with this lane's
 // corner voxel and weight and the read's gradient in voxel units. The value
