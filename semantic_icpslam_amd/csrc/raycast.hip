@@ -361,7 +361,7 @@ SICP_DEV bool ray_setup(const MapDev& m, const View<float>& zmin, const View<flo
 // a lane that needs a table probe or an interpolated read waits while the
 // others march on, and the waiting lanes are served together when enough of
 // them wait: the same samples, each ray's in the same order. First pass at
-// 640x480 / 5 mm 122 to 92 us, at 2 mm 174 to 134, 1280x720 / 4 mm (half)
+// 640x480 / 5 mm 119 to 81 us, at 2 mm 174 to 134, 1280x720 / 4 mm (half)
 // 221 to 143, 320x240 / 1 cm 95 to 59.
 //
 // Blocks are named by a 30-bit tag relative to the wavefront's own origin
@@ -377,12 +377,12 @@ constexpr int kRayLdsEntries = 256;  // one 64-bit word each: tag + 1, slot
 constexpr uint32_t kTagX = 1u, kTagY = 1u << 10, kTagZ = 1u << 20;
 constexpr uint32_t kNoTag = 0xffffffffu;
 // Samples of a one-voxel run read together, and the waiting lanes' share that
-// has them served: measured at 640x480 / 5 mm, 2 mm, 1280x720 / 4 mm and
-// 320x240 / 1 cm, first pass in us: two samples 92, 149, 160, 66; one 101,
-// 153, 174, 74; three and four 110 to 118 (640x480). Serving the waiting
-// lanes when they are a third of the marching ones, as above; only when none
-// marches 135 (640x480); in every iteration 113; at half or a quarter the
-// same within 1.
+// has them served: measured (on other frames than above, and before the order
+// of tiles below) at 640x480 / 5 mm, 2 mm, 1280x720 / 4 mm and 320x240 / 1 cm,
+// first pass in us: two samples 92, 149, 160, 66; one 101, 153, 174, 74; three
+// and four 110 to 118 (640x480). Serving the waiting lanes when they are a
+// third of the marching ones, as above; only when none marches 135 (640x480);
+// in every iteration 113; at half or a quarter the same within 1.
 constexpr int kRayAhead = 2, kRayServe = 3;
 // Workgroups go to the eight XCDs in turn, each with an L2 of its own:
 // super-tiles of 8x8 tiles are given to one XCD, so that neighbouring rays

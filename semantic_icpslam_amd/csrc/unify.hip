@@ -25,7 +25,7 @@
 // whole column's x and y and three each z; the probes then read the staged
 // words; and where every neighbour bears the label tallied first (nine blocks
 // in ten) one compare, count and maximum per neighbour replace the walk over
-// the tallies. 6000 to 7000 visible blocks at 640x480 / 5 mm: 315 us before,
+// the tallies. 6000 to 7000 visible blocks at 640x480 / 5 mm: 312 us before,
 // 91 now; the blocks on a boundary, 43 us each against 11, set the end. Four
 // wavefronts a SIMD (the staging loop holds its 21 loads in registers): three
 // 92 us, five and more 111 to 127.
