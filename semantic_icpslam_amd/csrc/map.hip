@@ -610,13 +610,14 @@ struct FuseArgs {
 };
 
 // Channel c of label L's colour (FuseMap.cu:18,570-572): (palette x label) % 255
-// in wrapping int arithmetic, which may be negative, narrowed to the byte that
-// the voxel keeps: the records are packed into words, where a sign would fill
-// the bytes above.
+// in wrapping int arithmetic, narrowed to the byte that the voxel keeps: the
+// first channel's product wraps from label 65 on and may be negative (the others
+// stay below 2^30), and the records are packed into words, where a sign would
+// fill the bytes above.
 SICP_DEV int palette_channel(int c, int L) {
     const int pal = c == 0 ? (1 << 25) - 1 : (c == 1 ? (1 << 15) - 1 : (1 << 21) - 1);
     int prod = (int)((uint32_t)pal * (uint32_t)L);
-    return prod % 255 & 0xff;
+    return c == 0 ? prod % 255 & 0xff : prod % 255;
 }
 
 SICP_DEV int u8i(float v) { return (int)(uint8_t)(uint32_t)(int)v; }
